@@ -33,6 +33,7 @@
 #include "ion_state.hpp"
 #include "pkj_model.hpp"
 #include "record.hpp"
+#include "rkc_resident.hpp"
 
 namespace cbrkc {
 
@@ -231,17 +232,14 @@ struct PkjState {
 // pkj_update_ion_RKC (pkj_ion.cu:304-358) followed by pkj_update_matrix
 // (solve_rkc.cu:369-395), fused: one pass over the compartment state.
 // With do_ion == 0 only the current is rebuilt (RKC_vec_initialize).
-__global__ void __launch_bounds__(256) k_pkj_ion_b(PkjState S, const double *__restrict__ vnew, double DT, int do_ion) {
+__device__ inline double pkj_ion_current(const PkjState &S, int i, double vn, double DT, bool do_ion) {
   using namespace pkj;
   const int nc = S.nc;
-  int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= nc) return;
   double g[NGATE], c[NCOND];
 #pragma unroll
   for (int k = 0; k < NGATE; k++) g[k] = S.gate[(size_t)k * nc + i];
 #pragma unroll
   for (int k = 0; k < NCOND; k++) c[k] = S.cond[(size_t)k * nc + i];
-  const double vn = vnew[i];
   double rev = S.rev[i];
   if (do_ion) {
     const double vo = S.v[i];
@@ -260,7 +258,12 @@ __global__ void __launch_bounds__(256) k_pkj_ion_b(PkjState S, const double *__r
   if (S.syn_g) bb += S.syn_g[i] * (vn - S.syn_e);
   // pkj_update_matrix_new (solve_rkc.cu:358-367, 1245-1249)
   if (S.net_s) bb += S.net_s[i] * S.net_decay;
-  S.b[i] = bb;
+  return bb;
+}
+
+__global__ void __launch_bounds__(256) k_pkj_ion_b(PkjState S, const double *__restrict__ vnew, double DT, int do_ion) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < S.nc) S.b[i] = pkj_ion_current(S, i, vnew[i], DT, do_ion != 0);
 }
 
 
@@ -269,24 +272,28 @@ __global__ void __launch_bounds__(256) k_pkj_ion_b(PkjState S, const double *__r
 // (gap.cu:149-160, solve_rkc.cu:400-410), fused.  The gap current uses the
 // partners' voltages after the update (elem[v] = vnew there) and is added in
 // partner order 0..3 (the reference adds with atomics in no fixed order).
-__global__ void __launch_bounds__(256) k_io_ion_b(IoState S, const double *__restrict__ vnew, double DT, int do_ion) {
+// dend(cell): the new voltage of a cell's dendrite.
+template <class Dend>
+__device__ inline double io_ion_gap_current(const IoState &S, int i, double vn, double DT, bool do_ion, Dend dend) {
   using namespace io;
-  const int nc = S.nc;
-  int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= nc) return;
-  const double vn = vnew[i];
-  double bb = io_ion_current(S, i, vn, DT, do_ion != 0);
+  double bb = io_ion_current(S, i, vn, DT, do_ion);
   if (do_ion && S.n > 1 && i % COMP == 0) {
     const int cell = i / COMP;
 #pragma unroll
     for (int s = 0; s < 4; s++) {
       const int pre = S.nbr[cell * 4 + s];
-      const double diff_v = (pre > -1) ? (vn - vnew[pre * COMP]) : 0.0;
+      const double diff_v = (pre > -1) ? (vn - dend(pre)) : 0.0;
       bb += gap_current<double>(diff_v);
     }
   }
   if (S.syn_g) bb += S.syn_g[i] * (vn - S.syn_e);
-  S.b[i] = bb;
+  return bb;
+}
+
+__global__ void __launch_bounds__(256) k_io_ion_b(IoState S, const double *__restrict__ vnew, double DT, int do_ion) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < S.nc)
+    S.b[i] = io_ion_gap_current(S, i, vnew[i], DT, do_ion != 0, [&](int cell) { return vnew[cell * io::COMP]; });
 }
 
 
@@ -295,16 +302,17 @@ __global__ void __launch_bounds__(256) k_io_ion_b(IoState S, const double *__res
 // three reference kernels touch one compartment's state each, in this order
 // (solve_rkc.cu:1174-1179).  The intercell gap junctions are in the cable
 // matrix, not here.
-__global__ void __launch_bounds__(256) k_go_ion_b(GoState S, const double *__restrict__ vnew, double DT, int do_ion) {
-  const int nc = S.nc;
-  int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= nc) return;
-  const double vn = vnew[i];
-  double bb = go_ion_current(S, i, vn, DT, do_ion != 0);
+__device__ inline double go_ion_net_current(const GoState &S, int i, double vn, double DT, bool do_ion) {
+  double bb = go_ion_current(S, i, vn, DT, do_ion);
   if (S.syn_g) bb += S.syn_g[i] * (vn - S.syn_e);
   // go_update_matrix_new (solve_rkc.cu:279-286, 1181)
   if (S.net_s) bb += S.net_s[i];
-  S.b[i] = bb;
+  return bb;
+}
+
+__global__ void __launch_bounds__(256) k_go_ion_b(GoState S, const double *__restrict__ vnew, double DT, int do_ion) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < S.nc) S.b[i] = go_ion_net_current(S, i, vnew[i], DT, do_ion != 0);
 }
 
 
@@ -313,12 +321,8 @@ __global__ void __launch_bounds__(256) k_go_ion_b(GoState S, const double *__res
 // the reference's order (solve_rkc.cu:1111-1116): the Na scheme sees the
 // voltage of the previous ion update and the new one, then the gates move and
 // the stored voltage becomes the new one.
-__global__ void __launch_bounds__(256) k_gr_ion_b(GrState S, const double *__restrict__ vnew, double DT, int do_ion) {
-  const int nc = S.nc;
-  int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= nc) return;
-  const double vn = vnew[i];
-  double bb = gr_ion_current(S, i, vn, DT, do_ion != 0);
+__device__ inline double gr_ion_net_current(const GrState &S, int i, double vn, double DT, bool do_ion) {
+  double bb = gr_ion_current(S, i, vn, DT, do_ion);
   if (S.syn_g) bb += S.syn_g[i] * (vn - S.syn_e);
   // add_mfgr_val / add_gogr_val (solve_rkc.cu:200-224, 1117-1118), one
   // synapse after the other
@@ -328,8 +332,73 @@ __global__ void __launch_bounds__(256) k_gr_ion_b(GrState S, const double *__res
       const double gs = syn_entry(S.net, j, E);
       bb += gs * (vn - E);
     }
-  S.b[i] = bb;
+  return bb;
 }
+
+__global__ void __launch_bounds__(256) k_gr_ion_b(GrState S, const double *__restrict__ vnew, double DT, int do_ion) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < S.nc) S.b[i] = gr_ion_net_current(S, i, vnew[i], DT, do_ion != 0);
+}
+
+__global__ void k_coop_probe() {}
+
+// Whether this process may launch cooperatively on the current device: the
+// barrier resource behind it belongs to one process at a time, which keeps
+// it to its end, so while another one holds it every such launch is refused.
+bool coop_available(hipStream_t st) {
+  int dev = 0, coop = 0;
+  CB_HIP(hipGetDevice(&dev));
+  CB_HIP(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev));
+  if (!coop) return false;
+  const hipError_t e = hipLaunchCooperativeKernel((const void *)k_coop_probe, dim3(1), dim3(64), nullptr, 0, st);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  CB_HIP(hipStreamSynchronize(st));
+  return true;
+}
+
+// The models of the resident kernel.  512 threads hold a Purkinje cell's 1600
+// compartments four to a thread; the granule and Golgi updates keep their 12 x 12
+// and 6 x 6 systems in registers, which takes one wave per SIMD.
+struct PkjModel {
+  using State = PkjState;
+  static constexpr int NT = 512, NONFINITE_STATUS = NONFINITE;
+  static constexpr bool GAP = false;
+  template <class Dend>
+  __device__ static double ion(State S, int i, double vn, double dt, Dend) {
+    if (S.net_s) S.net_decay = exp(-dt / 0.6);
+    return pkj_ion_current(S, i, vn, dt, true);
+  }
+};
+struct IoModel {
+  using State = IoState;
+  static constexpr int NT = 256, NONFINITE_STATUS = NONFINITE;
+  static constexpr bool GAP = true;
+  template <class Dend>
+  __device__ static double ion(const State &S, int i, double vn, double dt, Dend dend) {
+    return io_ion_gap_current(S, i, vn, dt, true, dend);
+  }
+};
+struct GoModel {
+  using State = GoState;
+  static constexpr int NT = 256, NONFINITE_STATUS = NONFINITE;
+  static constexpr bool GAP = false;
+  template <class Dend>
+  __device__ static double ion(const State &S, int i, double vn, double dt, Dend) {
+    return go_ion_net_current(S, i, vn, dt, true);
+  }
+};
+struct GrModel {
+  using State = GrState;
+  static constexpr int NT = 256, NONFINITE_STATUS = NONFINITE;
+  static constexpr bool GAP = false;
+  template <class Dend>
+  __device__ static double ion(const State &S, int i, double vn, double dt, Dend) {
+    return gr_ion_net_current(S, i, vn, dt, true);
+  }
+};
 
 // xx_set_current shape: one compartment per cell, a time window (pkj.cu:333-344)
 __global__ void k_set_current(double *__restrict__ iext, const double *__restrict__ amp, int comp, int stim_comp,
@@ -410,10 +479,17 @@ class GlobalRkc : public Engine {
       CB_HIP(hipMemset(syn_g_, 0, sizeof(double) * nc_));
     }
     hmax_ = H_MAX;
+    row_h_ = row;
+    col_h_ = col;
+    val_h_ = val;
   }
 
   ~GlobalRkc() override {
     (void)hipStreamSynchronize(st_);
+    for (void *p : res_bufs_) (void)hipFree(p);
+    if (rec_) (void)hipFree(rec_);
+    if (bits_) (void)hipFree(bits_);
+    if (ctl_host_) (void)hipHostFree(ctl_host_);
     for (void *p : {(void *)v_, (void *)iext_, (void *)cm_, (void *)b_, (void *)dammy_, (void *)row_, (void *)col_,
                     (void *)val_, (void *)red_a_, (void *)red_b_, (void *)bad_, (void *)amp_, (void *)syn_g_,
                     (void *)zero_, (void *)net_s_})
@@ -425,10 +501,32 @@ class GlobalRkc : public Engine {
 
   int nc() const override { return nc_; }
   int ncell() const override { return n_; }
-  Stats stats() const override { return st; }
+  Stats stats() const override {
+    if (!resident_) return st;
+    const RkcCtl &c = *ctl_host_;
+    Stats s;
+    s.steps = c.steps;
+    s.rejects = c.rejects;
+    s.stages = c.stages;
+    s.rho_iters = c.rho_iters;
+    s.ion_updates = c.ions;
+    s.macro_steps = c.macro;
+    return s;
+  }
   void controller(double *o, double *hw) const override {
+    if (resident_) {
+      const RkcCtl &c = *ctl_host_;
+      std::memcpy(o, c.o, sizeof(o_));
+      std::memcpy(hw, c.hw, sizeof(hw_));
+      return;
+    }
     std::memcpy(o, o_, sizeof(o_));
     std::memcpy(hw, hw_, sizeof(hw_));
+  }
+  std::string mapping() const override {
+    if (!resident_) return "one thread per compartment, one launch per stage";
+    return std::to_string(A_.nblk) + " workgroups of " + std::to_string(A_.cpb) +
+           " cells, many macro steps per launch" + (A_.imp0 ? ", gap-junction values exchanged per stage" : "");
   }
   void sync() override { CB_HIP(hipStreamSynchronize(st_)); }
 
@@ -437,6 +535,11 @@ class GlobalRkc : public Engine {
   }
 
   void advance() override {
+    if (resident_) {
+      if (net_.on() && net_s_) syn_macro_current(net_, vec_[Y], net_s_, nc_, st_);
+      for (const long m0 = macro_; macro_ == m0; check_steps()) res_launch(A_, 1, 0.0, (int)macro_);
+      return;
+    }
     if (syn_.on) {
       double lam = syn_.rate_hz * H_MAX * 1e-3;
       double p = 1.0 - std::exp(-lam);
@@ -474,6 +577,48 @@ class GlobalRkc : public Engine {
     k_rkcint<<<nblk(nc_), 256, 0, st_>>>(vec_[VNEW], a1, a2, b1, b2, vec_[VT1], vec_[VT2], vec_[YN], vec_[FN], nc_);
     o_[TEND] += H_MAX;
     st.macro_steps++;
+  }
+
+  // a run of the resident kernel: the stimulus, the recorder and the raster
+  // are in it, RES_RUN macro steps to a launch.  The Golgi and Purkinje
+  // network coupling takes the macro step's synaptic current from its starting
+  // y, so it goes step by step.
+  void run(int nsteps, double t0, int rec_comp, double *rec_out) override {
+    if (!resident_ || (net_.on() && net_s_) || nsteps <= 0) {
+      Engine::run(nsteps, t0, rec_comp, rec_out);
+      return;
+    }
+    const size_t per = rec_comp >= 0 ? n_ : nc_;
+    const int words = (n_ + 31) / 32;
+    const bool raster = raster_comp_ >= 0;
+    if (rec_out) grow(rec_, rec_cap_, (size_t)nsteps * per);
+    if (raster) {
+      grow(bits_, bits_cap_, (size_t)nsteps * words);
+      CB_HIP(hipMemsetAsync(bits_, 0, sizeof(uint32_t) * (size_t)nsteps * words, st_));
+    }
+    const long m0 = macro_;
+    while (macro_ < m0 + nsteps) {
+      const int k = (int)(macro_ - m0);
+      RkcArgs a = A_;
+      a.do_stim = 1;
+      if (rec_out) a.rec = rec_ + (size_t)k * per;
+      a.rec_comp = rec_comp;
+      if (raster) {
+        a.bits = bits_ + (size_t)k * words;
+        a.prev = raster_prev();
+        a.raster_comp = raster_comp_;
+        a.thr = raster_thr_;
+        a.words = words;
+      }
+      res_launch(a, std::min(RES_RUN, nsteps - k), t0 + k * H_MAX, (int)macro_);
+      check_steps();
+    }
+    std::vector<uint32_t> bits((size_t)(raster ? nsteps : 0) * words);
+    if (rec_out)
+      CB_HIP(hipMemcpyAsync(rec_out, rec_, sizeof(double) * (size_t)nsteps * per, hipMemcpyDeviceToHost, st_));
+    if (raster) CB_HIP(hipMemcpyAsync(bits.data(), bits_, sizeof(uint32_t) * bits.size(), hipMemcpyDeviceToHost, st_));
+    CB_HIP(hipStreamSynchronize(st_));
+    if (raster) append_spikes(bits, nsteps, words, t0, H_MAX);
   }
 
   const double *device_v() const override { return v_; }
@@ -525,6 +670,216 @@ class GlobalRkc : public Engine {
     init(sol.atol, sol.rtol);
     if (sol.ion_interval > 0) integ_ = sol.ion_interval;
     refresh_fn_ = sol.refresh_fn;
+    make_resident();
+    row_h_.clear();
+    col_h_.clear();
+    val_h_.clear();
+  }
+
+  // the cell type's resident kernel: its threads per workgroup and address,
+  // and a launch of it with the type's state
+  virtual int res_threads() const = 0;
+  virtual const void *res_kernel() const = 0;
+  virtual void res_launch(const RkcArgs &a, int nsteps, double t0, int step0) = 0;
+  virtual bool res_strict() const { return false; }
+
+  template <class Model>
+  void launch_model(const RkcArgs &a, const typename Model::State &S, int nsteps, double t0, int step0) {
+    RkcArgs av = a;
+    typename Model::State sv = S;
+    void *args[] = {&av, &sv, &nsteps, &t0, &step0};
+    const void *f = (const void *)k_rkc_steps<Model>;
+    if (a.nblk == 1)
+      CB_HIP(hipLaunchKernel(f, dim3(1), dim3(Model::NT), args, res_lds_, st_));
+    else   // the workgroups wait for one another: all of them resident at once
+      CB_HIP(hipLaunchCooperativeKernel(f, dim3(a.nblk), dim3(Model::NT), args, (unsigned)res_lds_, st_));
+  }
+
+  // waits for the launch, takes the kernel's question if it stopped for one
+  // (the next launch brings the answer); a failed step ends the run as on the
+  // other path
+  void check_steps() {
+    CB_HIP(hipGetLastError());
+    CB_HIP(hipStreamSynchronize(st_));
+    const RkcCtl &c = *ctl_host_;
+    macro_ = c.macro;
+    A_.resume = c.status == ASK_POW;
+    if (A_.resume) {
+      A_.p1 = std::pow(c.err, 1.0 / 3.0);
+      A_.p2 = std::pow(c.err, 2.0 / 3.0);
+    }
+    if (c.status == 0 || A_.resume) return;
+    if (c.status == NONFINITE)
+      throw Error("RKC: non-finite state (error estimate " + std::to_string(c.err) + ")", NONFINITE);
+    if (c.status == TIMED_OUT) throw Error("RKC: a workgroup of the step kernel waited for another one in vain");
+    throw Error("RKC failed: idid = " + std::to_string(c.status), c.status);
+  }
+
+  template <typename T>
+  void grow(T *&p, size_t &cap, size_t n) {
+    if (cap >= n) return;
+    if (p) CB_HIP(hipFree(p));
+    p = nullptr;
+    cap = 0;
+    p = dalloc<T>(n);
+    cap = n;
+  }
+
+  template <typename T>
+  T *res_put(const std::vector<T> &h) {
+    T *d = dalloc<T>(h.size());
+    res_bufs_.push_back((void *)d);
+    h2d(d, h);
+    return d;
+  }
+
+  // Decides whether the population runs on the resident kernel and lays out
+  // its tables.  Whole cells go to a workgroup, as few as leave at most one
+  // workgroup per CU (more CUs shorten the ion update, whose rows run one to a
+  // thread) but at least a row per thread; the population has to fit the LDS of
+  // the chip's CUs.  Larger ones are bound by the vectors' traffic and stay on
+  // the launch-per-stage path, and so do populations of several workgroups in a
+  // process that may not launch cooperatively.
+  void make_resident() {
+    int dev = 0, ncu = 0, lds_max = 0;
+    CB_HIP(hipGetDevice(&dev));
+    CB_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+    CB_HIP(hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
+    const int NT = res_threads();
+    RkcArgs a{};
+    a.n = n_;
+    a.nc = nc_;
+    a.comp = comp_;
+    a.cpb = std::min(n_, std::max((n_ + ncu - 1) / ncu, std::max(1, NT / comp_)));
+    a.nblk = (n_ + a.cpb - 1) / a.cpb;
+    a.nch = (nc_ + RED_BLOCK - 1) / RED_BLOCK;
+    if (a.nch > 2048) return;
+    const int RM = a.cpb * comp_;
+    if (RM > 4096) return;   // (local indices have 16 bits)
+    // local rows, ghosts and who posts them
+    std::vector<unsigned short> lrow, lcol;
+    std::vector<double> lval;
+    std::vector<int> lnz0(1, 0), imp0(1, 0), imp;
+    auto block_of = [&](int r) { return r / RM; };
+    for (int w = 0; w < a.nblk; w++) {
+      const int r0 = w * RM, r1 = std::min(nc_, r0 + RM), R = r1 - r0;
+      const size_t m0 = imp.size();
+      for (int i = r0; i < r1; i++) {
+        lrow.push_back((unsigned short)((int)lval.size() - lnz0[w]));
+        for (int j = row_h_[i]; j < row_h_[i + 1]; j++) {
+          const int c = col_h_[j];
+          if (c == i) continue;   // the stored diagonal adds val (y_i - y_i) = 0
+          int l = c - r0;
+          if (c < r0 || c >= r1) {
+            size_t k = m0;
+            while (k < imp.size() && imp[k] != c) k++;
+            if (k == imp.size()) imp.push_back(c);
+            l = R + (int)(k - m0);
+          }
+          lcol.push_back((unsigned short)l);
+          lval.push_back(val_h_[j]);
+        }
+      }
+      const int nz = (int)lval.size() - lnz0[w];
+      if (nz > 65535 || imp.size() - m0 > 4096) return;
+      lrow.push_back((unsigned short)nz);
+      lnz0.push_back((int)lval.size());
+      imp0.push_back((int)imp.size());
+      a.nnz_max = std::max(a.nnz_max, nz);
+      a.ghost_max = std::max(a.ghost_max, (int)(imp.size() - m0));
+    }
+    const int RS = RM + a.ghost_max;
+    res_lds_ = sizeof(double) * ((size_t)5 * RS + 3 * RM + RED_BLOCK + a.nch + 8 + 4 * RES_COEF + a.nnz_max) +
+               sizeof(unsigned short) * ((size_t)RM + 1 + a.nnz_max);
+    res_lds_ = (res_lds_ + 15) & ~(size_t)15;
+    if (res_lds_ > (size_t)lds_max) return;
+    CB_HIP(hipFuncSetAttribute(res_kernel(), hipFuncAttributeMaxDynamicSharedMemorySize, (int)res_lds_));
+    int fit = 0;
+    CB_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, res_kernel(), NT, res_lds_));
+    if (fit < 1 || (a.nblk > 1 && !coop_available(st_))) return;
+    const int nslot = (int)imp.size();
+    if (nslot > 0) {
+      if ((size_t)nslot * 3 * GHOST_STAGES * sizeof(double) > (size_t)1 << 30) return;
+      std::vector<std::vector<std::pair<int, int>>> exp(a.nblk);
+      for (int s = 0; s < nslot; s++) exp[block_of(imp[s])].push_back({imp[s] % RM, s});
+      std::vector<int> exp0(1, 0), er, es;
+      for (auto &e : exp) {
+        for (auto &x : e) {
+          er.push_back(x.first);
+          es.push_back(x.second);
+        }
+        exp0.push_back((int)er.size());
+      }
+      a.imp0 = res_put(imp0);
+      a.exp0 = res_put(exp0);
+      a.exp_row = res_put(er);
+      a.exp_slot = res_put(es);
+      a.ghost = empty_mail((size_t)3 * GHOST_STAGES * nslot);
+      a.nslot = nslot;
+    }
+    a.lrow = res_put(lrow);
+    a.lcol = res_put(lcol);
+    a.lval = res_put(lval);
+    a.lnz0 = res_put(lnz0);
+    if (a.nblk > 1) {
+      a.terms = empty_mail((size_t)3 * nc_);
+      a.parts = empty_mail((size_t)3 * a.nch);
+      a.gap = empty_mail((size_t)3 * n_);
+    }
+    a.y = vec_[Y];
+    a.yn = vec_[YN];
+    a.fn = vec_[FN];
+    a.ede = vec_[EDE];
+    a.vnew = vec_[VNEW];
+    a.b = b_;
+    a.v1 = vec_[VT1];
+    a.v2 = vec_[VT2];
+    a.cm = cm_;
+    a.coef = res_put(rkc_stage_table(RES_COEF));
+    RkcCtl c{};
+    std::memcpy(c.o, o_, sizeof(o_));
+    std::memcpy(c.hw, hw_, sizeof(hw_));
+    c.sum_dt = sum_dt_;
+    c.errold3 = std::pow(o_[ERROLD], 1.0 / 3.0);
+    c.steps = st.steps;
+    c.rejects = st.rejects;
+    c.stages = st.stages;
+    c.rho_iters = st.rho_iters;
+    c.ions = st.ion_updates;
+    c.last = last_;
+    c.newspc = newspc_;
+    c.jacatt = jacatt_;
+    a.ctl = res_put(std::vector<RkcCtl>(1, c));
+    CB_HIP(hipHostMalloc((void **)&ctl_host_, sizeof(RkcCtl), hipHostMallocMapped | hipHostMallocCoherent));
+    *ctl_host_ = c;
+    CB_HIP(hipHostGetDevicePointer((void **)&a.ctl_host, ctl_host_, 0));
+    a.integ = integ_;
+    a.rho_floor = rho_floor_;
+    a.strict = res_strict();
+    a.refresh_fn = refresh_fn_;
+    a.iext = iext_;
+    a.amp = amp_;
+    a.stim_comp = stim_.comp;
+    a.stim_t0 = stim_.t0;
+    a.stim_t1 = stim_.t1;
+    if (syn_.on) {
+      a.syn_g = syn_g_;
+      a.syn_decay = std::exp(-H_MAX / syn_.tau_ms);
+      a.syn_p = 1.0 - std::exp(-syn_.rate_hz * H_MAX * 1e-3);
+      a.syn_event = syn_.g_event;
+      a.k0 = (uint32_t)syn_.seed;
+      a.k1 = (uint32_t)(syn_.seed >> 32);
+    }
+    A_ = a;
+    CB_HIP(hipStreamSynchronize(st_));
+    resident_ = true;
+  }
+
+  double *empty_mail(size_t n) {
+    unsigned long long e = MAIL_EMPTY;
+    double x;
+    std::memcpy(&x, &e, sizeof(x));
+    return res_put(std::vector<double>(n, x));
   }
 
   Csr csr() const { return Csr{row_, col_, val_}; }
@@ -827,6 +1182,19 @@ class GlobalRkc : public Engine {
   double rho_floor_ = 0.0;
   double sum_dt_ = 0.0, integ_ = 0.0, hmin_, hmax_;
   Stats st;
+  // the resident kernel's tables and workspaces
+  static constexpr int RES_RUN = 64;   // macro steps per launch
+  bool resident_ = false;
+  RkcArgs A_{};
+  RkcCtl *ctl_host_ = nullptr;   // written by the kernel as it ends
+  size_t res_lds_ = 0;
+  long macro_ = 0;
+  std::vector<void *> res_bufs_;
+  std::vector<int> row_h_, col_h_;
+  std::vector<double> val_h_;
+  double *rec_ = nullptr;
+  uint32_t *bits_ = nullptr;
+  size_t rec_cap_ = 0, bits_cap_ = 0;
 };
 
 // Purkinje cells (pkj.cu, pkj_solve.cu, pkj_ion.cu)
@@ -851,6 +1219,12 @@ class GlobalPkj : public GlobalRkc {
   static StimSpec with_amp(StimSpec s, int n) {
     if (s.amp.size() != (size_t)n) s.amp.assign(n, pkj::CURRENT);
     return s;
+  }
+  int res_threads() const override { return PkjModel::NT; }
+  const void *res_kernel() const override { return (const void *)k_rkc_steps<PkjModel>; }
+  void res_launch(const RkcArgs &a, int nsteps, double t0, int step0) override {
+    launch_model<PkjModel>(a, PkjState{v_, ca_, rev_, iext_, shell_, cond_, gate_, b_, syn_g_, syn_.e_syn, nc_,
+                                     net_.on() ? net_s_ : nullptr, 0.0}, nsteps, t0, step0);
   }
   void model_b(const double *vv, bool do_ion, double dt) override {
     // the granule input enters at ion updates only (pkj_update_ion_and_matrix)
@@ -899,6 +1273,12 @@ class GlobalIo : public GlobalRkc {
     return s;
   }
   bool trigger() const override { return sum_dt_ > integ_; }   // strict for IO, solve_rkc.cu:1347
+  int res_threads() const override { return IoModel::NT; }
+  const void *res_kernel() const override { return (const void *)k_rkc_steps<IoModel>; }
+  bool res_strict() const override { return true; }
+  void res_launch(const RkcArgs &a, int nsteps, double t0, int step0) override {
+    launch_model<IoModel>(a, IoState{v_, ca_, iext_, cond_, gate_, compart_, nbr_, b_, syn_g_, syn_.e_syn, nc_, n_}, nsteps, t0, step0);
+  }
   void model_b(const double *vv, bool do_ion, double dt) override {
     IoState S{v_, ca_, iext_, cond_, gate_, compart_, nbr_, b_, syn_g_, syn_.e_syn, nc_, n_};
     k_io_ion_b<<<nblk(nc_), 256, 0, st_>>>(S, vv, dt, do_ion ? 1 : 0);
@@ -940,6 +1320,12 @@ class GlobalGo : public GlobalRkc {
   static StimSpec with_amp(StimSpec s, int n) {
     if (s.amp.size() != (size_t)n) s.amp.assign(n, go::STIM);
     return s;
+  }
+  int res_threads() const override { return GoModel::NT; }
+  const void *res_kernel() const override { return (const void *)k_rkc_steps<GoModel>; }
+  void res_launch(const RkcArgs &a, int nsteps, double t0, int step0) override {
+    launch_model<GoModel>(a, GoState{v_, ca_, ca2_, rev_, ca_old_, iext_, area_, cond_, gate_, b_, syn_g_, syn_.e_syn, nc_,
+                                   net_.on() ? net_s_ : nullptr}, nsteps, t0, step0);
   }
   void model_b(const double *vv, bool do_ion, double dt) override {
     const bool net = do_ion && net_.on();
@@ -990,6 +1376,12 @@ class GlobalGr : public GlobalRkc {
     return s;
   }
   bool trigger() const override { return sum_dt_ > integ_; }   // strict for GR, solve_rkc.cu:1148
+  int res_threads() const override { return GrModel::NT; }
+  const void *res_kernel() const override { return (const void *)k_rkc_steps<GrModel>; }
+  bool res_strict() const override { return true; }
+  void res_launch(const RkcArgs &a, int nsteps, double t0, int step0) override {
+    launch_model<GrModel>(a, GrState{v_, iext_, ca_, compart_, cond_, gate_, na_, b_, syn_g_, syn_.e_syn, nc_, net_}, nsteps, t0, step0);
+  }
   void model_b(const double *vv, bool do_ion, double dt) override {
     GrState S{v_, iext_, ca_, compart_, cond_, gate_, na_, b_, syn_g_, syn_.e_syn, nc_,
               do_ion ? net_ : SynIn()};

@@ -1,0 +1,563 @@
+// The population-global RKC controller and its steps in one kernel: many
+// macro steps of rkclow / step / rkcrho (solve_rkc.cu:562-1096) and the ion
+// updates between them without the host.
+//
+// What it replaces took one launch per Chebyshev stage, four more and a read
+// back by the host per step attempt: 3-5 us a launch whatever the population
+// (two thirds of a small population's time), plus the host's answer.  Here
+// every workgroup owns whole cells, keeps their seven vectors and its rows of
+// the cable matrix in LDS and runs the controller's scalar arithmetic itself
+// on the same sums; a stage costs a barrier, a step attempt one exchange of
+// the error norm's partial sums.  Cells whose cable matrix couples them
+// (gap junctions) also exchange the coupled compartments' values at every
+// stage.  The additions of every right-hand side, stage and norm are those of
+// the launch-per-stage path in the same order, so the two agree bit for bit.
+// Measured, calls of Population.run (us): 16 granule cells, one macro step,
+// 29260 -> 13690; 256 Golgi cells, 40 steps, 84390 -> 45370; 64 coupled
+// Purkinje cells, 8 steps, 2875 -> 2179; 9 uncoupled ones 8225 -> 6842.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include "grid_mail.hpp"
+#include "philox.hpp"
+
+namespace cbrkc {
+
+// The controller between launches (solve_rkc.cu's others[] and hwork[]), one
+// record per population
+struct RkcCtl {
+  double o[16], hw[8];
+  double sum_dt;
+  double errold3;             // o[ERROLD]^(1/3)
+  double err, h;              // of the step attempt that stopped the kernel (status NONFINITE, ASK_POW)
+  long long steps, rejects, stages, rho_iters, ions, macro;
+  int last, newspc, jacatt, status;
+  unsigned q, ions_q;         // numbers (modulo 3) of the next sum and gap-current exchange
+  int ghost_used;             // coupled-value exchanges before the last sum
+  int loops;
+};
+
+// Stage counts up to RES_COEF read their coefficients from the table; larger
+// ones run the recurrence in the kernel
+constexpr int ASK_POW = 9;   // status: the host has to give the powers of err
+constexpr int RES_COEF = 128;
+constexpr int GHOST_STAGES = 136;   // exchanges of coupled values between two sums
+
+struct RkcArgs {
+  int n, nc, comp, nblk, cpb;            // cells, rows, rows per cell, workgroups, cells per workgroup
+  int nnz_max, ghost_max, nch;           // LDS sizes: matrix entries and ghosts of a workgroup, chunks
+  const int *row, *col;                  // CSR of the cable matrix
+  const double *val;
+  // the same rows with local columns: rows of workgroup w start at lrow[its
+  // first row + w], entries without the diagonal, columns local (ghosts from
+  // the workgroup's row count on)
+  const unsigned short *lrow, *lcol;
+  const double *lval;
+  const int *lnz0;                       // first entry of each workgroup (nblk + 1)
+  const int *imp0, *exp0, *exp_row, *exp_slot;   // ghosts fetched, rows posted (null: uncoupled cells)
+  double *ghost;                         // [3][GHOST_STAGES][nslot]
+  int nslot;
+  double *terms, *parts;                 // grid_sum's mailboxes
+  double *gap;                           // [3][n]: dendrite voltages for the olive's gap currents
+  double *y, *yn, *fn, *ede, *vnew, *b, *v1, *v2;
+  const double *cm, *coef;
+  RkcCtl *ctl, *ctl_host;                // the record, and its copy in mapped host memory
+  int resume;                            // 1: the attempt that stopped goes on with err's powers p1, p2
+  double p1, p2;
+  double integ, rho_floor;
+  int strict, refresh_fn;
+  // per macro step: the stimulus, the Poisson drive, the recorder
+  double *iext;
+  const double *amp;
+  int stim_comp, do_stim;
+  double stim_t0, stim_t1;
+  double *syn_g;                         // null: no drive
+  double syn_decay, syn_p, syn_event;
+  uint32_t k0, k1;
+  double *rec;                           // this launch's recording, or null
+  int rec_comp;                          // < 0: every compartment
+  uint32_t *bits;
+  double *prev;
+  int raster_comp, words;
+  double thr;
+};
+
+// x^(1/3) and x^(2/3) with the exponents 1.0 / 3.0 and 2.0 / 3.0 as the
+// controller writes them: the cube root in double, its remainder by fused
+// multiply-adds, and the factor x^(-d) for the exponent's own rounding
+// d = 1/3 - fl(1/3) to first order; the error before the last rounding is
+// below 1e-5 ulp.  The reference's controller rounds as the host's libm does,
+// and at the granule cell's tolerance one last bit of a step size moves its
+// voltage by 1e-4 mV within 0.5 ms.  libm's pow misses the nearest double only
+// where the value lies within 0.0083 ulp of the middle between two (measured,
+// 12 million arguments, 8e-4 of them missed), so a result that is POW_SLACK or more away from
+// a middle is libm's result too; for the others (sure = false, one in 50) the
+// kernel stops and the host answers with pow.
+constexpr double POW_SLACK = 0.01;
+struct CubeRoots {
+  double p1, p2;
+  bool sure1, sure2;
+};
+__device__ inline double round_sure(double hi, double lo, bool &sure) {
+  const double s = hi + lo, rem = (hi - s) + lo;
+  const long long e = (__double_as_longlong(s) & 0x7FF0000000000000ll) - (52ll << 52);
+  const double ulp = __longlong_as_double(e);   // s within (1e-20, 1e20): a normal number
+  sure = fabs(fabs(rem) - 0.5 * ulp) > POW_SLACK * ulp;
+  return s;
+}
+__device__ inline CubeRoots cube_roots(double x) {
+  CubeRoots r;
+  if (!(x > 1e-30 && x < 1e30)) {
+    r.p1 = r.p2 = 0.0;
+    r.sure1 = r.sure2 = false;
+    return r;
+  }
+  const float l2 = __builtin_amdgcn_logf((float)x);
+  double y = (double)__builtin_amdgcn_exp2f(l2 * (1.0f / 3.0f));   // relative error ~1e-6
+  y = y - (y * y * y - x) / (3.0 * (y * y));                       // ~1e-12
+  y = y - (y * y * y - x) / (3.0 * (y * y));                       // rounding level
+  const double p = y * y, pe = fma(y, y, -p);
+  const double q = p * y, qe = fma(p, y, -q);
+  const double c = ((x - q) - qe - pe * y) / (3.0 * p);
+  const double d = 1.850371707708594e-17 * ((double)l2 * 0.6931471805599453);
+  r.p1 = round_sure(y, c - y * d, r.sure1);
+  r.p2 = round_sure(p, pe + 2.0 * y * c - p * (2.0 * d), r.sure2);
+  return r;
+}
+
+// Model: NT threads, the state struct, ion(S, i, vn, dt) = ion update and
+// frozen current of row i, GAP = the olive's explicit gap currents.
+template <class Model>
+__global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, typename Model::State S, int nsteps, double t0,
+                                                         int step0) {
+  constexpr int NT = Model::NT;
+  constexpr double UR = 2.22e-16, H = 0.125;
+  extern __shared__ double sm[];
+  const int tid = threadIdx.x, w = blockIdx.x;
+  const int cell0 = w * A.cpb, cells = min(A.cpb, A.n - cell0);
+  const int r0 = cell0 * A.comp, R = cells * A.comp, RM = A.cpb * A.comp, RS = RM + A.ghost_max;
+  double *Yv = sm, *YN = Yv + RS, *FN = YN + RS, *V1 = FN + RS, *V2 = V1 + RS;
+  double *B = V2 + RS, *CM = B + RM, *T = CM + RM, *part = T + RM + RED_BLOCK, *C4 = part + A.nch + 8;
+  double *LV = C4 + 4 * RES_COEF;
+  unsigned short *LR = (unsigned short *)(LV + A.nnz_max), *LC = LR + RM + 1;
+  int late = 0;
+  SumPlan P;
+  P.set(A.nc, r0, r0 + R);
+
+  RkcCtl *ctl = A.ctl;
+  const double at = ctl->o[4], rt = ctl->o[5], hmin = ctl->hw[6], mmax = ctl->o[0];
+  double absh = ctl->o[1], sprad = ctl->o[2], naccpt = ctl->o[3], idid = ctl->o[6], gt = ctl->o[7],
+         gt_old = ctl->o[8], lt = ctl->o[9], tend = ctl->o[10], errold = ctl->o[11], hold = ctl->o[12];
+  double hw0 = ctl->hw[0], hw1 = ctl->hw[1], sum_dt = ctl->sum_dt, err = ctl->err;
+  bool last = ctl->last, newspc = ctl->newspc, jacatt = ctl->jacatt;
+  long long n_step = ctl->steps, n_rej = ctl->rejects, n_stage = ctl->stages, n_rho = ctl->rho_iters, n_ion = ctl->ions;
+  unsigned q = ctl->q, gq = ctl->ions_q;
+  int status = 0, done_steps = 0;
+  double errold3 = ctl->errold3, h_now = ctl->h;
+  bool resume = A.resume != 0;
+  int loops = ctl->loops;
+  CubeRoots ce;
+  ce.p1 = A.p1;
+  ce.p2 = A.p2;
+
+  {   // the workgroup's rows
+    const int z0 = A.lnz0[w], nz = A.lnz0[w + 1] - z0;
+    for (int k = tid; k < nz; k += NT) {
+      LV[k] = A.lval[z0 + k];
+      LC[k] = A.lcol[z0 + k];
+    }
+    for (int i = tid; i <= R; i += NT) LR[i] = A.lrow[r0 + w + i];
+    for (int i = tid; i < R; i += NT) {
+      Yv[i] = A.y[r0 + i];
+      YN[i] = A.yn[r0 + i];
+      FN[i] = A.fn[r0 + i];
+      B[i] = A.b[r0 + i];
+      CM[i] = A.cm[r0 + i];
+      if (resume) {
+        V1[i] = A.v1[r0 + i];
+        V2[i] = A.v2[r0 + i];
+      }
+    }
+  }
+  __syncthreads();
+
+  auto rhs = [&](int i, const double *y) {
+    double d = -B[i];
+    const double yi = y[i];
+    const int e = LR[i + 1];
+    for (int j = LR[i]; j < e; j++) d += LV[j] * (y[LC[j]] - yi);
+    return d / CM[i];
+  };
+  auto total = [&]() { return grid_sum<NT>(P, T, part, A.terms, A.parts, q, &late); };
+  // coupled cells: the neighbours' compartments of vector v into its tail.
+  // Every exchange between two sums has slots of its own; they are emptied
+  // like the sum's, after the next one.
+  int gs = 0, gs_old = ctl->ghost_used;
+  const bool coupled = A.imp0 != nullptr;
+  auto finish_sum = [&]() {
+    const double s = total();
+    if (coupled) {
+      double *old = A.ghost + (size_t)(q == 2 ? 0 : q + 1) * GHOST_STAGES * A.nslot;   // of the sum before this one
+      const int e0 = A.exp0[w], ne = A.exp0[w + 1] - e0;
+      for (int k = tid; k < ne * gs_old; k += NT) mail_clear(old + (size_t)(k / ne) * A.nslot + A.exp_slot[e0 + k % ne]);
+      gs_old = gs;
+      gs = 0;
+    }
+    return s;
+  };
+  auto fetch = [&](double *v) {
+    if (!coupled) return;
+    if (gs == GHOST_STAGES) {   // out of slots: a sum of nothing in between
+      for (int i = tid; i < R; i += NT) T[i] = 0.0;
+      finish_sum();
+    }
+    double *g = A.ghost + ((size_t)q * GHOST_STAGES + gs) * A.nslot;
+    for (int k = A.exp0[w] + tid; k < A.exp0[w + 1]; k += NT) mail_put(g + A.exp_slot[k], v[A.exp_row[k]]);
+    const int m0 = A.imp0[w], ni = A.imp0[w + 1] - m0;
+    for (int k = tid; k < ni; k += NT) v[R + k] = mail_get(g + m0 + k, &late);
+    gs++;
+    __syncthreads();
+  };
+
+  auto ion_and_b = [&](double dt) {
+    n_ion++;
+    if constexpr (Model::GAP) {
+      // the dendrites' new voltages, for the gap currents of other workgroups' cells
+      if (!P.alone) {
+        for (int c = tid; c < cells; c += NT) {
+          mail_clear(A.gap + (size_t)(gq == 2 ? 0 : gq + 1) * A.n + cell0 + c);
+          mail_put(A.gap + (size_t)gq * A.n + cell0 + c, Yv[c * A.comp]);
+        }
+      }
+    }
+    for (int i = tid; i < R; i += NT) {
+      const double vn = Yv[i];
+      B[i] = Model::ion(S, r0 + i, vn, dt, [&](int cell) {
+        if (cell >= cell0 && cell < cell0 + cells) return Yv[(cell - cell0) * A.comp];
+        return mail_get(A.gap + (size_t)gq * A.n + cell, &late);
+      });
+    }
+    gq = gq == 2 ? 0 : gq + 1;
+    if (A.refresh_fn) {
+      __syncthreads();
+      fetch(YN);
+      for (int i = tid; i < R; i += NT) FN[i] = rhs(i, YN);
+    }
+    late = __syncthreads_or(late);
+  };
+
+  // rkcrho (solve_rkc.cu:562-754)
+  auto rkcrho = [&]() {
+    const int itmax = 1000;
+    double so[3] = {0.0, 0.0, 0.0};
+    const double sqrtu = sqrt(UR), small = 1.0 / 0.125;
+    for (int i = tid; i < R; i += NT) T[i] = YN[i] * YN[i];
+    const double ynrm = sqrt(finish_sum());
+    for (int i = tid; i < R; i += NT) {
+      const double v = A.ede[r0 + i];
+      T[i] = v * v;
+    }
+    const double vnrm = sqrt(finish_sum());
+    double dynrm;
+    if (ynrm != 0.0 && vnrm != 0.0) {
+      dynrm = ynrm * sqrtu;
+      const double f = dynrm / vnrm;
+      for (int i = tid; i < R; i += NT) V1[i] = f * A.ede[r0 + i] + YN[i];
+    } else if (ynrm != 0.0) {
+      dynrm = ynrm * sqrtu;
+      for (int i = tid; i < R; i += NT) V1[i] = sqrtu * YN[i] + YN[i];
+    } else if (vnrm != 0.0) {
+      dynrm = UR;
+      const double f = dynrm / vnrm;
+      for (int i = tid; i < R; i += NT) V1[i] = f * A.ede[r0 + i];
+    } else {
+      dynrm = UR;
+      for (int i = tid; i < R; i += NT) V1[i] = dynrm;
+    }
+    double sigma = 0.0, sigmal;
+    for (int iter = 0; iter < itmax && !late; iter++) {
+      n_rho++;
+      __syncthreads();
+      fetch(V1);
+      for (int i = tid; i < R; i += NT) {
+        const double F = rhs(i, V1);
+        V2[i] = F;
+        const double d = -1.0 * FN[i] + F;
+        T[i] = d * d;
+      }
+      const double dfnrm = sqrt(finish_sum());
+      sigmal = sigma;
+      sigma = dfnrm / dynrm;
+      so[0] = so[1];
+      so[1] = so[2];
+      so[2] = sprad;
+      sprad = 1.2 * sigma;
+      bool done = iter >= 1 && fabs(sigma - sigmal) <= ((sigma > small) ? sigma : small) * 0.001;
+      if (!done && iter > itmax / 2 && fabs(so[2] - so[0]) < 0.00001 && fabs(so[1] - sprad) < 0.00001) {
+        sprad = (sprad + so[2]) / 2.0;
+        done = true;
+      }
+      if (done) {
+        for (int i = tid; i < R; i += NT) A.ede[r0 + i] = -1.0 * YN[i] + V1[i];
+        return;
+      }
+      if (dfnrm != 0.0) {
+        const double al = dynrm / dfnrm;
+        for (int i = tid; i < R; i += NT) {
+          const double t = -1.0 * V2[i] + FN[i];
+          V1[i] = al * t + YN[i];
+        }
+      } else {
+        const int id = iter % A.nc - r0;
+        if (id >= 0 && id < R && id % NT == tid) V1[id] = 2.0 * Yv[id] - V1[id];
+      }
+    }
+    idid = 6;
+  };
+
+  // step (solve_rkc.cu:815-906)
+  auto step = [&](double h, int m) {
+    double w0 = 0.0, w1 = 0.0, mus;
+    const bool tab = m >= 2 && m <= RES_COEF;
+    if (tab) {
+      const double *ct = A.coef + (size_t)m * RES_COEF * 4;
+      for (int k = tid; k < 4 * m; k += NT) C4[k] = ct[k];
+      mus = ct[0];
+    } else {
+      w0 = 1.0 + 2.0 / (13.0 * m * m);
+      const double t1 = w0 * w0 - 1.0, t2 = sqrt(t1);
+      const double arg = m * log(w0 + t2);
+      w1 = sinh(arg) * t1 / (cosh(arg) * m * t2 - w0 * sinh(arg));
+      mus = w1 * (1.0 / ((2.0 * w0) * (2.0 * w0)));
+    }
+    const double hm = h * mus;
+    for (int i = tid; i < R; i += NT) {
+      const double y0 = YN[i];
+      V2[i] = y0;
+      V1[i] = hm * FN[i] + y0;
+    }
+    n_stage++;
+    __syncthreads();
+    double bjm1 = 1.0 / ((2.0 * w0) * (2.0 * w0)), bjm2 = bjm1;
+    double zjm1 = w0, zjm2 = 1.0, dzjm1 = 1.0, dzjm2 = 0.0, d2zjm1 = 0.0, d2zjm2 = 0.0;
+    for (int j = 1; j < m; j++) {
+      double mu, nu, ajm1;
+      if (tab) {
+        mu = C4[4 * j];
+        nu = C4[4 * j + 1];
+        mus = C4[4 * j + 2];
+        ajm1 = C4[4 * j + 3];
+      } else {
+        const double zj = 2.0 * w0 * zjm1 - zjm2, dzj = 2.0 * w0 * dzjm1 - dzjm2 + 2.0 * zjm1;
+        const double d2zj = 2.0 * w0 * d2zjm1 - d2zjm2 + 4.0 * dzjm1;
+        const double bj = d2zj / (dzj * dzj);
+        ajm1 = 1.0 - zjm1 * bjm1;
+        mu = 2.0 * w0 * bj / bjm1;
+        nu = -bj / bjm2;
+        mus = mu * w1 / w0;
+        bjm2 = bjm1; bjm1 = bj;
+        zjm2 = zjm1; zjm1 = zj;
+        dzjm2 = dzjm1; dzjm1 = dzj;
+        d2zjm2 = d2zjm1; d2zjm1 = d2zj;
+      }
+      const double omn = 1.0 - mu - nu, hs = h * mus;
+      fetch(V1);
+      for (int i = tid; i < R; i += NT) {
+        const double F = rhs(i, V1);
+        Yv[i] = mu * V1[i] + nu * V2[i] + omn * YN[i] + hs * (F - ajm1 * FN[i]);
+      }
+      n_stage++;
+      double *t = V2;
+      V2 = V1;
+      V1 = Yv;
+      Yv = t;
+      __syncthreads();
+    }
+    double *t = Yv;
+    Yv = V1;
+    V1 = V2;
+    V2 = t;
+  };
+
+  // an attempt of rkclow (solve_rkc.cu:908-1096) up to its error norm
+  auto attempt = [&]() {
+    if (newspc) {
+      rkcrho();
+      if (sprad < A.rho_floor) sprad = A.rho_floor;
+      jacatt = true;
+    }
+    last = false;
+    if (1.1 * absh >= fabs(tend - lt)) {
+      absh = fabs(tend - lt);
+      last = true;
+    }
+    const double mr = sqrt(1.54 * absh * sprad + 1.0);
+    int m = (mr < mmax) ? 1 + (int)mr : (int)mmax + 1;
+    if (m > mmax) {
+      m = (int)mmax;
+      absh = (m * m - 1) / (1.54 * sprad);
+      last = false;
+    }
+    double h = absh;
+    if (h <= hmin) h = hmin;
+    h_now = h;
+    step(h, m);
+    // f(Y_m) and the error estimate (every weight is positive: atol > 0)
+    fetch(Yv);
+    for (int i = tid; i < R; i += NT) {
+      const double F = rhs(i, Yv);
+      V1[i] = F;
+      const double yi = Yv[i], yni = YN[i];
+      const double ay = fabs(yi), ayn = fabs(yni);
+      const double wt = at + rt * ((ay > ayn) ? ay : ayn);
+      const double est = 0.8 * (yni - yi) + 0.4 * h * (FN[i] + F);
+      T[i] = (est / wt) * (est / wt);
+    }
+    n_stage++;
+    err = sqrt(finish_sum() / (double)A.nc);
+  };
+
+  auto rkclow = [&]() {
+    if (!resume) loops = 0;
+    while (!late) {
+      if (resume) {
+        resume = false;
+      } else {
+        if (++loops > 1000) return;
+        attempt();
+        if (late) return;
+        if (!isfinite(err)) {
+          status = Model::NONFINITE_STATUS;
+          return;
+        }
+        ce = cube_roots(err);
+        // err^(2/3) enters an accepted step's factor only
+        const bool accepts = err <= 1.0 || !ce.sure1 || 0.8 * absh / ce.p1 < hmin;
+        if (!ce.sure1 || (accepts && !ce.sure2)) {
+          status = ASK_POW;
+          return;
+        }
+      }
+      const double h = h_now;
+      if (err > 1.0) {
+        n_rej++;
+        absh = 0.8 * absh / ce.p1;
+        if (absh < hmin) {
+          idid = 4;   // and fall through to the accept branch, as the reference does
+        } else {
+          newspc = !jacatt;
+          continue;
+        }
+      }
+      n_step++;
+      naccpt += 1;
+      lt += h;
+      gt = lt;
+      jacatt = false;
+      newspc = false;   // nstsig is never advanced in the reference
+      hw0 = h;
+      hw1 = lt;
+      double *t = V2;
+      V2 = FN;
+      FN = V1;
+      V1 = YN;
+      YN = Yv;
+      Yv = t;
+      double fac = 10.0, t1, t2;
+      if (naccpt == 1) {
+        t2 = ce.p1;
+        if (0.8 < fac * t2) fac = 0.8 / t2;
+      } else {
+        t1 = 0.8 * absh * errold3;
+        t2 = fabs(hold) * ce.p2;
+        if (t1 < fac * t2) fac = t1 / t2;
+      }
+      absh = ((0.1 > fac) ? 0.1 : fac) * absh;
+      const double hm = fmin(H, absh);
+      absh = (hmin > hm) ? hmin : hm;
+      errold = err;
+      errold3 = ce.p1;
+      hold = h;
+      idid = last ? 1 : 2;
+      return;
+    }
+  };
+
+  for (int s = 0; s < nsteps; s++) {
+    const double t = t0 + s * H;
+    for (int i = tid; i < R && !resume; i += NT) {
+      const int cell = (r0 + i) / A.comp, k = r0 + i - cell * A.comp;
+      if (A.do_stim && k == A.stim_comp) A.iext[r0 + i] = (A.stim_t0 <= t && t < A.stim_t1) ? A.amp[cell] : 0.0;
+      if (A.syn_g) {
+        const u32x4 r = philox4x32_10((uint32_t)(r0 + i), (uint32_t)(step0 + s), 0x5359u, 0u, A.k0, A.k1);
+        const double u = u01_53(r.v[0], r.v[1]);
+        A.syn_g[r0 + i] = A.syn_g[r0 + i] * A.syn_decay + ((u < A.syn_p) ? A.syn_event : 0.0);
+      }
+    }
+    if (sum_dt != 0.0 && !resume) {
+      ion_and_b(sum_dt);
+      sum_dt = 0.0;
+    }
+    while (true) {
+      rkclow();
+      if (late || status != 0) break;
+      sum_dt += gt - gt_old;
+      gt_old = gt;
+      if ((A.strict ? sum_dt > A.integ : sum_dt >= A.integ) && idid == 2.0) {
+        ion_and_b(sum_dt);
+        sum_dt = 0.0;
+      }
+      if (idid == 2.0) continue;
+      if (idid == 1.0) break;
+      status = (int)idid;
+      break;
+    }
+    if (late) status = TIMED_OUT;
+    if (status != 0) break;
+    // rkcint at gt_old (solve_rkc.cu:794-813), the recorder and the raster
+    const double tlast = hw1 - hw0, x = (gt_old - tlast) / hw0;
+    const double a1 = (1.0 + 2.0 * x) * (x - 1.0) * (x - 1.0), a2 = (3.0 - 2.0 * x) * x * x;
+    const double b1 = hw0 * x * (x - 1.0) * (x - 1.0), b2 = hw0 * (x - 1.0) * x * x;
+    for (int i = tid; i < R; i += NT) {
+      const double v = a1 * V1[i] + a2 * YN[i] + b1 * V2[i] + b2 * FN[i];
+      const int cell = (r0 + i) / A.comp, k = r0 + i - cell * A.comp;
+      A.vnew[r0 + i] = v;
+      if (A.rec) {
+        if (A.rec_comp < 0) A.rec[(size_t)s * A.nc + r0 + i] = v;
+        else if (k == A.rec_comp) A.rec[(size_t)s * A.n + cell] = v;
+      }
+      if (A.bits && k == A.raster_comp) {
+        if (v > A.thr && A.prev[cell] <= A.thr) atomicOr(&A.bits[(size_t)s * A.words + (cell >> 5)], 1u << (cell & 31));
+        A.prev[cell] = v;
+      }
+    }
+    tend += H;
+    done_steps++;
+  }
+
+  for (int i = tid; i < R; i += NT) {
+    A.y[r0 + i] = Yv[i];
+    A.yn[r0 + i] = YN[i];
+    A.fn[r0 + i] = FN[i];
+    A.b[r0 + i] = B[i];
+    if (status == ASK_POW) {
+      A.v1[r0 + i] = V1[i];
+      A.v2[r0 + i] = V2[i];
+    }
+  }
+  if ((w == 0 || status == TIMED_OUT) && tid == 0) {
+    RkcCtl c = *ctl;
+    c.o[1] = absh; c.o[2] = sprad; c.o[3] = naccpt; c.o[6] = idid; c.o[7] = gt;
+    c.o[8] = gt_old; c.o[9] = lt; c.o[10] = tend; c.o[11] = errold; c.o[12] = hold;
+    c.hw[0] = hw0; c.hw[1] = hw1;
+    c.sum_dt = sum_dt; c.errold3 = errold3; c.err = err; c.h = h_now;
+    c.steps = n_step; c.rejects = n_rej; c.stages = n_stage; c.rho_iters = n_rho; c.ions = n_ion;
+    c.macro += done_steps;
+    c.last = last; c.newspc = newspc; c.jacatt = jacatt; c.status = status;
+    c.q = q; c.ions_q = gq; c.ghost_used = gs_old; c.loops = loops;
+    *ctl = c;
+    *A.ctl_host = c;
+  }
+}
+
+}  // namespace cbrkc
