@@ -151,6 +151,11 @@ class Engine {
 // state afterwards (glibc rand() and random() share that state).
 void create_stream(hipStream_t *st);
 
+// Whether this process may launch cooperatively on the current device: the
+// barrier resource behind it belongs to one process at a time, which keeps
+// it to its end, so while another one holds it every such launch is refused.
+bool coop_available(hipStream_t st);
+
 // Tolerances and the operator-splitting interval of one population.
 struct SolverSpec {
   double atol = 1e-6, rtol = 1e-6;

@@ -42,6 +42,7 @@
 
 #include "detsum.hpp"
 #include "engine.hpp"
+#include "kry_resident.hpp"
 #include "record.hpp"
 #include "go_model.hpp"
 #include "gr_model.hpp"
@@ -72,7 +73,7 @@ struct CnSys {
   double *part, *scal;
   int *flag;
   int nc, bicg;
-  int direct;                        // 1: the per-cell tree solve replaces the Krylov loop
+  int direct;                        // 1: the per-cell tree solve or the resident kernel replaces the launches
   double dt;                         // the step [ms]: CN_DT / BE_DT, or a whole fraction of H_MAX
   SynIn syn;                         // incoming synapses (none: syn.on() false)
 };
@@ -122,6 +123,7 @@ __device__ bool block_sum_last(const CnSys &S, double x, double *lds, double *ou
 // b = r = p = bb (and the shadow vectors of BiCG); returns bb
 __device__ inline double set_rhs(const CnSys &S, int i, double bb) {
   S.b[i] = bb;
+  if (S.direct) return bb;           // the tree solve and the resident kernel start from b
   S.r[i] = bb;
   S.p[0][i] = bb;
   if (S.bicg) {
@@ -1126,6 +1128,7 @@ class CnEngine : public Engine {
     CB_HIP(hipMemset(S_.scal, 0, sizeof(double) * S_NSCAL));
     CB_HIP(hipMemset(S_.flag, 0, sizeof(int) * F_NFLAG));
     S_.nc = nc_;
+    if (!direct_) make_resident(row, col, val, dpos, trow, tcol, tsrc, bicg);
     S_.bicg = bicg ? 1 : 0;
     S_.dt = dt_;
     amp_ = dup(stim_.amp);
@@ -1133,6 +1136,8 @@ class CnEngine : public Engine {
   }
   ~CnEngine() override {
     (void)hipStreamSynchronize(st_);
+    for (void *p : res_bufs_) (void)hipFree(p);
+    if (late_host_) (void)hipHostFree(late_host_);
     for (const void *p : {(const void *)S_.row, (const void *)S_.col, (const void *)S_.dpos, (const void *)S_.val,
                           (const void *)S_.trow, (const void *)S_.tcol, (const void *)S_.tsrc, (const void *)S_.cm,
                           (const void *)S_.v, (const void *)S_.vold, (const void *)S_.iext, (const void *)S_.gamma1,
@@ -1210,6 +1215,8 @@ class CnEngine : public Engine {
     return HINES_WAVE;
   }
   std::string mapping() const override {
+    if (res_fn_)
+      return "Krylov solve in one kernel, " + std::to_string(res_grid_) + " workgroups of " + std::to_string(A_.rb) + " rows";
     if (!direct_) return nb_ <= KRY_SMALL_BLOCKS ? "Krylov solve in one workgroup" : "Krylov solve, two launches per iteration";
     std::string m = chain_ ? "tree solve by unbranched runs, one lane per run, one wavefront per cell"
                            : "tree solve level by level, one wavefront per cell";
@@ -1224,6 +1231,12 @@ class CnEngine : public Engine {
     prep();
     if (direct_) {
       tree_solve(chain_, S_.diag, S_.b, S_.v);
+    } else if (res_fn_) {
+      void *args[] = {&A_};
+      if (res_grid_ == 1)
+        CB_HIP(hipLaunchKernel(res_fn_, dim3(1), dim3(res_nt_), args, res_lds_, st_));
+      else   // the workgroups wait for one another: all of them resident at once
+        CB_HIP(hipLaunchCooperativeKernel(res_fn_, dim3(res_grid_), dim3(res_nt_), args, (unsigned)res_lds_, st_));
     } else if (nb_ <= KRY_SMALL_BLOCKS) {
       k_kry_small<<<1, NB, 0, st_>>>(S_);
     } else {
@@ -1277,6 +1290,7 @@ class CnEngine : public Engine {
     CB_HIP(hipStreamSynchronize(st_));
     if (drec) CB_HIP(hipFree(drec));
     if (dbits) CB_HIP(hipFree(dbits));
+    check_late();
     if (raster) append_spikes(bits, nsteps, words, t0, H_MAX);
   }
   const double *device_vnew() const override { return S_.v; }
@@ -1301,10 +1315,174 @@ class CnEngine : public Engine {
     }
     if (!src) throw Error("field not available for this population");
     CB_HIP(hipStreamSynchronize(st_));
+    check_late();
     CB_HIP(hipMemcpy(dst, src, sizeof(double) * nc_, hipMemcpyDeviceToHost));
   }
 
  protected:
+  void check_late() const {
+    if (late_host_ && *(volatile int *)late_host_) throw Error("CN / BE: a workgroup of the solve waited for another one in vain");
+  }
+
+  template <typename T>
+  T *res_put(const std::vector<T> &h) {
+    T *d = dup(h);
+    res_bufs_.push_back((void *)d);
+    return d;
+  }
+
+  // The resident kernel's shape and tables.  One workgroup of 1024 threads when
+  // the rows fit it and its LDS (no exchange between workgroups), else
+  // workgroups of 512 threads with as few rows per thread as leave at most one
+  // workgroup per CU.  Larger systems, and those of several workgroups in a
+  // process that may not launch cooperatively, stay on the launches per
+  // iteration.
+  void make_resident(const std::vector<int> &row, const std::vector<int> &col, const std::vector<double> &val,
+                     const std::vector<int> &dpos, const std::vector<int> &trow, const std::vector<int> &tcol,
+                     const std::vector<int> &tsrc, bool bicg) {
+    int dev = 0, ncu = 0, lds_max = 0;
+    CB_HIP(hipGetDevice(&dev));
+    CB_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+    CB_HIP(hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
+    const int nch = (nc_ + NB - 1) / NB;
+    if (nch > 2048) return;
+    for (int shape = 0; shape < 4; shape++) {
+      const int nt = shape == 0 ? 1024 : 512, k = shape == 0 ? 4 : 1 << (shape - 1);
+      const int rb = shape == 0 ? nch * NB : nt * k, grid = (nc_ + rb - 1) / rb;
+      if (rb > nt * k || grid > ncu) continue;
+      if (plan_resident(row, col, val, dpos, trow, tcol, tsrc, bicg, nt, k, rb, grid, (size_t)lds_max)) return;
+    }
+  }
+
+  static const void *kry_kernel(int nt, int k, bool bicg) {
+    if (nt == 1024) return bicg ? (const void *)k_kry_resident<1024, 4, true> : (const void *)k_kry_resident<1024, 4, false>;
+    switch (k) {
+      case 1: return bicg ? (const void *)k_kry_resident<512, 1, true> : (const void *)k_kry_resident<512, 1, false>;
+      case 2: return bicg ? (const void *)k_kry_resident<512, 2, true> : (const void *)k_kry_resident<512, 2, false>;
+    }
+    return bicg ? (const void *)k_kry_resident<512, 4, true> : (const void *)k_kry_resident<512, 4, false>;
+  }
+
+  bool plan_resident(const std::vector<int> &row, const std::vector<int> &col, const std::vector<double> &val,
+                     const std::vector<int> &dpos, const std::vector<int> &trow, const std::vector<int> &tcol,
+                     const std::vector<int> &tsrc, bool bicg, int nt, int k, int rb, int grid, size_t lds_max) {
+    KryArgs a{};
+    a.nc = nc_;
+    a.nch = (nc_ + NB - 1) / NB;
+    a.rb = rb;
+    std::vector<unsigned short> lrow, lcol, ldpos(nc_), tr, tc, tdpos(nc_);
+    std::vector<double> lval, tv;
+    std::vector<int> lnz0(1, 0), imp0(1, 0), imp;
+    std::vector<int> at(nc_, -1);   // ghost index of a row in the present workgroup
+    for (int w = 0; w < grid; w++) {
+      const int r0 = w * rb, r1 = std::min(nc_, r0 + rb), z0 = lnz0[w];
+      const size_t m0 = imp.size();
+      auto local = [&](int c) {
+        if (c >= r0 && c < r1) return c - r0;
+        if (at[c] < 0) {
+          at[c] = (int)(imp.size() - m0);
+          imp.push_back(c);
+        }
+        return rb + at[c];
+      };
+      for (int i = r0; i < r0 + rb; i++) {   // (rows past the last one are empty)
+        lrow.push_back((unsigned short)((int)lval.size() - z0));
+        tr.push_back(lrow.back());
+        if (i >= r1) continue;
+        // the sparsity is symmetric, so a row of the transpose has the row's columns
+        if (trow[i + 1] - trow[i] != row[i + 1] - row[i]) return false;
+        for (int e = 0; e < row[i + 1] - row[i]; e++) {
+          const int j = row[i] + e, t = trow[i] + e;
+          if (j == dpos[i]) ldpos[i] = (unsigned short)((int)lval.size() - z0);
+          if (tcol[t] == i) tdpos[i] = (unsigned short)((int)lval.size() - z0);
+          const int lc = local(col[j]), lt = local(tcol[t]);
+          if (lc > 65535 || lt > 65535) return false;
+          lcol.push_back((unsigned short)lc);
+          lval.push_back(val[j]);
+          tc.push_back((unsigned short)lt);
+          tv.push_back(val[tsrc[t]]);
+        }
+      }
+      const int nz = (int)lval.size() - z0;
+      if (nz > 65535) return false;
+      lrow.push_back((unsigned short)nz);
+      tr.push_back((unsigned short)nz);
+      lnz0.push_back((int)lval.size());
+      for (size_t g = m0; g < imp.size(); g++) at[imp[g]] = -1;
+      imp0.push_back((int)imp.size());
+      a.nnz_max = std::max(a.nnz_max, nz);
+      a.ghost_max = std::max(a.ghost_max, (int)(imp.size() - m0));
+    }
+    const size_t m = bicg ? 2 : 1;
+    size_t lds = sizeof(double) * (m * (rb + a.ghost_max) + rb + a.nch + 8 + m * a.nnz_max) +
+                 sizeof(unsigned short) * m * (rb + 1 + a.nnz_max);
+    lds = (lds + 15) & ~(size_t)15;
+    if (lds > lds_max) return false;
+    const void *fn = kry_kernel(nt, k, bicg);
+    CB_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    int fit = 0;
+    CB_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, fn, nt, lds));
+    if (fit < 1 || (grid > 1 && !coop_available(st_))) return false;
+    a.nslot = (int)imp.size();
+    if (a.nslot > 0) {
+      std::vector<std::vector<std::pair<int, int>>> out(grid);   // (thread, row and slot) of each workgroup
+      for (int s = 0; s < a.nslot; s++) out[imp[s] / rb].push_back({imp[s] % rb % nt, s});
+      std::vector<int> exp0(1, 0), et(1, 0), er, es;
+      for (auto &o : out) {
+        std::stable_sort(o.begin(), o.end());
+        size_t n = 0;
+        for (int t = 0; t < nt; t++) {
+          for (; n < o.size() && o[n].first == t; n++) {
+            er.push_back(imp[o[n].second] % rb);
+            es.push_back(o[n].second);
+          }
+          et.push_back((int)er.size());
+        }
+        exp0.push_back((int)er.size());
+      }
+      a.imp0 = res_put(imp0);
+      a.imp = res_put(imp);
+      a.exp0 = res_put(exp0);
+      a.exp_t0 = res_put(et);
+      a.exp_row = res_put(er);
+      a.exp_slot = res_put(es);
+    }
+    unsigned long long e = MAIL_EMPTY;
+    double empty;
+    std::memcpy(&empty, &e, sizeof(empty));
+    a.ghost = res_put(std::vector<double>((size_t)6 * std::max(1, a.nslot), empty));
+    a.parts = res_put(std::vector<double>((size_t)3 * a.nch, empty));
+    a.q = res_put(std::vector<unsigned>(1, 0u));
+    a.lrow = res_put(lrow);
+    a.lcol = res_put(lcol);
+    a.ldpos = res_put(ldpos);
+    a.lval = res_put(lval);
+    a.lnz0 = res_put(lnz0);
+    if (bicg) {
+      a.trow = res_put(tr);
+      a.tcol = res_put(tc);
+      a.tdpos = res_put(tdpos);
+      a.tval = res_put(tv);
+    }
+    CB_HIP(hipHostMalloc((void **)&late_host_, sizeof(int), hipHostMallocMapped | hipHostMallocCoherent));
+    *late_host_ = 0;
+    CB_HIP(hipHostGetDevicePointer((void **)&a.late, late_host_, 0));
+    a.diag = S_.diag;
+    a.b = S_.b;
+    a.v = S_.v;
+    a.flag = S_.flag;
+    a.f_done = F_DONE;
+    a.f_iters = F_ITERS;
+    a.f_total = F_TOTAL;
+    A_ = a;
+    res_lds_ = lds;
+    res_grid_ = grid;
+    res_nt_ = nt;
+    res_fn_ = fn;
+    S_.direct = 1;
+    return true;
+  }
+
   virtual void prep() = 0;
   virtual const double *model_field(int) const { return nullptr; }
   virtual bool takes_synapses() const { return true; }
@@ -1331,6 +1509,13 @@ class CnEngine : public Engine {
   bool chain_ = false;   // the solve by unbranched runs is in use
   bool has_chain_ = false;   // every cell at most CHAIN_SEGS runs: the run walk applies
   double tune_ms_[2] = {0.0, 0.0};
+  // the resident Krylov kernel (null: launches per iteration)
+  const void *res_fn_ = nullptr;
+  KryArgs A_{};
+  size_t res_lds_ = 0;
+  int res_grid_ = 0, res_nt_ = 0;
+  std::vector<void *> res_bufs_;
+  int *late_host_ = nullptr;
   double *amp_ = nullptr, *rec_ = nullptr;
   hipStream_t st_{};
   Stats st;

@@ -18,6 +18,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstdlib>
 
 #include <cmath>
@@ -341,23 +342,6 @@ __global__ void __launch_bounds__(256) k_gr_ion_b(GrState S, const double *__res
 }
 
 __global__ void k_coop_probe() {}
-
-// Whether this process may launch cooperatively on the current device: the
-// barrier resource behind it belongs to one process at a time, which keeps
-// it to its end, so while another one holds it every such launch is refused.
-bool coop_available(hipStream_t st) {
-  int dev = 0, coop = 0;
-  CB_HIP(hipGetDevice(&dev));
-  CB_HIP(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev));
-  if (!coop) return false;
-  const hipError_t e = hipLaunchCooperativeKernel((const void *)k_coop_probe, dim3(1), dim3(64), nullptr, 0, st);
-  if (e != hipSuccess) {
-    (void)hipGetLastError();
-    return false;
-  }
-  CB_HIP(hipStreamSynchronize(st));
-  return true;
-}
 
 // The models of the resident kernel.  512 threads hold a Purkinje cell's 1600
 // compartments four to a thread; the granule and Golgi updates keep their 12 x 12
@@ -1409,6 +1393,23 @@ void create_stream(hipStream_t *st) {
   const hipError_t e = hipStreamCreate(st);
   setstate(caller);
   CB_HIP(e);
+}
+
+bool coop_available(hipStream_t st) {
+  static std::atomic<bool> granted[64];   // per device, once and for the process's life
+  int dev = 0, coop = 0;
+  CB_HIP(hipGetDevice(&dev));
+  if (dev >= 0 && dev < 64 && granted[dev]) return true;
+  CB_HIP(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev));
+  if (!coop) return false;
+  const hipError_t e = hipLaunchCooperativeKernel((const void *)k_coop_probe, dim3(1), dim3(64), nullptr, 0, st);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  CB_HIP(hipStreamSynchronize(st));
+  if (dev >= 0 && dev < 64) granted[dev] = true;
+  return true;
 }
 
 void Engine::set_raster(int comp, double thr) {
