@@ -345,42 +345,40 @@ __global__ void k_coop_probe() {}
 
 // The models of the resident kernel.  512 threads hold a Purkinje cell's 1600
 // compartments four to a thread; the granule and Golgi updates keep their 12 x 12
-// and 6 x 6 systems in registers, which takes one wave per SIMD.
+// and 6 x 6 systems in registers, which takes one wave per SIMD.  K0 <= K1 <= K2:
+// the rows per thread a kernel is built for (0: none).
 struct PkjModel {
   using State = PkjState;
-  static constexpr int NT = 512, NONFINITE_STATUS = NONFINITE;
+  static constexpr int NT = 512, K0 = 0, K1 = 0, K2 = 4, NONFINITE_STATUS = NONFINITE;
   static constexpr bool GAP = false;
-  template <class Dend>
-  __device__ static double ion(State S, int i, double vn, double dt, Dend) {
+  __device__ __attribute__((noinline)) static double ion(const State *Sp, int i, double vn, double dt, GapView *) {
+    State S = *Sp;
     if (S.net_s) S.net_decay = exp(-dt / 0.6);
     return pkj_ion_current(S, i, vn, dt, true);
   }
 };
 struct IoModel {
   using State = IoState;
-  static constexpr int NT = 256, NONFINITE_STATUS = NONFINITE;
+  static constexpr int NT = 256, K0 = 0, K1 = 1, K2 = 7, NONFINITE_STATUS = NONFINITE;
   static constexpr bool GAP = true;
-  template <class Dend>
-  __device__ static double ion(const State &S, int i, double vn, double dt, Dend dend) {
-    return io_ion_gap_current(S, i, vn, dt, true, dend);
+  __device__ __forceinline__ static double ion(const State *S, int i, double vn, double dt, GapView *gap) {
+    return io_ion_gap_current(*S, i, vn, dt, true, [&](int cell) { return (*gap)(cell); });
   }
 };
 struct GoModel {
   using State = GoState;
-  static constexpr int NT = 256, NONFINITE_STATUS = NONFINITE;
+  static constexpr int NT = 256, K0 = 0, K1 = 1, K2 = 7, NONFINITE_STATUS = NONFINITE;
   static constexpr bool GAP = false;
-  template <class Dend>
-  __device__ static double ion(const State &S, int i, double vn, double dt, Dend) {
-    return go_ion_net_current(S, i, vn, dt, true);
+  __device__ __forceinline__ static double ion(const State *S, int i, double vn, double dt, GapView *) {
+    return go_ion_net_current(*S, i, vn, dt, true);
   }
 };
 struct GrModel {
   using State = GrState;
-  static constexpr int NT = 256, NONFINITE_STATUS = NONFINITE;
+  static constexpr int NT = 256, K0 = 1, K1 = 3, K2 = 7, NONFINITE_STATUS = NONFINITE;
   static constexpr bool GAP = false;
-  template <class Dend>
-  __device__ static double ion(const State &S, int i, double vn, double dt, Dend) {
-    return gr_ion_net_current(S, i, vn, dt, true);
+  __device__ __attribute__((noinline)) static double ion(const State *S, int i, double vn, double dt, GapView *) {
+    return gr_ion_net_current(*S, i, vn, dt, true);
   }
 };
 
@@ -663,20 +661,40 @@ class GlobalRkc : public Engine {
   // the cell type's resident kernel: its threads per workgroup and address,
   // and a launch of it with the type's state
   virtual int res_threads() const = 0;
-  virtual const void *res_kernel() const = 0;
+  virtual int res_rows() const = 0;   // most rows per thread
   virtual void res_launch(const RkcArgs &a, int nsteps, double t0, int step0) = 0;
   virtual bool res_strict() const { return false; }
 
+  // the kernel for k rows per thread (the next of the model's shapes)
   template <class Model>
-  void launch_model(const RkcArgs &a, const typename Model::State &S, int nsteps, double t0, int step0) {
+  static const void *kernel_of(int k) {
+    if constexpr (Model::K0 > 0)
+      if (k <= Model::K0) return (const void *)k_rkc_steps<Model, Model::K0>;
+    if constexpr (Model::K1 > 0)
+      if (k <= Model::K1) return (const void *)k_rkc_steps<Model, Model::K1>;
+    return (const void *)k_rkc_steps<Model, Model::K2>;
+  }
+  virtual const void *res_kernel(int k) const = 0;
+
+  template <class State>
+  void launch_model(const RkcArgs &a, const State &S, int nsteps, double t0, int step0) {
+    // the kernel reads the model's pointers from device memory; they change
+    // when synapses are attached
+    if (!state_dev_) {
+      CB_HIP(hipMalloc(&state_dev_, sizeof(State)));
+      res_bufs_.push_back(state_dev_);
+    }
+    if (state_host_.size() != sizeof(State) || std::memcmp(state_host_.data(), &S, sizeof(State)) != 0) {
+      state_host_.assign((const char *)&S, (const char *)&S + sizeof(State));
+      CB_HIP(hipMemcpyAsync(state_dev_, state_host_.data(), sizeof(State), hipMemcpyHostToDevice, st_));
+    }
     RkcArgs av = a;
-    typename Model::State sv = S;
+    const State *sv = (const State *)state_dev_;
     void *args[] = {&av, &sv, &nsteps, &t0, &step0};
-    const void *f = (const void *)k_rkc_steps<Model>;
     if (a.nblk == 1)
-      CB_HIP(hipLaunchKernel(f, dim3(1), dim3(Model::NT), args, res_lds_, st_));
+      CB_HIP(hipLaunchKernel(res_fn_, dim3(1), dim3(res_threads()), args, res_lds_, st_));
     else   // the workgroups wait for one another: all of them resident at once
-      CB_HIP(hipLaunchCooperativeKernel(f, dim3(a.nblk), dim3(Model::NT), args, (unsigned)res_lds_, st_));
+      CB_HIP(hipLaunchCooperativeKernel(res_fn_, dim3(a.nblk), dim3(res_threads()), args, (unsigned)res_lds_, st_));
   }
 
   // waits for the launch, takes the kernel's question if it stopped for one
@@ -739,47 +757,59 @@ class GlobalRkc : public Engine {
     a.nch = (nc_ + RED_BLOCK - 1) / RED_BLOCK;
     if (a.nch > 2048) return;
     const int RM = a.cpb * comp_;
-    if (RM > 4096) return;   // (local indices have 16 bits)
+    if (RM > NT * res_rows()) return;
     // local rows, ghosts and who posts them
-    std::vector<unsigned short> lrow, lcol;
-    std::vector<double> lval;
-    std::vector<int> lnz0(1, 0), imp0(1, 0), imp;
+    std::vector<uint2> lcol(nc_);
+    std::vector<double> lval((size_t)ROW_W * nc_, 0.0), xval;
+    std::vector<unsigned short> xcol;
+    std::vector<int> x0(1, 0), imp0(1, 0), imp, at(nc_, -1);
     auto block_of = [&](int r) { return r / RM; };
     for (int w = 0; w < a.nblk; w++) {
       const int r0 = w * RM, r1 = std::min(nc_, r0 + RM), R = r1 - r0;
       const size_t m0 = imp.size();
       for (int i = r0; i < r1; i++) {
-        lrow.push_back((unsigned short)((int)lval.size() - lnz0[w]));
+        unsigned c4[4] = {(unsigned)(i - r0), (unsigned)(i - r0), (unsigned)(i - r0), 0u};
+        const unsigned xs = (unsigned)((int)xval.size() - x0[w]);
+        int e = 0;
         for (int j = row_h_[i]; j < row_h_[i + 1]; j++) {
           const int c = col_h_[j];
           if (c == i) continue;   // the stored diagonal adds val (y_i - y_i) = 0
           int l = c - r0;
           if (c < r0 || c >= r1) {
-            size_t k = m0;
-            while (k < imp.size() && imp[k] != c) k++;
-            if (k == imp.size()) imp.push_back(c);
-            l = R + (int)(k - m0);
+            if (at[c] < 0) {
+              at[c] = (int)(imp.size() - m0);
+              imp.push_back(c);
+            }
+            l = R + at[c];
           }
-          lcol.push_back((unsigned short)l);
-          lval.push_back(val_h_[j]);
+          if (e < ROW_W) {
+            c4[e] = (unsigned)l;
+            lval[(size_t)e * nc_ + i] = val_h_[j];
+          } else {
+            xcol.push_back((unsigned short)l);
+            xval.push_back(val_h_[j]);
+          }
+          e++;
         }
+        if (e > ROW_W) c4[3] = xs << 4 | (unsigned)(e - ROW_W);
+        if (e > ROW_W + 15 || xs > 4095u || R + (int)(imp.size() - m0) > 65535) return;
+        lcol[i] = make_uint2(c4[0] | c4[1] << 16, c4[2] | c4[3] << 16);
       }
-      const int nz = (int)lval.size() - lnz0[w];
-      if (nz > 65535 || imp.size() - m0 > 4096) return;
-      lrow.push_back((unsigned short)nz);
-      lnz0.push_back((int)lval.size());
+      for (size_t g = m0; g < imp.size(); g++) at[imp[g]] = -1;
+      x0.push_back((int)xval.size());
       imp0.push_back((int)imp.size());
-      a.nnz_max = std::max(a.nnz_max, nz);
+      a.ext_max = std::max(a.ext_max, x0[w + 1] - x0[w]);
       a.ghost_max = std::max(a.ghost_max, (int)(imp.size() - m0));
     }
     const int RS = RM + a.ghost_max;
-    res_lds_ = sizeof(double) * ((size_t)5 * RS + 3 * RM + RED_BLOCK + a.nch + 8 + 4 * RES_COEF + a.nnz_max) +
-               sizeof(unsigned short) * ((size_t)RM + 1 + a.nnz_max);
+    res_lds_ = sizeof(double) * ((size_t)5 * RS + RM + RED_BLOCK + a.nch + 8 + 4 * RES_COEF + a.ext_max) +
+               sizeof(unsigned short) * a.ext_max;
     res_lds_ = (res_lds_ + 15) & ~(size_t)15;
     if (res_lds_ > (size_t)lds_max) return;
-    CB_HIP(hipFuncSetAttribute(res_kernel(), hipFuncAttributeMaxDynamicSharedMemorySize, (int)res_lds_));
+    res_fn_ = res_kernel((RM + NT - 1) / NT);
+    CB_HIP(hipFuncSetAttribute(res_fn_, hipFuncAttributeMaxDynamicSharedMemorySize, (int)res_lds_));
     int fit = 0;
-    CB_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, res_kernel(), NT, res_lds_));
+    CB_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, res_fn_, NT, res_lds_));
     if (fit < 1 || (a.nblk > 1 && !coop_available(st_))) return;
     const int nslot = (int)imp.size();
     if (nslot > 0) {
@@ -801,10 +831,11 @@ class GlobalRkc : public Engine {
       a.ghost = empty_mail((size_t)3 * GHOST_STAGES * nslot);
       a.nslot = nslot;
     }
-    a.lrow = res_put(lrow);
     a.lcol = res_put(lcol);
     a.lval = res_put(lval);
-    a.lnz0 = res_put(lnz0);
+    a.xcol = res_put(xcol);
+    a.xval = res_put(xval);
+    a.x0 = res_put(x0);
     if (a.nblk > 1) {
       a.terms = empty_mail((size_t)3 * nc_);
       a.parts = empty_mail((size_t)3 * a.nch);
@@ -1171,6 +1202,9 @@ class GlobalRkc : public Engine {
   bool resident_ = false;
   RkcArgs A_{};
   RkcCtl *ctl_host_ = nullptr;   // written by the kernel as it ends
+  const void *res_fn_ = nullptr;
+  void *state_dev_ = nullptr;    // the model's state struct, and what is in it
+  std::vector<char> state_host_;
   size_t res_lds_ = 0;
   long macro_ = 0;
   std::vector<void *> res_bufs_;
@@ -1205,9 +1239,10 @@ class GlobalPkj : public GlobalRkc {
     return s;
   }
   int res_threads() const override { return PkjModel::NT; }
-  const void *res_kernel() const override { return (const void *)k_rkc_steps<PkjModel>; }
+  int res_rows() const override { return PkjModel::K2; }
+  const void *res_kernel(int k) const override { return kernel_of<PkjModel>(k); }
   void res_launch(const RkcArgs &a, int nsteps, double t0, int step0) override {
-    launch_model<PkjModel>(a, PkjState{v_, ca_, rev_, iext_, shell_, cond_, gate_, b_, syn_g_, syn_.e_syn, nc_,
+    launch_model(a, PkjState{v_, ca_, rev_, iext_, shell_, cond_, gate_, b_, syn_g_, syn_.e_syn, nc_,
                                      net_.on() ? net_s_ : nullptr, 0.0}, nsteps, t0, step0);
   }
   void model_b(const double *vv, bool do_ion, double dt) override {
@@ -1258,10 +1293,11 @@ class GlobalIo : public GlobalRkc {
   }
   bool trigger() const override { return sum_dt_ > integ_; }   // strict for IO, solve_rkc.cu:1347
   int res_threads() const override { return IoModel::NT; }
-  const void *res_kernel() const override { return (const void *)k_rkc_steps<IoModel>; }
+  int res_rows() const override { return IoModel::K2; }
+  const void *res_kernel(int k) const override { return kernel_of<IoModel>(k); }
   bool res_strict() const override { return true; }
   void res_launch(const RkcArgs &a, int nsteps, double t0, int step0) override {
-    launch_model<IoModel>(a, IoState{v_, ca_, iext_, cond_, gate_, compart_, nbr_, b_, syn_g_, syn_.e_syn, nc_, n_}, nsteps, t0, step0);
+    launch_model(a, IoState{v_, ca_, iext_, cond_, gate_, compart_, nbr_, b_, syn_g_, syn_.e_syn, nc_, n_}, nsteps, t0, step0);
   }
   void model_b(const double *vv, bool do_ion, double dt) override {
     IoState S{v_, ca_, iext_, cond_, gate_, compart_, nbr_, b_, syn_g_, syn_.e_syn, nc_, n_};
@@ -1306,9 +1342,10 @@ class GlobalGo : public GlobalRkc {
     return s;
   }
   int res_threads() const override { return GoModel::NT; }
-  const void *res_kernel() const override { return (const void *)k_rkc_steps<GoModel>; }
+  int res_rows() const override { return GoModel::K2; }
+  const void *res_kernel(int k) const override { return kernel_of<GoModel>(k); }
   void res_launch(const RkcArgs &a, int nsteps, double t0, int step0) override {
-    launch_model<GoModel>(a, GoState{v_, ca_, ca2_, rev_, ca_old_, iext_, area_, cond_, gate_, b_, syn_g_, syn_.e_syn, nc_,
+    launch_model(a, GoState{v_, ca_, ca2_, rev_, ca_old_, iext_, area_, cond_, gate_, b_, syn_g_, syn_.e_syn, nc_,
                                    net_.on() ? net_s_ : nullptr}, nsteps, t0, step0);
   }
   void model_b(const double *vv, bool do_ion, double dt) override {
@@ -1361,10 +1398,11 @@ class GlobalGr : public GlobalRkc {
   }
   bool trigger() const override { return sum_dt_ > integ_; }   // strict for GR, solve_rkc.cu:1148
   int res_threads() const override { return GrModel::NT; }
-  const void *res_kernel() const override { return (const void *)k_rkc_steps<GrModel>; }
+  int res_rows() const override { return GrModel::K2; }
+  const void *res_kernel(int k) const override { return kernel_of<GrModel>(k); }
   bool res_strict() const override { return true; }
   void res_launch(const RkcArgs &a, int nsteps, double t0, int step0) override {
-    launch_model<GrModel>(a, GrState{v_, iext_, ca_, compart_, cond_, gate_, na_, b_, syn_g_, syn_.e_syn, nc_, net_}, nsteps, t0, step0);
+    launch_model(a, GrState{v_, iext_, ca_, compart_, cond_, gate_, na_, b_, syn_g_, syn_.e_syn, nc_, net_}, nsteps, t0, step0);
   }
   void model_b(const double *vv, bool do_ion, double dt) override {
     GrState S{v_, iext_, ca_, compart_, cond_, gate_, na_, b_, syn_g_, syn_.e_syn, nc_,

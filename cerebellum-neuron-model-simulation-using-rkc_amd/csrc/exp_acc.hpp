@@ -92,13 +92,6 @@ __host__ __device__ inline double exp_acc(double x) {
   return ldexp(acc.hi + acc.lo, (int)k);
 }
 
-// exp_acc out of line, for the arguments exp_cr cannot decide (inlined at
-// the models' sixty-odd exponentials it would be most of their code)
-#ifdef __HIPCC__
-__host__ __device__ __attribute__((noinline))
-#endif
-static double exp_acc_rare(double x) { return exp_acc(x); }
-
 // The same correctly rounded exp in a sixth of the operations, by Ziv's
 // method: a result accurate enough to round nearly always, its error bound
 // tested against the rounding, and exp_acc for what the test leaves open.
@@ -109,9 +102,9 @@ static double exp_acc_rare(double x) { return exp_acc(x); }
 // 2^-68 in all, against the 2^-67 tested, which leaves one argument in 8000
 // to exp_acc.  Both return the double nearest to exp(x), so the results are
 // the same bit for bit.
-// Measured, calls of Population.run (us): 8x8 olive cells, 40 RKC steps, 6466 ->
-// 4059; 256 granule cells, 8 intervals of Crank-Nicolson on the tree solve,
-// 8062 -> 5821; 256 Golgi cells, 40 RKC steps, 45370 -> 40310.
+// Measured, one update of 33536 Golgi compartments (39 distinct exponentials):
+// 69 us with exp_acc at every place, 31 with exp_cr inlined there, 25 with one
+// copy of it (exp_call below).
 __host__ __device__ inline double exp_cr(double x) {
   if (!(x > -708.0 && x < 709.0)) return exp(x);
   const double L1 = 0.6931471806019545, L2 = -4.2009150726810846e-11, L3 = -1.3124698417785255e-27;
@@ -143,7 +136,7 @@ __host__ __device__ inline double exp_cr(double x) {
   }
   const double d = h * 6.7762635780344027e-21;   // 2^-67
   const double up = h + (l + d), dn = h + (l - d);
-  if (up != dn) return exp_acc_rare(x);
+  if (up != dn) return exp_acc(x);
   return ldexp(up, (int)k);
 }
 
@@ -162,7 +155,12 @@ static inline double mexp(double x) { return exp_cr(x); }
 static inline double mexp(double x) { return ::exp(x); }
 #else
 __host__ inline double mexp(double x) { return ::exp(x); }
-__device__ inline double mexp(double x) { return exp_cr(x); }
+// One function rather than sixty-odd copies: a model's update is then a few
+// thousand instructions and fits the instruction cache, and equal arguments (a
+// gate's rates enter its steady state and its time constant) are evaluated
+// once.
+__device__ __attribute__((noinline, const)) static double exp_call(double x) { return exp_cr(x); }
+__device__ inline double mexp(double x) { return exp_call(x); }
 #endif
 
 }  // namespace cbrkc

@@ -12,9 +12,11 @@
 // (gap junctions) also exchange the coupled compartments' values at every
 // stage.  The additions of every right-hand side, stage and norm are those of
 // the launch-per-stage path in the same order, so the two agree bit for bit.
-// Measured, calls of Population.run (us): 16 granule cells, one macro step,
-// 29260 -> 13690; 256 Golgi cells, 40 steps, 84390 -> 45370; 64 coupled
-// Purkinje cells, 8 steps, 2875 -> 2179; 9 uncoupled ones 8225 -> 6842.
+// Measured, Population.run from the initial state and then on average over the
+// next passes (ms): 64 olive cells, 40 macro steps, 81.4 / 13.7 -> 11.9 / 3.1;
+// 256 Golgi cells, 40 steps, 22.7 / 65.1 -> 8.6 / 24.5; 16 granule cells, one
+// step, 39.0 / 25.9 -> 12.0 / 8.3; 64 coupled Purkinje cells, 8 steps, 10.0 /
+// 3.1 -> 4.9 / 1.7; 9 uncoupled ones 6.8 / 9.0 -> 3.9 / 5.4.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -41,19 +43,23 @@ struct RkcCtl {
 // ones run the recurrence in the kernel
 constexpr int ASK_POW = 9;   // status: the host has to give the powers of err
 constexpr int RES_COEF = 128;
+constexpr int ROW_W = 3;            // neighbours of a compartment held in registers (parent and two children)
 constexpr int GHOST_STAGES = 136;   // exchanges of coupled values between two sums
 
 struct RkcArgs {
   int n, nc, comp, nblk, cpb;            // cells, rows, rows per cell, workgroups, cells per workgroup
-  int nnz_max, ghost_max, nch;           // LDS sizes: matrix entries and ghosts of a workgroup, chunks
+  int ext_max, ghost_max, nch;           // LDS sizes: further entries and ghosts of a workgroup, chunks
   const int *row, *col;                  // CSR of the cable matrix
   const double *val;
-  // the same rows with local columns: rows of workgroup w start at lrow[its
-  // first row + w], entries without the diagonal, columns local (ghosts from
-  // the workgroup's row count on)
-  const unsigned short *lrow, *lcol;
+  // the same rows without the diagonal, columns local (ghosts from the
+  // workgroup's row count on): the first ROW_W entries of row i in lval[k nc + i]
+  // and the 16-bit quarters of lcol[i], whose last holds the row's further
+  // entries, start << 4 | count, in the workgroup's xcol / xval
+  const uint2 *lcol;
   const double *lval;
-  const int *lnz0;                       // first entry of each workgroup (nblk + 1)
+  const unsigned short *xcol;
+  const double *xval;
+  const int *x0;                         // first further entry of each workgroup (nblk + 1)
   const int *imp0, *exp0, *exp_row, *exp_slot;   // ghosts fetched, rows posted (null: uncoupled cells)
   double *ghost;                         // [3][GHOST_STAGES][nslot]
   int nslot;
@@ -125,10 +131,28 @@ __device__ inline CubeRoots cube_roots(double x) {
   return r;
 }
 
-// Model: NT threads, the state struct, ion(S, i, vn, dt) = ion update and
-// frozen current of row i, GAP = the olive's explicit gap currents.
-template <class Model>
-__global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, typename Model::State S, int nsteps, double t0,
+// The voltages behind the olive's explicit gap currents: a cell's dendrite in
+// the workgroup's vector or in the mailbox
+struct GapView {
+  const double *y, *gap;
+  int cell0, cells, comp, late;
+  __device__ double operator()(int cell) {
+    if (cell >= cell0 && cell < cell0 + cells) return y[(cell - cell0) * comp];
+    return mail_get(gap + cell, &late);
+  }
+};
+
+// Model: NT threads, the state struct, ion(S, i, vn, dt, gap) = ion update and
+// frozen current of row i, GAP = the olive's explicit gap currents.  The
+// update takes up to 430 registers, so nothing lives across it: the controller
+// stays in LDS (a copy for every wave), the thread's matrix rows are read again
+// after it, and it is inlined at one place only.
+// K: rows per thread (thread t owns rows t, t + NT, ...).  A thread's matrix
+// rows, capacitances and frozen currents stay in its registers, so a stage
+// reads the vectors only, all K rows' reads before the first use: from LDS,
+// one row after the other, a stage of 1600 rows took 1.9 us.
+template <class Model, int K>
+__global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, const typename Model::State *S, int nsteps, double t0,
                                                          int step0) {
   constexpr int NT = Model::NT;
   constexpr double UR = 2.22e-16, H = 0.125;
@@ -137,56 +161,100 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, typename Mod
   const int cell0 = w * A.cpb, cells = min(A.cpb, A.n - cell0);
   const int r0 = cell0 * A.comp, R = cells * A.comp, RM = A.cpb * A.comp, RS = RM + A.ghost_max;
   double *Yv = sm, *YN = Yv + RS, *FN = YN + RS, *V1 = FN + RS, *V2 = V1 + RS;
-  double *B = V2 + RS, *CM = B + RM, *T = CM + RM, *part = T + RM + RED_BLOCK, *C4 = part + A.nch + 8;
-  double *LV = C4 + 4 * RES_COEF;
-  unsigned short *LR = (unsigned short *)(LV + A.nnz_max), *LC = LR + RM + 1;
+  double *T = V2 + RS, *part = T + RM + RED_BLOCK, *C4 = part + A.nch + 8, *XV = C4 + 4 * RES_COEF;
+  unsigned short *XC = (unsigned short *)(XV + A.ext_max);
   int late = 0;
   SumPlan P;
   P.set(A.nc, r0, r0 + R);
 
   RkcCtl *ctl = A.ctl;
   const double at = ctl->o[4], rt = ctl->o[5], hmin = ctl->hw[6], mmax = ctl->o[0];
-  double absh = ctl->o[1], sprad = ctl->o[2], naccpt = ctl->o[3], idid = ctl->o[6], gt = ctl->o[7],
-         gt_old = ctl->o[8], lt = ctl->o[9], tend = ctl->o[10], errold = ctl->o[11], hold = ctl->o[12];
-  double hw0 = ctl->hw[0], hw1 = ctl->hw[1], sum_dt = ctl->sum_dt, err = ctl->err;
+  __shared__ double s_ctl[NT / 64][16];
+  __shared__ long long s_cnt[5];   // steps, rejects, stages, power iterations, ion updates: kept by thread 0
+  double *cs = s_ctl[tid >> 6];
+  double &absh = cs[0], &sprad = cs[1], &naccpt = cs[2], &idid = cs[3], &gt = cs[4], &gt_old = cs[5], &lt = cs[6],
+         &tend = cs[7], &errold = cs[8], &hold = cs[9], &hw0 = cs[10], &hw1 = cs[11], &sum_dt = cs[12], &err = cs[13],
+         &errold3 = cs[14], &h_now = cs[15];
+  absh = ctl->o[1]; sprad = ctl->o[2]; naccpt = ctl->o[3]; idid = ctl->o[6]; gt = ctl->o[7]; gt_old = ctl->o[8];
+  lt = ctl->o[9]; tend = ctl->o[10]; errold = ctl->o[11]; hold = ctl->o[12]; hw0 = ctl->hw[0]; hw1 = ctl->hw[1];
+  sum_dt = ctl->sum_dt; err = ctl->err; errold3 = ctl->errold3; h_now = ctl->h;
+  if (tid == 0) {
+    s_cnt[0] = ctl->steps; s_cnt[1] = ctl->rejects; s_cnt[2] = ctl->stages; s_cnt[3] = ctl->rho_iters;
+    s_cnt[4] = ctl->ions;
+  }
+  auto count = [&](int k, int n) {
+    if (tid == 0) s_cnt[k] += n;
+  };
   bool last = ctl->last, newspc = ctl->newspc, jacatt = ctl->jacatt;
-  long long n_step = ctl->steps, n_rej = ctl->rejects, n_stage = ctl->stages, n_rho = ctl->rho_iters, n_ion = ctl->ions;
   unsigned q = ctl->q, gq = ctl->ions_q;
   int status = 0, done_steps = 0;
-  double errold3 = ctl->errold3, h_now = ctl->h;
   bool resume = A.resume != 0;
   int loops = ctl->loops;
   CubeRoots ce;
   ce.p1 = A.p1;
   ce.p2 = A.p2;
 
-  {   // the workgroup's rows
-    const int z0 = A.lnz0[w], nz = A.lnz0[w + 1] - z0;
-    for (int k = tid; k < nz; k += NT) {
-      LV[k] = A.lval[z0 + k];
-      LC[k] = A.lcol[z0 + k];
+  // the workgroup's rows
+  double cm[K], bb[K], wt3[K][ROW_W];
+  uint2 nb[K];
+  {
+    const int x0 = A.x0[w], nx = A.x0[w + 1] - x0;
+    for (int k = tid; k < nx; k += NT) {
+      XV[k] = A.xval[x0 + k];
+      XC[k] = A.xcol[x0 + k];
     }
-    for (int i = tid; i <= R; i += NT) LR[i] = A.lrow[r0 + w + i];
     for (int i = tid; i < R; i += NT) {
       Yv[i] = A.y[r0 + i];
       YN[i] = A.yn[r0 + i];
       FN[i] = A.fn[r0 + i];
-      B[i] = A.b[r0 + i];
-      CM[i] = A.cm[r0 + i];
+      T[i] = A.b[r0 + i];
       if (resume) {
         V1[i] = A.v1[r0 + i];
         V2[i] = A.v2[r0 + i];
       }
     }
   }
+  // the thread's matrix rows and capacitances, and its frozen currents from T
+  auto load_rows = [&]() {
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+      const int i = tid + k * NT;
+      cm[k] = 1.0;
+      bb[k] = 0.0;
+      nb[k] = make_uint2(0u, 0u);
+#pragma unroll
+      for (int e = 0; e < ROW_W; e++) wt3[k][e] = 0.0;
+      if (i < R) {
+        bb[k] = T[i];
+        cm[k] = A.cm[r0 + i];
+        nb[k] = A.lcol[r0 + i];
+#pragma unroll
+        for (int e = 0; e < ROW_W; e++) wt3[k][e] = A.lval[(size_t)e * A.nc + r0 + i];
+      }
+    }
+  };
+  load_rows();
   __syncthreads();
 
-  auto rhs = [&](int i, const double *y) {
-    double d = -B[i];
-    const double yi = y[i];
-    const int e = LR[i + 1];
-    for (int j = LR[i]; j < e; j++) d += LV[j] * (y[LC[j]] - yi);
-    return d / CM[i];
+  // F(y) of the thread's k-th row, its sum in column order; a missing
+  // neighbour is the row itself with conductance 0 (adds an exact zero)
+  auto rhs = [&](int k, double yi, const double *y) {
+    double d = -bb[k];
+    d += wt3[k][0] * (y[nb[k].x & 0xFFFFu] - yi);
+    d += wt3[k][1] * (y[nb[k].x >> 16] - yi);
+    d += wt3[k][2] * (y[nb[k].y & 0xFFFFu] - yi);
+    const unsigned x = nb[k].y >> 16;
+    if (x & 15u)
+      for (unsigned j = x >> 4, e = j + (x & 15u); j < e; j++) d += XV[j] * (y[XC[j]] - yi);
+    return d / cm[k];
+  };
+  // f(k, i) for the thread's rows
+  auto rows = [&](auto f) {
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+      const int i = tid + k * NT;
+      if (i < R) f(k, i);
+    }
   };
   auto total = [&]() { return grid_sum<NT>(P, T, part, A.terms, A.parts, q, &late); };
   // coupled cells: the neighbours' compartments of vector v into its tail.
@@ -207,10 +275,6 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, typename Mod
   };
   auto fetch = [&](double *v) {
     if (!coupled) return;
-    if (gs == GHOST_STAGES) {   // out of slots: a sum of nothing in between
-      for (int i = tid; i < R; i += NT) T[i] = 0.0;
-      finish_sum();
-    }
     double *g = A.ghost + ((size_t)q * GHOST_STAGES + gs) * A.nslot;
     for (int k = A.exp0[w] + tid; k < A.exp0[w + 1]; k += NT) mail_put(g + A.exp_slot[k], v[A.exp_row[k]]);
     const int m0 = A.imp0[w], ni = A.imp0[w + 1] - m0;
@@ -220,7 +284,7 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, typename Mod
   };
 
   auto ion_and_b = [&](double dt) {
-    n_ion++;
+    count(4, 1);
     if constexpr (Model::GAP) {
       // the dendrites' new voltages, for the gap currents of other workgroups' cells
       if (!P.alone) {
@@ -230,18 +294,16 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, typename Mod
         }
       }
     }
-    for (int i = tid; i < R; i += NT) {
-      const double vn = Yv[i];
-      B[i] = Model::ion(S, r0 + i, vn, dt, [&](int cell) {
-        if (cell >= cell0 && cell < cell0 + cells) return Yv[(cell - cell0) * A.comp];
-        return mail_get(A.gap + (size_t)gq * A.n + cell, &late);
-      });
-    }
+    GapView gv{Yv, A.gap + (size_t)gq * A.n, cell0, cells, A.comp, 0};
+#pragma unroll 1
+    for (int i = tid; i < R; i += NT) T[i] = Model::ion(S, r0 + i, Yv[i], dt, &gv);
+    late |= gv.late;
+    load_rows();
     gq = gq == 2 ? 0 : gq + 1;
     if (A.refresh_fn) {
       __syncthreads();
       fetch(YN);
-      for (int i = tid; i < R; i += NT) FN[i] = rhs(i, YN);
+      rows([&](int k, int i) { FN[i] = rhs(k, YN[i], YN); });
     }
     late = __syncthreads_or(late);
   };
@@ -251,14 +313,16 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, typename Mod
     const int itmax = 1000;
     double so[3] = {0.0, 0.0, 0.0};
     const double sqrtu = sqrt(UR), small = 1.0 / 0.125;
-    for (int i = tid; i < R; i += NT) T[i] = YN[i] * YN[i];
-    const double ynrm = sqrt(finish_sum());
-    for (int i = tid; i < R; i += NT) {
-      const double v = A.ede[r0 + i];
-      T[i] = v * v;
+    double ynrm = 0.0, vnrm = 0.0, dynrm;
+#pragma unroll 1
+    for (int n = 0; n < 2; n++) {
+      for (int i = tid; i < R; i += NT) {
+        const double v = n == 0 ? YN[i] : A.ede[r0 + i];
+        T[i] = v * v;
+      }
+      ynrm = vnrm;
+      vnrm = sqrt(finish_sum());
     }
-    const double vnrm = sqrt(finish_sum());
-    double dynrm;
     if (ynrm != 0.0 && vnrm != 0.0) {
       dynrm = ynrm * sqrtu;
       const double f = dynrm / vnrm;
@@ -276,15 +340,15 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, typename Mod
     }
     double sigma = 0.0, sigmal;
     for (int iter = 0; iter < itmax && !late; iter++) {
-      n_rho++;
+      count(3, 1);
       __syncthreads();
       fetch(V1);
-      for (int i = tid; i < R; i += NT) {
-        const double F = rhs(i, V1);
+      rows([&](int k, int i) {
+        const double F = rhs(k, V1[i], V1);
         V2[i] = F;
         const double d = -1.0 * FN[i] + F;
         T[i] = d * d;
-      }
+      });
       const double dfnrm = sqrt(finish_sum());
       sigmal = sigma;
       sigma = dfnrm / dynrm;
@@ -336,7 +400,7 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, typename Mod
       V2[i] = y0;
       V1[i] = hm * FN[i] + y0;
     }
-    n_stage++;
+    count(2, m);
     __syncthreads();
     double bjm1 = 1.0 / ((2.0 * w0) * (2.0 * w0)), bjm2 = bjm1;
     double zjm1 = w0, zjm2 = 1.0, dzjm1 = 1.0, dzjm2 = 0.0, d2zjm1 = 0.0, d2zjm2 = 0.0;
@@ -361,12 +425,20 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, typename Mod
         d2zjm2 = d2zjm1; d2zjm1 = d2zj;
       }
       const double omn = 1.0 - mu - nu, hs = h * mus;
-      fetch(V1);
-      for (int i = tid; i < R; i += NT) {
-        const double F = rhs(i, V1);
-        Yv[i] = mu * V1[i] + nu * V2[i] + omn * YN[i] + hs * (F - ajm1 * FN[i]);
+      if (coupled && gs >= GHOST_STAGES - 2) {   // nearly out of slots: a sum of nothing in between
+        for (int i = tid; i < R; i += NT) T[i] = 0.0;
+        finish_sum();
       }
-      n_stage++;
+      fetch(V1);
+      // every row's reads before the first division: without a value kept
+      // apart the compiler orders a row's store before the next row's reads
+      double yo[K];
+      rows([&](int k, int i) {
+        const double v1 = V1[i];
+        const double F = rhs(k, v1, V1);
+        yo[k] = mu * v1 + nu * V2[i] + omn * YN[i] + hs * (F - ajm1 * FN[i]);
+      });
+      rows([&](int k, int i) { Yv[i] = yo[k]; });
       double *t = V2;
       V2 = V1;
       V1 = Yv;
@@ -404,16 +476,21 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, typename Mod
     step(h, m);
     // f(Y_m) and the error estimate (every weight is positive: atol > 0)
     fetch(Yv);
-    for (int i = tid; i < R; i += NT) {
-      const double F = rhs(i, Yv);
-      V1[i] = F;
+    double fo[K], to[K];
+    rows([&](int k, int i) {
       const double yi = Yv[i], yni = YN[i];
+      const double F = rhs(k, yi, Yv);
       const double ay = fabs(yi), ayn = fabs(yni);
       const double wt = at + rt * ((ay > ayn) ? ay : ayn);
       const double est = 0.8 * (yni - yi) + 0.4 * h * (FN[i] + F);
-      T[i] = (est / wt) * (est / wt);
-    }
-    n_stage++;
+      fo[k] = F;
+      to[k] = (est / wt) * (est / wt);
+    });
+    rows([&](int k, int i) {
+      V1[i] = fo[k];
+      T[i] = to[k];
+    });
+    count(2, 1);
     err = sqrt(finish_sum() / (double)A.nc);
   };
 
@@ -440,7 +517,7 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, typename Mod
       }
       const double h = h_now;
       if (err > 1.0) {
-        n_rej++;
+        count(1, 1);
         absh = 0.8 * absh / ce.p1;
         if (absh < hmin) {
           idid = 4;   // and fall through to the accept branch, as the reference does
@@ -449,7 +526,7 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, typename Mod
           continue;
         }
       }
-      n_step++;
+      count(0, 1);
       naccpt += 1;
       lt += h;
       gt = lt;
@@ -494,19 +571,18 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, typename Mod
         A.syn_g[r0 + i] = A.syn_g[r0 + i] * A.syn_decay + ((u < A.syn_p) ? A.syn_event : 0.0);
       }
     }
-    if (sum_dt != 0.0 && !resume) {
-      ion_and_b(sum_dt);
-      sum_dt = 0.0;
-    }
+    bool ion_due = sum_dt != 0.0 && !resume;
     while (true) {
+      if (ion_due) {
+        ion_and_b(sum_dt);
+        sum_dt = 0.0;
+        ion_due = false;
+      }
       rkclow();
       if (late || status != 0) break;
       sum_dt += gt - gt_old;
       gt_old = gt;
-      if ((A.strict ? sum_dt > A.integ : sum_dt >= A.integ) && idid == 2.0) {
-        ion_and_b(sum_dt);
-        sum_dt = 0.0;
-      }
+      ion_due = (A.strict ? sum_dt > A.integ : sum_dt >= A.integ) && idid == 2.0;
       if (idid == 2.0) continue;
       if (idid == 1.0) break;
       status = (int)idid;
@@ -535,23 +611,23 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, typename Mod
     done_steps++;
   }
 
-  for (int i = tid; i < R; i += NT) {
+  rows([&](int k, int i) {
     A.y[r0 + i] = Yv[i];
     A.yn[r0 + i] = YN[i];
     A.fn[r0 + i] = FN[i];
-    A.b[r0 + i] = B[i];
+    A.b[r0 + i] = bb[k];
     if (status == ASK_POW) {
       A.v1[r0 + i] = V1[i];
       A.v2[r0 + i] = V2[i];
     }
-  }
+  });
   if ((w == 0 || status == TIMED_OUT) && tid == 0) {
     RkcCtl c = *ctl;
     c.o[1] = absh; c.o[2] = sprad; c.o[3] = naccpt; c.o[6] = idid; c.o[7] = gt;
     c.o[8] = gt_old; c.o[9] = lt; c.o[10] = tend; c.o[11] = errold; c.o[12] = hold;
     c.hw[0] = hw0; c.hw[1] = hw1;
     c.sum_dt = sum_dt; c.errold3 = errold3; c.err = err; c.h = h_now;
-    c.steps = n_step; c.rejects = n_rej; c.stages = n_stage; c.rho_iters = n_rho; c.ions = n_ion;
+    c.steps = s_cnt[0]; c.rejects = s_cnt[1]; c.stages = s_cnt[2]; c.rho_iters = s_cnt[3]; c.ions = s_cnt[4];
     c.macro += done_steps;
     c.last = last; c.newspc = newspc; c.jacatt = jacatt; c.status = status;
     c.q = q; c.ions_q = gq; c.ghost_used = gs_old; c.loops = loops;
