@@ -34,7 +34,7 @@
 #include "ion_state.hpp"
 #include "pkj_model.hpp"
 #include "record.hpp"
-#include "rkc_resident.hpp"
+#include "rkc_models.hpp"
 
 namespace cbrkc {
 
@@ -218,78 +218,11 @@ __global__ void __launch_bounds__(256) k_rkcint(double *__restrict__ vnew, doubl
   if (i < nc) vnew[i] = a1 * vt1[i] + a2 * yn[i] + b1 * vt2[i] + b2 * fn[i];
 }
 
-struct PkjState {
-  double *v, *ca, *rev, *iext, *shell;
-  const double *cond;   // [NCOND][nc]
-  double *gate;         // [NGATE][nc]
-  double *b;
-  const double *syn_g;  // may be null
-  double syn_e;
-  int nc;
-  const double *net_s;  // synaptic current of the macro step (granule input), may be null
-  double net_decay;     // exp(-dt / 0.6), dt the ion interval
-};
-
-// pkj_update_ion_RKC (pkj_ion.cu:304-358) followed by pkj_update_matrix
-// (solve_rkc.cu:369-395), fused: one pass over the compartment state.
-// With do_ion == 0 only the current is rebuilt (RKC_vec_initialize).
-__device__ inline double pkj_ion_current(const PkjState &S, int i, double vn, double DT, bool do_ion) {
-  using namespace pkj;
-  const int nc = S.nc;
-  double g[NGATE], c[NCOND];
-#pragma unroll
-  for (int k = 0; k < NGATE; k++) g[k] = S.gate[(size_t)k * nc + i];
-#pragma unroll
-  for (int k = 0; k < NCOND; k++) c[k] = S.cond[(size_t)k * nc + i];
-  double rev = S.rev[i];
-  if (do_ion) {
-    const double vo = S.v[i];
-    const double vm = 0.5 * (vn + vo);
-    double ca = S.ca[i];
-    double caq = ca_rk4(vo, ca, rev, S.shell[i], c[g_CaP] * g[m_CaP] * g[h_CaP], c[g_CaT] * g[m_CaT] * g[h_CaT], DT,
-                        i % 1599 == 0);
-    gates_cn<double>(vm, caq, DT, g);
-#pragma unroll
-    for (int k = 0; k < NGATE; k++) S.gate[(size_t)k * nc + i] = g[k];
-    S.ca[i] = ca;
-    S.rev[i] = rev;
-    S.v[i] = vn;
-  }
-  double bb = current<double>(vn, S.iext[i], rev, c, g);
-  if (S.syn_g) bb += S.syn_g[i] * (vn - S.syn_e);
-  // pkj_update_matrix_new (solve_rkc.cu:358-367, 1245-1249)
-  if (S.net_s) bb += S.net_s[i] * S.net_decay;
-  return bb;
-}
-
 __global__ void __launch_bounds__(256) k_pkj_ion_b(PkjState S, const double *__restrict__ vnew, double DT, int do_ion) {
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i < S.nc) S.b[i] = pkj_ion_current(S, i, vnew[i], DT, do_ion != 0);
 }
 
-
-// io_update_ion_RKC (io_ion.cu:90-127), io_update_matrix (solve_rkc.cu:412-434)
-// and, on each dendrite, the gap currents of io_gap_update / add_io_gap_val
-// (gap.cu:149-160, solve_rkc.cu:400-410), fused.  The gap current uses the
-// partners' voltages after the update (elem[v] = vnew there) and is added in
-// partner order 0..3 (the reference adds with atomics in no fixed order).
-// dend(cell): the new voltage of a cell's dendrite.
-template <class Dend>
-__device__ inline double io_ion_gap_current(const IoState &S, int i, double vn, double DT, bool do_ion, Dend dend) {
-  using namespace io;
-  double bb = io_ion_current(S, i, vn, DT, do_ion);
-  if (do_ion && S.n > 1 && i % COMP == 0) {
-    const int cell = i / COMP;
-#pragma unroll
-    for (int s = 0; s < 4; s++) {
-      const int pre = S.nbr[cell * 4 + s];
-      const double diff_v = (pre > -1) ? (vn - dend(pre)) : 0.0;
-      bb += gap_current<double>(diff_v);
-    }
-  }
-  if (S.syn_g) bb += S.syn_g[i] * (vn - S.syn_e);
-  return bb;
-}
 
 __global__ void __launch_bounds__(256) k_io_ion_b(IoState S, const double *__restrict__ vnew, double DT, int do_ion) {
   const int i = blockIdx.x * 256 + threadIdx.x;
@@ -298,43 +231,11 @@ __global__ void __launch_bounds__(256) k_io_ion_b(IoState S, const double *__res
 }
 
 
-// go_update_ion_RKC_exp_imp (go_ion.cu:379-437), go_KAHP_update_2order
-// (go_ion.cu:88-213) and go_update_matrix (solve_rkc.cu:288-314), fused: the
-// three reference kernels touch one compartment's state each, in this order
-// (solve_rkc.cu:1174-1179).  The intercell gap junctions are in the cable
-// matrix, not here.
-__device__ inline double go_ion_net_current(const GoState &S, int i, double vn, double DT, bool do_ion) {
-  double bb = go_ion_current(S, i, vn, DT, do_ion);
-  if (S.syn_g) bb += S.syn_g[i] * (vn - S.syn_e);
-  // go_update_matrix_new (solve_rkc.cu:279-286, 1181)
-  if (S.net_s) bb += S.net_s[i];
-  return bb;
-}
-
 __global__ void __launch_bounds__(256) k_go_ion_b(GoState S, const double *__restrict__ vnew, double DT, int do_ion) {
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i < S.nc) S.b[i] = go_ion_net_current(S, i, vnew[i], DT, do_ion != 0);
 }
 
-
-// gr_Na_update_2order (gr_ion.cu:45-207), gr_update_ion_RKC_exp_imp
-// (gr_ion.cu:461-480) and gr_update_matrix (solve_rkc.cu:226-249), fused in
-// the reference's order (solve_rkc.cu:1111-1116): the Na scheme sees the
-// voltage of the previous ion update and the new one, then the gates move and
-// the stored voltage becomes the new one.
-__device__ inline double gr_ion_net_current(const GrState &S, int i, double vn, double DT, bool do_ion) {
-  double bb = gr_ion_current(S, i, vn, DT, do_ion);
-  if (S.syn_g) bb += S.syn_g[i] * (vn - S.syn_e);
-  // add_mfgr_val / add_gogr_val (solve_rkc.cu:200-224, 1117-1118), one
-  // synapse after the other
-  if (S.net.on())
-    for (int j = S.net.row[i]; j < S.net.row[i + 1]; j++) {
-      double E;
-      const double gs = syn_entry(S.net, j, E);
-      bb += gs * (vn - E);
-    }
-  return bb;
-}
 
 __global__ void __launch_bounds__(256) k_gr_ion_b(GrState S, const double *__restrict__ vnew, double DT, int do_ion) {
   const int i = blockIdx.x * 256 + threadIdx.x;
@@ -342,45 +243,6 @@ __global__ void __launch_bounds__(256) k_gr_ion_b(GrState S, const double *__res
 }
 
 __global__ void k_coop_probe() {}
-
-// The models of the resident kernel.  512 threads hold a Purkinje cell's 1600
-// compartments four to a thread; the granule and Golgi updates keep their 12 x 12
-// and 6 x 6 systems in registers, which takes one wave per SIMD.  K0 <= K1 <= K2:
-// the rows per thread a kernel is built for (0: none).
-struct PkjModel {
-  using State = PkjState;
-  static constexpr int NT = 512, K0 = 0, K1 = 0, K2 = 4, NONFINITE_STATUS = NONFINITE;
-  static constexpr bool GAP = false;
-  __device__ __attribute__((noinline)) static double ion(const State *Sp, int i, double vn, double dt, GapView *) {
-    State S = *Sp;
-    if (S.net_s) S.net_decay = exp(-dt / 0.6);
-    return pkj_ion_current(S, i, vn, dt, true);
-  }
-};
-struct IoModel {
-  using State = IoState;
-  static constexpr int NT = 256, K0 = 0, K1 = 1, K2 = 7, NONFINITE_STATUS = NONFINITE;
-  static constexpr bool GAP = true;
-  __device__ __forceinline__ static double ion(const State *S, int i, double vn, double dt, GapView *gap) {
-    return io_ion_gap_current(*S, i, vn, dt, true, [&](int cell) { return (*gap)(cell); });
-  }
-};
-struct GoModel {
-  using State = GoState;
-  static constexpr int NT = 256, K0 = 0, K1 = 1, K2 = 7, NONFINITE_STATUS = NONFINITE;
-  static constexpr bool GAP = false;
-  __device__ __forceinline__ static double ion(const State *S, int i, double vn, double dt, GapView *) {
-    return go_ion_net_current(*S, i, vn, dt, true);
-  }
-};
-struct GrModel {
-  using State = GrState;
-  static constexpr int NT = 256, K0 = 1, K1 = 3, K2 = 7, NONFINITE_STATUS = NONFINITE;
-  static constexpr bool GAP = false;
-  __device__ __attribute__((noinline)) static double ion(const State *S, int i, double vn, double dt, GapView *) {
-    return gr_ion_net_current(*S, i, vn, dt, true);
-  }
-};
 
 // xx_set_current shape: one compartment per cell, a time window (pkj.cu:333-344)
 __global__ void k_set_current(double *__restrict__ iext, const double *__restrict__ amp, int comp, int stim_comp,
@@ -508,7 +370,8 @@ class GlobalRkc : public Engine {
   std::string mapping() const override {
     if (!resident_) return "one thread per compartment, one launch per stage";
     return std::to_string(A_.nblk) + " workgroups of " + std::to_string(A_.cpb) +
-           " cells, many macro steps per launch" + (A_.imp0 ? ", gap-junction values exchanged per stage" : "");
+           " cells, many macro steps per launch" +
+           (A_.nhelp ? ", " + std::to_string(A_.nhelp) + " helpers each for the ion updates" : "") + (A_.imp0 ? ", gap-junction values exchanged per stage" : "");
   }
   void sync() override { CB_HIP(hipStreamSynchronize(st_)); }
 
@@ -664,16 +527,9 @@ class GlobalRkc : public Engine {
   virtual int res_rows() const = 0;   // most rows per thread
   virtual void res_launch(const RkcArgs &a, int nsteps, double t0, int step0) = 0;
   virtual bool res_strict() const { return false; }
+  virtual bool res_help() const { return false; }
 
-  // the kernel for k rows per thread (the next of the model's shapes)
-  template <class Model>
-  static const void *kernel_of(int k) {
-    if constexpr (Model::K0 > 0)
-      if (k <= Model::K0) return (const void *)k_rkc_steps<Model, Model::K0>;
-    if constexpr (Model::K1 > 0)
-      if (k <= Model::K1) return (const void *)k_rkc_steps<Model, Model::K1>;
-    return (const void *)k_rkc_steps<Model, Model::K2>;
-  }
+  // the kernel for k rows per thread
   virtual const void *res_kernel(int k) const = 0;
 
   template <class State>
@@ -691,10 +547,11 @@ class GlobalRkc : public Engine {
     RkcArgs av = a;
     const State *sv = (const State *)state_dev_;
     void *args[] = {&av, &sv, &nsteps, &t0, &step0};
-    if (a.nblk == 1)
+    av.gq0 = ctl_host_->ions_q;
+    if (res_grid_ == 1)
       CB_HIP(hipLaunchKernel(res_fn_, dim3(1), dim3(res_threads()), args, res_lds_, st_));
     else   // the workgroups wait for one another: all of them resident at once
-      CB_HIP(hipLaunchCooperativeKernel(res_fn_, dim3(a.nblk), dim3(res_threads()), args, (unsigned)res_lds_, st_));
+      CB_HIP(hipLaunchCooperativeKernel(res_fn_, dim3(res_grid_), dim3(res_threads()), args, (unsigned)res_lds_, st_));
   }
 
   // waits for the launch, takes the kernel's question if it stopped for one
@@ -811,6 +668,15 @@ class GlobalRkc : public Engine {
     int fit = 0;
     CB_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, res_fn_, NT, res_lds_));
     if (fit < 1 || (a.nblk > 1 && !coop_available(st_))) return;
+    // helpers for the ion update, as far as the CUs go, where a workgroup has
+    // more rows than threads; not under the Poisson drive (which its rows'
+    // threads advance)
+    a.own = RM;
+    if (res_help() && !syn_.on && RM > NT && coop_available(st_)) {
+      a.nhelp = std::min((RM + NT - 1) / NT - 1, (ncu - a.nblk) / a.nblk);
+      a.own = ((RM + a.nhelp) / (a.nhelp + 1) + 63) / 64 * 64;
+    }
+    res_grid_ = a.nblk * (1 + a.nhelp);
     const int nslot = (int)imp.size();
     if (nslot > 0) {
       if ((size_t)nslot * 3 * GHOST_STAGES * sizeof(double) > (size_t)1 << 30) return;
@@ -840,6 +706,11 @@ class GlobalRkc : public Engine {
       a.terms = empty_mail((size_t)3 * nc_);
       a.parts = empty_mail((size_t)3 * a.nch);
       a.gap = empty_mail((size_t)3 * n_);
+    }
+    if (a.nhelp > 0) {
+      a.req = empty_mail((size_t)6 * a.nblk);
+      a.vin = empty_mail((size_t)3 * nc_);
+      a.bout = empty_mail((size_t)3 * nc_);
     }
     a.y = vec_[Y];
     a.yn = vec_[YN];
@@ -1206,6 +1077,7 @@ class GlobalRkc : public Engine {
   void *state_dev_ = nullptr;    // the model's state struct, and what is in it
   std::vector<char> state_host_;
   size_t res_lds_ = 0;
+  int res_grid_ = 1;             // workgroups with their helpers
   long macro_ = 0;
   std::vector<void *> res_bufs_;
   std::vector<int> row_h_, col_h_;
@@ -1240,7 +1112,8 @@ class GlobalPkj : public GlobalRkc {
   }
   int res_threads() const override { return PkjModel::NT; }
   int res_rows() const override { return PkjModel::K2; }
-  const void *res_kernel(int k) const override { return kernel_of<PkjModel>(k); }
+  const void *res_kernel(int k) const override { return rkc_kernel_pkj(k); }
+  bool res_help() const override { return PkjModel::HELP; }
   void res_launch(const RkcArgs &a, int nsteps, double t0, int step0) override {
     launch_model(a, PkjState{v_, ca_, rev_, iext_, shell_, cond_, gate_, b_, syn_g_, syn_.e_syn, nc_,
                                      net_.on() ? net_s_ : nullptr, 0.0}, nsteps, t0, step0);
@@ -1294,7 +1167,7 @@ class GlobalIo : public GlobalRkc {
   bool trigger() const override { return sum_dt_ > integ_; }   // strict for IO, solve_rkc.cu:1347
   int res_threads() const override { return IoModel::NT; }
   int res_rows() const override { return IoModel::K2; }
-  const void *res_kernel(int k) const override { return kernel_of<IoModel>(k); }
+  const void *res_kernel(int k) const override { return rkc_kernel_io(k); }
   bool res_strict() const override { return true; }
   void res_launch(const RkcArgs &a, int nsteps, double t0, int step0) override {
     launch_model(a, IoState{v_, ca_, iext_, cond_, gate_, compart_, nbr_, b_, syn_g_, syn_.e_syn, nc_, n_}, nsteps, t0, step0);
@@ -1343,7 +1216,7 @@ class GlobalGo : public GlobalRkc {
   }
   int res_threads() const override { return GoModel::NT; }
   int res_rows() const override { return GoModel::K2; }
-  const void *res_kernel(int k) const override { return kernel_of<GoModel>(k); }
+  const void *res_kernel(int k) const override { return rkc_kernel_go(k); }
   void res_launch(const RkcArgs &a, int nsteps, double t0, int step0) override {
     launch_model(a, GoState{v_, ca_, ca2_, rev_, ca_old_, iext_, area_, cond_, gate_, b_, syn_g_, syn_.e_syn, nc_,
                                    net_.on() ? net_s_ : nullptr}, nsteps, t0, step0);
@@ -1399,7 +1272,8 @@ class GlobalGr : public GlobalRkc {
   bool trigger() const override { return sum_dt_ > integ_; }   // strict for GR, solve_rkc.cu:1148
   int res_threads() const override { return GrModel::NT; }
   int res_rows() const override { return GrModel::K2; }
-  const void *res_kernel(int k) const override { return kernel_of<GrModel>(k); }
+  const void *res_kernel(int k) const override { return rkc_kernel_gr(k); }
+  bool res_help() const override { return GrModel::HELP; }
   bool res_strict() const override { return true; }
   void res_launch(const RkcArgs &a, int nsteps, double t0, int step0) override {
     launch_model(a, GrState{v_, iext_, ca_, compart_, cond_, gate_, na_, b_, syn_g_, syn_.e_syn, nc_, net_}, nsteps, t0, step0);

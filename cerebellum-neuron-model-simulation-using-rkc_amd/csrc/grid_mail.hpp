@@ -54,6 +54,18 @@ __device__ inline double mail_get(const double *slot, int *late) {
   }
   return __longlong_as_double((long long)b);
 }
+// mail_get for a wait that may be long: it leaves 256 cycles between looks
+__device__ inline double mail_wait(const double *slot, int *late) {
+  const unsigned long long t0 = wall_clock64();
+  while (__hip_atomic_load((const unsigned long long *)slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == MAIL_EMPTY) {
+    __builtin_amdgcn_s_sleep(4);
+    if (wall_clock64() - t0 > SPIN_TICKS) {
+      *late = 1;
+      return 0.0;
+    }
+  }
+  return mail_get(slot, late);
+}
 // the thread's own stores have reached memory
 __device__ inline void mail_settle() {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");

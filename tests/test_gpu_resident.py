@@ -3,7 +3,8 @@ where its layout has edges, against the oracle: one and several workgroups,
 256-row chunks of the norms that span workgroups (Golgi cells of 131 rows:
 three per chunk; a last workgroup of a few rows), gap junctions in the cable
 matrix exchanged per stage, the olive's gap currents between workgroups, and
-the largest population the kernel takes.
+the largest population the kernel takes; ion updates shared with helper
+workgroups (granule cells: 578 rows as 256 + 256 + 66).
 
 Without ion updates the first macro step uses only correctly rounded
 arithmetic and libm's pow for the step sizes, so voltages, derivative,
@@ -18,6 +19,7 @@ import pytest
 import cbrkc
 import orc
 from test_oracle_go import go_pop
+from test_oracle_gr import gr_pop
 from test_oracle_io import io_pop
 
 pytestmark = pytest.mark.gpu
@@ -46,12 +48,15 @@ def test_purkinje_without_ion_updates_is_bit_exact(ref_data, nx, ny, coupled):
     assert all(so[k] == sg[k] for k in ("steps", "rejects", "stages", "rho_iters")), (so, sg)
 
 
-@pytest.mark.parametrize("cell,nx,ny", [("io", 5, 5), ("io", 10, 9), ("io", 13, 40), ("go", 1, 1), ("go", 5, 3)])
+@pytest.mark.parametrize("cell,nx,ny", [("io", 5, 5), ("io", 10, 9), ("io", 13, 40), ("go", 1, 1), ("go", 5, 3), ("gr", 1, 1),
+                                        ("gr", 3, 1)])
 def test_grids_first_macro_step(ref_data, cell, nx, ny):
     print(f"{cell} {nx}x{ny}", flush=True)
     n = nx * ny
-    v0 = -60.0 + 0.03 * np.arange(n) % 2.0
-    if cell == "io":
+    v0 = (-70.0 if cell == "gr" else -60.0) + 0.03 * np.arange(n) % 2.0
+    if cell == "gr":
+        o, kind, f = gr_pop(ref_data, nx, ny, v0=v0), cbrkc.GR, "Gr.txt"
+    elif cell == "io":
         o, kind, f = io_pop(ref_data, nx, ny, v0=v0), cbrkc.IO, "IO.txt"
     else:
         o, kind, f = go_pop(ref_data, nx, ny, v0=v0), cbrkc.GO, "Go_131.txt"
