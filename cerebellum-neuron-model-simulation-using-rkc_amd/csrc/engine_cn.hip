@@ -689,11 +689,6 @@ __global__ void k_cn_stim(double *__restrict__ iext, const double *__restrict__ 
   }
 }
 
-__global__ void k_cn_record(const double *__restrict__ v, double *__restrict__ out, int comp, int rec, int n) {
-  int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c < n) out[c] = v[rec + (size_t)c * comp];
-}
-
 // ---- the exact per-cell solve (Hines elimination on each cell's tree) ----
 //
 // Each cell's compartments are renumbered breadth-first from the centre of
@@ -1132,7 +1127,6 @@ class CnEngine : public Engine {
     S_.bicg = bicg ? 1 : 0;
     S_.dt = dt_;
     amp_ = dup(stim_.amp);
-    rec_ = dal<double>(n_);
   }
   ~CnEngine() override {
     (void)hipStreamSynchronize(st_);
@@ -1145,7 +1139,7 @@ class CnEngine : public Engine {
                           (const void *)S_.ap, (const void *)S_.rs, (const void *)S_.atps, (const void *)S_.p[0],
                           (const void *)S_.p[1], (const void *)S_.ps[0], (const void *)S_.ps[1],
                           (const void *)S_.part, (const void *)S_.scal, (const void *)S_.flag, (const void *)amp_,
-                          (const void *)rec_, (const void *)P_.perm, (const void *)P_.up, (const void *)P_.dn,
+                          (const void *)rec_, (const void *)bits_, (const void *)P_.perm, (const void *)P_.up, (const void *)P_.dn,
                           (const void *)P_.meta, (const void *)P_.lev, (const void *)P_.lev_off,
                           (const void *)Q_.perm, (const void *)Q_.up, (const void *)Q_.dn, (const void *)Q_.seg,
                           (const void *)Q_.kids, (const void *)Q_.nseg, (const void *)Q_.nh})
@@ -1163,7 +1157,12 @@ class CnEngine : public Engine {
     s.stages = f[F_TOTAL];
     return s;
   }
+  // the stimulated compartments hold the window's state until it changes, so
+  // most steps need no launch (of 5 us, five an interval)
   void set_current(double t) override {
+    const int on = stim_.t0 <= t && t < stim_.t1;
+    if (on == stim_on_) return;
+    stim_on_ = on;
     k_cn_stim<<<(n_ + 127) / 128, 128, 0, st_>>>(S_.iext, amp_, comp_, stim_.comp, stim_.t0, stim_.t1, t, n_);
   }
   // one exact tree solve of (diag, b) into v: by unbranched runs or level
@@ -1255,11 +1254,11 @@ class CnEngine : public Engine {
     const int per = rec_comp >= 0 ? 1 : comp_;
     const int words = (n_ + 31) / 32;
     const bool raster = raster_comp_ >= 0;
-    double *drec = nullptr;
-    uint32_t *dbits = nullptr;
-    if (rec_out) drec = dal<double>((size_t)nsteps * n_ * per);
+    if (rec_out) grow(rec_, rec_cap_, (size_t)nsteps * n_ * per);
+    if (raster) grow(bits_, bits_cap_, (size_t)nsteps * words);
+    double *drec = rec_out ? rec_ : nullptr;
+    uint32_t *dbits = raster ? bits_ : nullptr;
     if (raster) {
-      dbits = dal<uint32_t>((size_t)nsteps * words);
       CB_HIP(hipMemsetAsync(dbits, 0, sizeof(uint32_t) * (size_t)nsteps * words, st_));
     }
     for (int k = 0; k < nsteps; k++) {
@@ -1288,8 +1287,6 @@ class CnEngine : public Engine {
       CB_HIP(hipMemcpyAsync(rec_out, drec, sizeof(double) * (size_t)nsteps * n_ * per, hipMemcpyDeviceToHost, st_));
     if (dbits) CB_HIP(hipMemcpyAsync(bits.data(), dbits, sizeof(uint32_t) * bits.size(), hipMemcpyDeviceToHost, st_));
     CB_HIP(hipStreamSynchronize(st_));
-    if (drec) CB_HIP(hipFree(drec));
-    if (dbits) CB_HIP(hipFree(dbits));
     check_late();
     if (raster) append_spikes(bits, nsteps, words, t0, H_MAX);
   }
@@ -1320,6 +1317,15 @@ class CnEngine : public Engine {
   }
 
  protected:
+  template <typename T>
+  static void grow(T *&p, size_t &cap, size_t n) {
+    if (cap >= n) return;
+    if (p) CB_HIP(hipFree(p));
+    p = nullptr;
+    cap = 0;
+    p = dal<T>(n);
+    cap = n;
+  }
   void check_late() const {
     if (late_host_ && *(volatile int *)late_host_) throw Error("CN / BE: a workgroup of the solve waited for another one in vain");
   }
@@ -1516,7 +1522,11 @@ class CnEngine : public Engine {
   int res_grid_ = 0, res_nt_ = 0;
   std::vector<void *> res_bufs_;
   int *late_host_ = nullptr;
+  int stim_on_ = -1;             // the window's state in iext (-1: not set yet)
+  // the recording's buffers, kept for the next run
   double *amp_ = nullptr, *rec_ = nullptr;
+  uint32_t *bits_ = nullptr;
+  size_t rec_cap_ = 0, bits_cap_ = 0;
   hipStream_t st_{};
   Stats st;
 };
