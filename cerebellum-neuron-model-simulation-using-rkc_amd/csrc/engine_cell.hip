@@ -1439,6 +1439,8 @@ class CellPkj : public Engine {
   }
 
   bool select_mapping(int threads) override {
+    // (the FP64 engine takes its 512 threads by itself; asked for, they stay refused)
+    if (sizeof(T) == 8 && threads == 512) return false;
     for (size_t v = 0; v < variants_.size(); v++)
       if (variants_[v].nt == threads && (long)variants_[v].nt * variants_[v].k >= C_) {
         cur_ = (int)v;
@@ -1518,6 +1520,7 @@ class CellPkj : public Engine {
     } else {
       v.push_back({256, 7});
       v.push_back({320, 5});
+      v.push_back({512, 4});
     }
     return v;
   }
@@ -1536,10 +1539,15 @@ class CellPkj : public Engine {
     return (size_t)C_ * (5 * sizeof(T) + 4) + red;
   }
 
+  // 512 threads to a cell: with 256 or 320 a cell's waves leave half of the
+  // issue slots of its CU idle, and the second cell on the CU fills them only
+  // where there are twice as many cells as CUs (16 macro steps, ms at 256 / 320
+  // / 512 threads; FP64: 16 cells 29 / 31 / 22, 256 cells 34 / 34 / 26, 400 cells 43 /
+  // 46 / 35; mixed: 16 cells 18 / 14 / 10.6, 400 cells 23 / 18 / 14)
   void choose_default() {
     cur_ = 0;
     for (size_t v = 0; v < variants_.size(); v++)
-      if (variants_[v].nt == (sizeof(T) == 4 ? 320 : 256)) cur_ = (int)v;
+      if (variants_[v].nt == 512) cur_ = (int)v;
   }
 
   template <int NT, int K>
