@@ -25,7 +25,8 @@
 // conductances + I_ext (minus the inferior olive's gap currents); the solve is
 // the same CG / BiCG.
 //
-// The Krylov loop runs on the device without host round trips: each
+// The Krylov loop runs on the device without host round trips, for systems
+// that fit the chip's LDS in one kernel (kry_resident.hpp); otherwise each
 // iteration is two launches, every dot product is reduced deterministically
 // (256-wide stride-halving trees, the partials reduced again with the same
 // tree by whichever block finishes last), and a device flag set on
@@ -1288,6 +1289,11 @@ class CnEngine : public Engine {
     if (dbits) CB_HIP(hipMemcpyAsync(bits.data(), dbits, sizeof(uint32_t) * bits.size(), hipMemcpyDeviceToHost, st_));
     CB_HIP(hipStreamSynchronize(st_));
     check_late();
+    if (rec_cap_ > REC_KEPT) {   // a large recording's buffer is given back
+      (void)hipFree(rec_);
+      rec_ = nullptr;
+      rec_cap_ = 0;
+    }
     if (raster) append_spikes(bits, nsteps, words, t0, H_MAX);
   }
   const double *device_vnew() const override { return S_.v; }
@@ -1522,6 +1528,7 @@ class CnEngine : public Engine {
   int res_grid_ = 0, res_nt_ = 0;
   std::vector<void *> res_bufs_;
   int *late_host_ = nullptr;
+  static constexpr size_t REC_KEPT = (size_t)8 << 20;   // doubles of recording kept for the next run
   int stim_on_ = -1;             // the window's state in iext (-1: not set yet)
   // the recording's buffers, kept for the next run
   double *amp_ = nullptr, *rec_ = nullptr;

@@ -1,6 +1,11 @@
 // Plain FP64 RKC with one population-global controller: the reference's
 // semantics (solve_rkc.cu) on MI355X.
 //
+// Populations that fit the LDS of the chip's CUs run on the resident kernel
+// (rkc_resident.hpp: many macro steps a launch, the controller on the device).
+// The rest of this file is the launch-per-stage path of larger ones, which also
+// initialises every population; the two give the same bits.
+//
 // One thread per compartment, structure-of-arrays FP64 state in HBM.  The
 // differences from the reference are in how the work is laid out, not in
 // what is computed:
@@ -463,6 +468,11 @@ class GlobalRkc : public Engine {
       CB_HIP(hipMemcpyAsync(rec_out, rec_, sizeof(double) * (size_t)nsteps * per, hipMemcpyDeviceToHost, st_));
     if (raster) CB_HIP(hipMemcpyAsync(bits.data(), bits_, sizeof(uint32_t) * bits.size(), hipMemcpyDeviceToHost, st_));
     CB_HIP(hipStreamSynchronize(st_));
+    if (rec_cap_ > REC_KEPT) {   // a large recording's buffer is given back
+      (void)hipFree(rec_);
+      rec_ = nullptr;
+      rec_cap_ = 0;
+    }
     if (raster) append_spikes(bits, nsteps, words, t0, H_MAX);
   }
 
@@ -1070,6 +1080,7 @@ class GlobalRkc : public Engine {
   Stats st;
   // the resident kernel's tables and workspaces
   static constexpr int RES_RUN = 64;   // macro steps per launch
+  static constexpr size_t REC_KEPT = (size_t)8 << 20;   // doubles of recording kept for the next run
   bool resident_ = false;
   RkcArgs A_{};
   RkcCtl *ctl_host_ = nullptr;   // written by the kernel as it ends
