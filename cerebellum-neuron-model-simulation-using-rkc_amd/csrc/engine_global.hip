@@ -161,6 +161,11 @@ __global__ void __launch_bounds__(256) k_scale(double s, const double *__restric
   if (i < nc) C[i] = s * A[i];
 }
 
+__global__ void __launch_bounds__(256) k_empty_mail(unsigned long long *slots, size_t n) {
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < n) slots[i] = MAIL_EMPTY;
+}
+
 __global__ void __launch_bounds__(256) k_fill(double s, double *__restrict__ C, int nc) {
   int i = blockIdx.x * 256 + threadIdx.x;
   if (i < nc) C[i] = s;
@@ -731,7 +736,8 @@ class GlobalRkc : public Engine {
     a.v1 = vec_[VT1];
     a.v2 = vec_[VT2];
     a.cm = cm_;
-    a.coef = res_put(rkc_stage_table(RES_COEF));
+    static const std::vector<double> stage_table = rkc_stage_table(RES_COEF);   // the same for every population
+    a.coef = res_put(stage_table);
     RkcCtl c{};
     std::memcpy(c.o, o_, sizeof(o_));
     std::memcpy(c.hw, hw_, sizeof(hw_));
@@ -772,10 +778,11 @@ class GlobalRkc : public Engine {
   }
 
   double *empty_mail(size_t n) {
-    unsigned long long e = MAIL_EMPTY;
-    double x;
-    std::memcpy(&x, &e, sizeof(x));
-    return res_put(std::vector<double>(n, x));
+    double *d = dalloc<double>(n);
+    res_bufs_.push_back((void *)d);
+    k_empty_mail<<<(unsigned)((n + 255) / 256), 256, 0, st_>>>((unsigned long long *)d, n);
+    CB_HIP(hipGetLastError());
+    return d;
   }
 
   Csr csr() const { return Csr{row_, col_, val_}; }
