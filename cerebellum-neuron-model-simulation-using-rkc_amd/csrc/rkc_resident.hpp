@@ -5,8 +5,8 @@
 // What it replaces took one launch per Chebyshev stage, four more and a read
 // back by the host per step attempt: 3-5 us a launch whatever the population
 // (two thirds of a small population's time), plus the host's answer.  Here
-// every workgroup owns whole cells, keeps their seven vectors and its rows of
-// the cable matrix in LDS and runs the controller's scalar arithmetic itself
+// every workgroup owns whole cells, keeps their five vectors in LDS and its rows
+// of the cable matrix in registers and runs the controller's scalar arithmetic itself
 // on the same sums; a stage costs a barrier, a step attempt one exchange of
 // the error norm's partial sums.  Cells whose cable matrix couples them
 // (gap junctions) also exchange the coupled compartments' values at every
