@@ -444,7 +444,7 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, const typena
         }
       } else {
         const int id = iter % A.nc - r0;
-        if (id >= 0 && id < R && id % NT == tid) V1[id] = 2.0 * Yv[id] - V1[id];
+        if (id >= 0 && id < R && id % NT == tid) V1[id] = 2.0 * YN[id] - V1[id];
       }
     }
     idid = 6;
