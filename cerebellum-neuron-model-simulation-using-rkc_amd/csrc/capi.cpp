@@ -700,6 +700,14 @@ int cb_pop_mapping(const cb_pop *p, char *buf, int len) {
   });
 }
 
+int cb_pop_launch_path(cb_pop *p, int on) {
+  return guarded([&]() -> int {
+    if (!p) return fail(CB_E_ARG, "null population");
+    if (!p->eng->use_launches(on != 0)) return fail(CB_E_UNSUP, "the population has one path only");
+    return CB_OK;
+  });
+}
+
 int cb_pop_controller(const cb_pop *p, double *o, double *hw) {
   return guarded([&]() -> int {
     if (!p || !o || !hw) return fail(CB_E_ARG, "null argument");

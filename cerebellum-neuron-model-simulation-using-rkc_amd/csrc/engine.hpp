@@ -85,6 +85,13 @@ class Engine {
   }
   // selects the mapping with this many threads per cell; false if none
   virtual bool select_mapping(int threads) { return threads == 0; }
+  // on: a launch per stage or iteration instead of the kernel that runs whole
+  // steps or solves (off: that kernel again); the results are the same bits.
+  // False where the engine or the population's size leaves no choice.
+  virtual bool use_launches(bool on) {
+    (void)on;
+    return false;
+  }
   // a description of the launch mapping in use (and of the last autotune trial)
   virtual std::string mapping() const { return "one thread per compartment"; }
   // event-timed duration of the main kernel (ms) and its launch count

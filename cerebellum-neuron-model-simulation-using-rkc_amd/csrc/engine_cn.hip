@@ -1214,8 +1214,14 @@ class CnEngine : public Engine {
     tune_ms_[1] = ms[1];
     return HINES_WAVE;
   }
+  bool use_launches(bool on) override {
+    if (direct_ || !res_fn_) return on && !direct_;
+    resident_ = !on;
+    S_.direct = resident_ ? 1 : 0;
+    return true;
+  }
   std::string mapping() const override {
-    if (res_fn_)
+    if (resident_)
       return "Krylov solve in one kernel, " + std::to_string(res_grid_) + " workgroups of " + std::to_string(A_.rb) + " rows";
     if (!direct_) return nb_ <= KRY_SMALL_BLOCKS ? "Krylov solve in one workgroup" : "Krylov solve, two launches per iteration";
     std::string m = chain_ ? "tree solve by unbranched runs, one lane per run, one wavefront per cell"
@@ -1231,7 +1237,7 @@ class CnEngine : public Engine {
     prep();
     if (direct_) {
       tree_solve(chain_, S_.diag, S_.b, S_.v);
-    } else if (res_fn_) {
+    } else if (resident_) {
       void *args[] = {&A_};
       if (res_grid_ == 1)
         CB_HIP(hipLaunchKernel(res_fn_, dim3(1), dim3(res_nt_), args, res_lds_, st_));
@@ -1491,6 +1497,7 @@ class CnEngine : public Engine {
     res_grid_ = grid;
     res_nt_ = nt;
     res_fn_ = fn;
+    resident_ = true;
     S_.direct = 1;
     return true;
   }
@@ -1521,8 +1528,10 @@ class CnEngine : public Engine {
   bool chain_ = false;   // the solve by unbranched runs is in use
   bool has_chain_ = false;   // every cell at most CHAIN_SEGS runs: the run walk applies
   double tune_ms_[2] = {0.0, 0.0};
-  // the resident Krylov kernel (null: launches per iteration)
+  // the resident Krylov kernel (null: the system does not fit it), and whether
+  // it is in use instead of the launches per iteration
   const void *res_fn_ = nullptr;
+  bool resident_ = false;
   KryArgs A_{};
   size_t res_lds_ = 0;
   int res_grid_ = 0, res_nt_ = 0;

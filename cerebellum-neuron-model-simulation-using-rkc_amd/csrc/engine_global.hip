@@ -384,12 +384,21 @@ class GlobalRkc : public Engine {
            (A_.nhelp ? ", " + std::to_string(A_.nhelp) + " helpers each for the ion updates" : "") + (A_.imp0 ? ", gap-junction values exchanged per stage" : "");
   }
   void sync() override { CB_HIP(hipStreamSynchronize(st_)); }
+  // the two paths keep the controller in different places, so the choice is
+  // made before the first macro step
+  bool use_launches(bool on) override {
+    if (!laid_out_) return on;
+    if (started_) throw Error("the path is chosen before the first macro step");
+    resident_ = !on;
+    return true;
+  }
 
   void set_current(double t) override {
     k_set_current<<<(n_ + 127) / 128, 128, 0, st_>>>(iext_, amp_, comp_, stim_.comp, stim_.t0, stim_.t1, t, n_);
   }
 
   void advance() override {
+    started_ = true;
     if (resident_) {
       if (net_.on() && net_s_) syn_macro_current(net_, vec_[Y], net_s_, nc_, st_);
       for (const long m0 = macro_; macro_ == m0; check_steps()) res_launch(A_, 1, 0.0, (int)macro_);
@@ -451,6 +460,7 @@ class GlobalRkc : public Engine {
       grow(bits_, bits_cap_, (size_t)nsteps * words);
       CB_HIP(hipMemsetAsync(bits_, 0, sizeof(uint32_t) * (size_t)nsteps * words, st_));
     }
+    started_ = true;
     const long m0 = macro_;
     while (macro_ < m0 + nsteps) {
       const int k = (int)(macro_ - m0);
@@ -774,7 +784,7 @@ class GlobalRkc : public Engine {
     }
     A_ = a;
     CB_HIP(hipStreamSynchronize(st_));
-    resident_ = true;
+    laid_out_ = resident_ = true;
   }
 
   double *empty_mail(size_t n) {
@@ -1088,7 +1098,8 @@ class GlobalRkc : public Engine {
   // the resident kernel's tables and workspaces
   static constexpr int RES_RUN = 64;   // macro steps per launch
   static constexpr size_t REC_KEPT = (size_t)8 << 20;   // doubles of recording kept for the next run
-  bool resident_ = false;
+  bool laid_out_ = false, resident_ = false;   // the resident kernel's tables exist; it is in use
+  bool started_ = false;                       // a macro step has been asked for
   RkcArgs A_{};
   RkcCtl *ctl_host_ = nullptr;   // written by the kernel as it ends
   const void *res_fn_ = nullptr;

@@ -202,6 +202,15 @@ int cb_pop_autotune(cb_pop *p, int trial_steps, int *threads);
  * counterpart in the reference. */
 int cb_pop_mapping(const cb_pop *p, char *buf, int len);
 
+/* Population-global RKC, CN and BE engines: on != 0 takes a kernel launch per
+ * Chebyshev stage or Krylov iteration in place of the kernel that runs whole
+ * steps or solves (the default where the population fits it), on == 0 goes
+ * back.  The results are the same bits; the path of larger populations can so
+ * be taken by a small one.  An RKC population chooses before its first macro step
+ * (CB_E_ARG afterwards).  CB_E_UNSUP for engines and populations with one path
+ * only.  No counterpart in the reference. */
+int cb_pop_launch_path(cb_pop *p, int on);
+
 /* Global-controller scalars: h_others[14] and h_work[8] (param.h:22,
  * solve_rkc.cu:453-476).  CB_E_UNSUP for per-cell engines. */
 int cb_pop_controller(const cb_pop *p, double *others14, double *hwork8);

@@ -1,0 +1,79 @@
+"""The two paths of the population-global engines against each other
+(cb_pop_launch_path): the resident kernels (csrc/rkc_resident.hpp,
+csrc/kry_resident.hpp) and the kernel launches per Chebyshev stage and Krylov
+iteration that larger populations take, and any population in a process that
+may not launch cooperatively.  Every voltage, current, gate, controller value,
+counter, recording and spike is the same bits, with ion updates, stimulus,
+gap junctions and Poisson drive; so the small populations here, and
+with them the oracle's tests of either path, cover both."""
+import os
+
+import numpy as np
+import pytest
+
+import cbrkc
+
+pytestmark = pytest.mark.gpu
+
+KIND = {"pkj": (cbrkc.PKJ, "Pkj.txt", -67.0, 18), "io": (cbrkc.IO, "IO.txt", -60.0, 10),
+        "go": (cbrkc.GO, "Go_131.txt", -60.0, 24), "gr": (cbrkc.GR, "Gr.txt", -70.0, 24)}
+T0 = 600.0   # inside the reference's stimulus windows
+FIELDS = (cbrkc.F_VNEW, cbrkc.F_V, cbrkc.F_CA, cbrkc.F_B, cbrkc.F_IEXT)
+
+
+def make(ref_data, cell, nx, ny, **kw):
+    kind, f, v, _ = KIND[cell.split()[0]]
+    gj = os.path.join(ref_data, "Pkj_GJ.csv") if cell == "pkj gj" else ""
+    v0 = v + 0.05 * (np.arange(nx * ny) % 31)
+    pops = [cbrkc.Population(kind, nx, ny, morph=os.path.join(ref_data, f), gj=gj, v0=v0, **kw) for _ in range(2)]
+    pops[1].launch_path()
+    assert "workgroups" in pops[0].mapping() and "workgroups" not in pops[1].mapping(), [p.mapping() for p in pops]
+    return pops
+
+
+def same(a, b, fields):
+    for f in fields:
+        try:
+            x = a.read(f)
+        except cbrkc.CbError:
+            continue
+        assert np.array_equal(x, b.read(f)), f
+    assert a.stats() == b.stats()
+
+
+@pytest.mark.parametrize("cell,nx,ny,kw", [
+    ("io", 2, 2, {}), ("io", 13, 40, {}), ("go", 1, 1, {}), ("go", 5, 3, {}), ("gr", 1, 1, {}), ("gr", 3, 1, {}),
+    ("pkj", 1, 1, {}), ("pkj", 3, 1, {}), ("pkj gj", 2, 2, {}),
+    ("pkj", 2, 1, dict(atol=1e-6, rtol=1e-4, **cbrkc.STABLE)),
+    ("pkj", 2, 1, dict(poisson=dict(rate_hz=2000.0, g_mS=1e-6, tau_ms=2.0, e_mV=0.0, seed=3)))])
+def test_rkc(ref_data, cell, nx, ny, kw):
+    print(f"{cell} {nx}x{ny} {kw}", flush=True)
+    a, b = make(ref_data, cell, nx, ny, **kw)
+    out = []
+    for p in (a, b):
+        p.set_raster(0, -60.0)
+        out.append([p.run(3, T0, 0), p.run(2, T0 + 0.375, -1)])
+        p.set_current(T0 + 0.625)
+        p.advance()
+    for x, y in zip(*out):
+        assert np.array_equal(x, y)
+    for x, y in zip(a.spikes(), b.spikes()):
+        assert np.array_equal(x, y)
+    same(a, b, FIELDS + (cbrkc.F_Y, cbrkc.F_YN, cbrkc.F_FN) + tuple(cbrkc.F_GATE0 + k for k in range(KIND[cell.split()[0]][3])))
+    for x, y in zip(a.controller(), b.controller()):
+        assert np.array_equal(x, y)
+    with pytest.raises(cbrkc.CbError):
+        a.launch_path()   # too late
+
+
+@pytest.mark.parametrize("solver", [cbrkc.CN, cbrkc.BE], ids=["cn", "be"])
+@pytest.mark.parametrize("cell,nx,ny", [("pkj", 1, 1), ("pkj", 3, 1), ("pkj gj", 3, 2), ("gr", 2, 4), ("go", 2, 2),
+                                        ("go", 7, 7), ("io", 1, 1), ("io", 9, 9), ("io", 40, 24)])
+def test_krylov(ref_data, cell, nx, ny, solver):
+    print(f"{cell} {nx}x{ny} solver {solver}", flush=True)
+    a, b = make(ref_data, cell, nx, ny, solver=solver)
+    assert np.array_equal(a.run(2, T0, 0), b.run(2, T0, 0))
+    b.launch_path(False)   # this engine may change its path at any time
+    a.launch_path()
+    assert np.array_equal(a.run(1, T0 + 0.25, -1), b.run(1, T0 + 0.25, -1))
+    same(a, b, FIELDS)
