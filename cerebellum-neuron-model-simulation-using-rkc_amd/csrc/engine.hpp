@@ -178,6 +178,8 @@ struct SolverSpec {
 // entries of 4 doubles; entry 0 = {mu~_1}, entry j = {mu_j, nu_j, mu~_j,
 // a_{j-1}} for j = 1..m-1 (solve_rkc.cu:815-906).
 std::vector<double> rkc_stage_table(int mtab);
+// w1 and mu~_1 of a step of m stages
+void rkc_stage_start(int m, double *w1, double *mus);
 
 // The batched engine over an uneven mix of cell types (granule, Golgi,
 // Purkinje, inferior olive; index = the C-ABI's cell type): every cell on

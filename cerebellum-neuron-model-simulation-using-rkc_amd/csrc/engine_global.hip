@@ -587,11 +587,12 @@ class GlobalRkc : public Engine {
     CB_HIP(hipStreamSynchronize(st_));
     const RkcCtl &c = *ctl_host_;
     macro_ = c.macro;
-    A_.resume = c.status == ASK_POW;
-    if (A_.resume) {
+    A_.resume = c.status == ASK_POW || c.status == ASK_STAGE ? c.status : 0;
+    if (c.status == ASK_POW) {
       A_.p1 = std::pow(c.err, 1.0 / 3.0);
       A_.p2 = std::pow(c.err, 2.0 / 3.0);
     }
+    if (c.status == ASK_STAGE) rkc_stage_start(c.m, &A_.asked.x, &A_.asked.y);
     if (c.status == 0 || A_.resume) return;
     if (c.status == NONFINITE)
       throw Error("RKC: non-finite state (error estimate " + std::to_string(c.err) + ")", NONFINITE);
@@ -748,6 +749,12 @@ class GlobalRkc : public Engine {
     a.cm = cm_;
     static const std::vector<double> stage_table = rkc_stage_table(RES_COEF);   // the same for every population
     a.coef = res_put(stage_table);
+    static const std::vector<double2> start_table = [] {
+      std::vector<double2> t(RES_START + 1);
+      for (int m = 0; m <= RES_START; m++) rkc_stage_start(m, &t[m].x, &t[m].y);
+      return t;
+    }();
+    a.start = res_put(start_table);
     RkcCtl c{};
     std::memcpy(c.o, o_, sizeof(o_));
     std::memcpy(c.hw, hw_, sizeof(hw_));

@@ -10,17 +10,23 @@
 
 namespace cbrkc {
 
+void rkc_stage_start(int m, double *w1, double *mus) {
+  const double w0 = 1.0 + 2.0 / (13.0 * m * m);
+  const double temp1 = w0 * w0 - 1.0;
+  const double temp2 = std::sqrt(temp1);
+  const double arg = m * std::log(w0 + temp2);
+  *w1 = std::sinh(arg) * temp1 / (std::cosh(arg) * m * temp2 - w0 * std::sinh(arg));
+  *mus = *w1 * (1.0 / ((2.0 * w0) * (2.0 * w0)));
+}
+
 std::vector<double> rkc_stage_table(int mtab) {
   std::vector<double> t((size_t)(mtab + 1) * mtab * 4, 0.0);
   for (int m = 2; m <= mtab; m++) {
     double *r = &t[(size_t)m * mtab * 4];
     const double w0 = 1.0 + 2.0 / (13.0 * m * m);
-    const double temp1 = w0 * w0 - 1.0;
-    const double temp2 = std::sqrt(temp1);
-    const double arg = m * std::log(w0 + temp2);
-    const double w1 = std::sinh(arg) * temp1 / (std::cosh(arg) * m * temp2 - w0 * std::sinh(arg));
+    double w1;
+    rkc_stage_start(m, &w1, &r[0]);   // r[0]: the first stage's multiplier of h F_0
     double bjm1 = 1.0 / ((2.0 * w0) * (2.0 * w0)), bjm2 = bjm1;
-    r[0] = w1 * bjm1;   // mu~_1, the first stage's multiplier of h F_0
     double zjm1 = w0, zjm2 = 1.0, dzjm1 = 1.0, dzjm2 = 0.0, d2zjm1 = 0.0, d2zjm2 = 0.0;
     for (int j = 1; j < m; j++) {
       const double zj = 2.0 * w0 * zjm1 - zjm2;

@@ -37,12 +37,20 @@ struct RkcCtl {
   unsigned q, ions_q;         // numbers (modulo 3) of the next sum and gap-current exchange
   int ghost_used;             // coupled-value exchanges before the last sum
   int loops;
+  int m;                      // stages of the attempt that stopped the kernel (status ASK_STAGE)
+  int ghost_now;              // coupled-value exchanges since the last sum
 };
 
-// Stage counts up to RES_COEF read their coefficients from the table; larger
-// ones run the recurrence in the kernel
-constexpr int ASK_POW = 9;   // status: the host has to give the powers of err
+// Stage counts up to RES_COEF read their coefficients from the table.  Larger
+// ones run the recurrence in the kernel from w1 and mu~_1, whose logarithm and
+// hyperbolic functions the host's libm gives: a table up to RES_START stages, and
+// beyond it the kernel ends to ask.  (The device's own functions differ in the
+// last bit, which a step of 176 stages, taken by Golgi cells as their synaptic
+// input sets in, carries to 1e-10 mV.)
+constexpr int ASK_POW = 9;     // status: the host has to give the powers of err
+constexpr int ASK_STAGE = 10;  // status: the host has to give w1 and mu~_1 for m
 constexpr int RES_COEF = 128;
+constexpr int RES_START = 4096;
 constexpr int ROW_W = 3;            // neighbours of a compartment held in registers (parent and two children)
 constexpr int GHOST_STAGES = 136;   // exchanges of coupled values between two sums
 
@@ -75,9 +83,13 @@ struct RkcArgs {
   unsigned gq0;                          // number of the launch's first ion update
   double *y, *yn, *fn, *ede, *vnew, *b, *v1, *v2;
   const double *cm, *coef;
+  const double2 *start;                  // {w1, mu~_1} of m = 0 .. RES_START stages
   RkcCtl *ctl, *ctl_host;                // the record, and its copy in mapped host memory
-  int resume;                            // 1: the attempt that stopped goes on with err's powers p1, p2
+  // the attempt that stopped goes on: ASK_POW with err's powers p1, p2,
+  // ASK_STAGE with w1 and mu~_1 in asked (0: no attempt stopped)
+  int resume;
   double p1, p2;
+  double2 asked;
   double integ, rho_floor;
   int strict, refresh_fn;
   // per macro step: the stimulus, the Poisson drive, the recorder
@@ -239,8 +251,8 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, const typena
   bool last = ctl->last, newspc = ctl->newspc, jacatt = ctl->jacatt;
   unsigned q = ctl->q, gq = A.gq0;
   int status = 0, done_steps = 0;
-  bool resume = A.resume != 0;
-  int loops = ctl->loops;
+  int resume = A.resume;
+  int loops = ctl->loops, m_now = ctl->m;
   CubeRoots ce;
   ce.p1 = A.p1;
   ce.p2 = A.p2;
@@ -259,7 +271,7 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, const typena
       YN[i] = A.yn[r0 + i];
       FN[i] = A.fn[r0 + i];
       T[i] = A.b[r0 + i];
-      if (resume) {
+      if (resume == ASK_POW) {
         V1[i] = A.v1[r0 + i];
         V2[i] = A.v2[r0 + i];
       }
@@ -311,7 +323,7 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, const typena
   // coupled cells: the neighbours' compartments of vector v into its tail.
   // Every exchange between two sums has slots of its own; they are emptied
   // like the sum's, after the next one.
-  int gs = 0, gs_old = ctl->ghost_used;
+  int gs = ctl->ghost_now, gs_old = ctl->ghost_used;
   const bool coupled = A.imp0 != nullptr;
   auto finish_sum = [&]() {
     const double s = total();
@@ -451,8 +463,8 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, const typena
   };
 
   // step (solve_rkc.cu:815-906)
-  auto step = [&](double h, int m) {
-    double w0 = 0.0, w1 = 0.0, mus;
+  auto step = [&](double h, int m, double w1, double mus) {
+    double w0 = 0.0;
     const bool tab = m >= 2 && m <= RES_COEF;
     if (tab) {
       const double *ct = A.coef + (size_t)m * RES_COEF * 4;
@@ -460,10 +472,6 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, const typena
       mus = ct[0];
     } else {
       w0 = 1.0 + 2.0 / (13.0 * m * m);
-      const double t1 = w0 * w0 - 1.0, t2 = sqrt(t1);
-      const double arg = m * log(w0 + t2);
-      w1 = sinh(arg) * t1 / (cosh(arg) * m * t2 - w0 * sinh(arg));
-      mus = w1 * (1.0 / ((2.0 * w0) * (2.0 * w0)));
     }
     const double hm = h * mus;
     for (int i = tid; i < R; i += NT) {
@@ -524,27 +532,39 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, const typena
 
   // an attempt of rkclow (solve_rkc.cu:908-1096) up to its error norm
   auto attempt = [&]() {
-    if (newspc) {
-      rkcrho();
-      if (sprad < A.rho_floor) sprad = A.rho_floor;
-      jacatt = true;
-    }
-    last = false;
-    if (1.1 * absh >= fabs(tend - lt)) {
-      absh = fabs(tend - lt);
-      last = true;
-    }
-    const double mr = sqrt(1.54 * absh * sprad + 1.0);
-    int m = (mr < mmax) ? 1 + (int)mr : (int)mmax + 1;
-    if (m > mmax) {
-      m = (int)mmax;
-      absh = (m * m - 1) / (1.54 * sprad);
+    double2 w = A.asked;
+    if (!resume) {
+      if (newspc) {
+        rkcrho();
+        if (sprad < A.rho_floor) sprad = A.rho_floor;
+        jacatt = true;
+      }
       last = false;
+      if (1.1 * absh >= fabs(tend - lt)) {
+        absh = fabs(tend - lt);
+        last = true;
+      }
+      const double mr = sqrt(1.54 * absh * sprad + 1.0);
+      int m = (mr < mmax) ? 1 + (int)mr : (int)mmax + 1;
+      if (m > mmax) {
+        m = (int)mmax;
+        absh = (m * m - 1) / (1.54 * sprad);
+        last = false;
+      }
+      double h = absh;
+      if (h <= hmin) h = hmin;
+      h_now = h;
+      m_now = m;
+      if (m > RES_START) {
+        status = ASK_STAGE;
+        return;
+      }
+      if (m < 2 || m > RES_COEF) w = A.start[m];
     }
-    double h = absh;
-    if (h <= hmin) h = hmin;
-    h_now = h;
-    step(h, m);
+    resume = 0;
+    const double h = h_now;
+    const int m = m_now;
+    step(h, m, w.x, w.y);
     // f(Y_m) and the error estimate (every weight is positive: atol > 0)
     fetch(Yv);
     double fo[K], to[K];
@@ -568,12 +588,12 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, const typena
   auto rkclow = [&]() {
     if (!resume) loops = 0;
     while (!late) {
-      if (resume) {
-        resume = false;
+      if (resume == ASK_POW) {
+        resume = 0;
       } else {
-        if (++loops > 1000) return;
+        if (!resume && ++loops > 1000) return;
         attempt();
-        if (late) return;
+        if (late || status != 0) return;
         if (!isfinite(err)) {
           status = Model::NONFINITE_STATUS;
           return;
@@ -707,7 +727,7 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, const typena
     c.steps = s_cnt[0]; c.rejects = s_cnt[1]; c.stages = s_cnt[2]; c.rho_iters = s_cnt[3]; c.ions = s_cnt[4];
     c.macro += done_steps;
     c.last = last; c.newspc = newspc; c.jacatt = jacatt; c.status = status;
-    c.q = q; c.ions_q = gq; c.ghost_used = gs_old; c.loops = loops;
+    c.q = q; c.ions_q = gq; c.ghost_used = gs_old; c.loops = loops; c.m = m_now; c.ghost_now = gs;
     *ctl = c;
     *A.ctl_host = c;
   }

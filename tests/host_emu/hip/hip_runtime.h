@@ -34,7 +34,8 @@ inline const char *hipGetErrorString(hipError_t) { return "host stand-in"; }
 // the wavefront exchanges of a 64-lane workgroup, and the device's atomics.
 #define __HIP_MEMORY_SCOPE_AGENT 0
 #define __hip_atomic_store(p, v, order, scope) __atomic_store_n(p, v, order)
-#define __hip_atomic_load(p, order, scope) __atomic_load_n(p, order)
+#define __hip_atomic_load(p, order, scope) (emu_pause(), __atomic_load_n(p, order))
+void emu_pause();
 void emu_syncthreads();
 int emu_syncthreads_or(int x);
 double emu_shfl_down(double x, int off);
@@ -55,6 +56,9 @@ inline int __double2hiint(double x) { return (int)(__double_as_longlong(x) >> 32
 inline double __hiloint2double(int hi, int lo) { return __longlong_as_double((long long)hi << 32 | (unsigned)lo); }
 struct uint2 {
   unsigned x, y;
+};
+struct double2 {
+  double x, y;
 };
 inline uint2 make_uint2(unsigned x, unsigned y) { return {x, y}; }
 inline int min(int a, int b) { return a < b ? a : b; }

@@ -46,6 +46,7 @@ thread_local emu_dim3 blockIdx;
 double emu_shfl_xor(double x, int) { return x; }
 void emu_wave_barrier() { t_group->bar.wait(); }
 void emu_syncthreads() { t_group->bar.wait(); }
+void emu_pause() { std::this_thread::yield(); }   // a poll lets the other lanes run
 int emu_syncthreads_or(int x) {
   t_group->is[threadIdx.x] = x;
   t_group->bar.wait();
@@ -80,6 +81,7 @@ static int *emu_late() { return &t_group->late; }
 
 namespace cbrkc {
 std::vector<double> rkc_stage_table(int mtab);
+void rkc_stage_start(int m, double *w1, double *mus);
 
 struct Still {   // constant frozen currents
   struct State {
@@ -95,12 +97,13 @@ using namespace cbrkc;
 extern "C" {
 // nsteps macro steps of n cells of comp rows (at most 64 K rows of a cell), cpb
 // cells to a workgroup, nhelp helpers to each; present: workgroups that are
-// started at all (fewer: the others wait in vain).  vec: y, yn, fn, ede, vnew.
+// started at all (fewer: the others wait in vain); launches: how often the
+// kernel was started.  vec: y, yn, fn, ede, vnew.
 // o16, hw8 and cnt5 (steps, rejects, stages, power iterations, ion updates)
 // come back.  Returns the last status.
 int emu_rkc(int n, int comp, int cpb, int nhelp, int present, const int *row, const int *col, const double *val,
             const double *cm, const double *b, double *vec, double *o16, double *hw8, long long *cnt5, int nsteps,
-            int *launches) {
+            double rho_floor, int refresh, int *launches) {
   const int nc = n * comp, RM = cpb * comp, nblk = (n + cpb - 1) / cpb;
   RkcArgs a{};
   a.n = n;
@@ -160,6 +163,8 @@ int emu_rkc(int n, int comp, int cpb, int nhelp, int present, const int *row, co
       parts((size_t)3 * a.nch, empty), gap((size_t)3 * n, empty), req((size_t)6 * nblk, empty),
       vin((size_t)3 * nc, empty), bout((size_t)3 * nc, empty), v1(nc), v2(nc), bb(b, b + nc), iext(nc), amp(n);
   const std::vector<double> table = rkc_stage_table(RES_COEF);
+  std::vector<double2> start(RES_START + 1);
+  for (int m = 0; m <= RES_START; m++) rkc_stage_start(m, &start[m].x, &start[m].y);
   if (nslot > 0) {
     a.imp0 = imp0.data();
     a.exp0 = exp0.data();
@@ -191,7 +196,10 @@ int emu_rkc(int n, int comp, int cpb, int nhelp, int present, const int *row, co
   a.v2 = v2.data();
   a.cm = cm;
   a.coef = table.data();
+  a.start = start.data();
   a.integ = 1e30;
+  a.rho_floor = rho_floor;
+  a.refresh_fn = refresh;
   a.iext = iext.data();
   a.amp = amp.data();
   RkcCtl ctl{}, host{};
@@ -232,11 +240,10 @@ int emu_rkc(int n, int comp, int cpb, int nhelp, int present, const int *row, co
         });
     for (auto &t : th) t.join();
     ++*launches;
-    a.resume = host.status == ASK_POW;
-    if (a.resume) {
-      a.p1 = std::pow(host.err, 1.0 / 3.0);
-      a.p2 = std::pow(host.err, 2.0 / 3.0);
-    }
+    a.resume = host.status == ASK_POW || host.status == ASK_STAGE ? host.status : 0;
+    a.p1 = std::pow(host.err, 1.0 / 3.0);
+    a.p2 = std::pow(host.err, 2.0 / 3.0);
+    if (host.status == ASK_STAGE) rkc_stage_start(host.m, &a.asked.x, &a.asked.y);
     if (host.status != 0 && !a.resume) break;
   }
   std::memcpy(o16, host.o, sizeof(host.o));

@@ -4,7 +4,7 @@ csrc/kry_resident.hpp) and the kernel launches per Chebyshev stage and Krylov
 iteration that larger populations take, and any population in a process that
 may not launch cooperatively.  Every voltage, current, gate, controller value,
 counter, recording and spike is the same bits, with ion updates, stimulus,
-gap junctions and Poisson drive; so the small populations here, and
+gap junctions, Poisson drive and synapses; so the small populations here, and
 with them the oracle's tests of either path, cover both."""
 import os
 
@@ -12,6 +12,7 @@ import numpy as np
 import pytest
 
 import cbrkc
+import test_gpu_net as TN
 
 pytestmark = pytest.mark.gpu
 
@@ -77,3 +78,32 @@ def test_krylov(ref_data, cell, nx, ny, solver):
     a.launch_path()
     assert np.array_equal(a.run(1, T0 + 0.25, -1), b.run(1, T0 + 0.25, -1))
     same(a, b, FIELDS)
+
+
+def test_network(ref_data, tmp_path):
+    # populations with their synapses: mossy fibres at a rate that
+    # makes granule cells fire, 3 ms
+    n = (64, 16, 3)
+    files = [str(tmp_path / f) for f in ("gr.txt", "go.txt", "pkj.txt")]
+    cbrkc.synth_gr_chains(files[0], os.path.join(ref_data, "Gr.txt"), 7, n[0])
+    cbrkc.synth_go_trees(files[1], os.path.join(ref_data, "Go_131.txt"), 8, n[1])
+    cbrkc.synth_pkj_morph(files[2], seed=9, ncell=n[2])
+    v0 = TN.v0_of(n)
+    pops, nets = [], []
+    for launches in (False, True):
+        p = TN.gpu_pops(files, v0)
+        for x in p:
+            if launches:
+                x.launch_path()
+        pops.append(p)
+        nets.append(cbrkc.Network(*p, cfg=cbrkc.net_config(seed=4, total=0, mf_rate_hz=200.0)))
+    for k in range(24):
+        print("interval", k, flush=True)
+        for net in nets:
+            net.run(1)
+        for x, y, name in zip(*pops, ("gr", "go")):
+            assert x.stats() == y.stats(), name
+            same(x, y, FIELDS + (cbrkc.F_Y, cbrkc.F_YN, cbrkc.F_FN))
+    for pop in (cbrkc.NET_GR, cbrkc.NET_GO, cbrkc.NET_PKJ):
+        g = [net.conductance(pop, cbrkc.NET_AMPA) for net in nets]
+        assert np.array_equal(*g) and g[0].any()

@@ -25,9 +25,12 @@ def emu(tmp_path_factory):
     return ctypes.CDLL(str(out / "libresident.so"))
 
 
-def run(emu, o, n, cpb=1, nsteps=1, nhelp=0, present=1 << 20):
+def run(emu, o, n, cpb=1, nsteps=1, nhelp=0, present=1 << 20, floor=0.0, refresh=False):
     """nsteps macro steps of the oracle population o, as n cells, on the host
-    build, from o's present state; o itself stays"""
+    build, from o's present state, with this floor of the spectral radius and
+    refresh of fn after ion updates; o itself stays"""
+    orc.lib().or_pop_set_rho_floor(o.h, floor)
+    orc.lib().or_pop_set_refresh_fn(o.h, 1 if refresh else 0)
     comp = o.nc // n
     row, col, val = o.csr()
     keep = [np.ascontiguousarray(x, dtype=np.float64) for x in (val, o.get(orc.CM), o.get(orc.B))]
@@ -38,7 +41,7 @@ def run(emu, o, n, cpb=1, nsteps=1, nhelp=0, present=1 << 20):
     launches = ctypes.c_int()
     p = lambda a: a.ctypes.data_as(ctypes.c_void_p)  # noqa: E731
     status = emu.emu_rkc(n, comp, cpb, nhelp, present, p(row), p(col), p(keep[0]), p(keep[1]), p(keep[2]), p(vec), p(c),
-                         p(hw), p(cnt), nsteps, ctypes.byref(launches))
+                         p(hw), p(cnt), nsteps, ctypes.c_double(floor), 1 if refresh else 0, ctypes.byref(launches))
     return dict(status=status, vec=vec, ctl=c[:14], hw=hw, cnt=cnt, launches=launches.value)
 
 
@@ -54,8 +57,8 @@ def check(o, r, nsteps=1):
     assert list(r["cnt"][:4]) == [s[k] for k in ("steps", "rejects", "stages", "rho_iters")]
 
 
-def cables(n, comp, g, seed=0, pairs=()):
-    """n chains of comp rows, their conductances about g, joined at pairs of rows"""
+def cables(n, comp, g, seed=0, pairs=(), spread=1.0):
+    """n chains of comp rows, their conductances about g, joined at pairs of rows; currents and voltages spread so far"""
     rng = np.random.default_rng(seed)
     L = np.zeros((n * comp, n * comp))
     for i in range(n * comp - 1):
@@ -63,8 +66,8 @@ def cables(n, comp, g, seed=0, pairs=()):
             L[i, i + 1] = L[i + 1, i] = g * rng.uniform(0.5, 1.5)
     for i, j in pairs:
         L[i, j] = L[j, i] = 0.3 * g
-    return orc.Pop.generic(L, rng.uniform(0.8, 1.2, n * comp), rng.uniform(-3.0, 3.0, n * comp),
-                           rng.uniform(-70.0, -60.0, n * comp))
+    return orc.Pop.generic(L, rng.uniform(0.8, 1.2, n * comp), spread * rng.uniform(-3.0, 3.0, n * comp),
+                           -65.0 + spread * rng.uniform(-5.0, 5.0, n * comp))
 
 
 @pytest.mark.parametrize("n,comp,cpb,nhelp", [(1, 40, 1, 0), (1, 150, 1, 2), (3, 20, 2, 0)])
@@ -76,6 +79,22 @@ def test_macro_steps(emu, n, comp, cpb, nhelp):
 def test_coupled_workgroups(emu):
     o = cables(2, 30, 5.0, pairs=[(3, 41), (29, 30), (3, 55)])
     check(o, run(emu, o, 2, nsteps=2), 2)
+
+
+@pytest.mark.parametrize("pairs,refresh", [((), False), ([(3, 41), (29, 30)], True)])
+@pytest.mark.parametrize("floor,m", [(2e5, 137), (6e8, 4097)])
+def test_many_stages(emu, floor, m, pairs, refresh):
+    # a spectral radius far above the cable's, as the power method gives it when
+    # synaptic input sets in: steps past the coefficient table and the coupled
+    # values' slots, and of more stages than RES_START, which the host is asked for
+    o = cables(2, 30, 0.5, pairs=pairs, spread=1e-3)
+    before = o.stats()
+    k = 1 if m > 4096 else 3
+    r = run(emu, o, 2, nsteps=k, floor=floor, refresh=refresh)
+    check(o, r, k)
+    s = o.stats()
+    assert s["stages"] - before["stages"] > m * (s["steps"] + s["rejects"] - before["steps"] - before["rejects"])
+    assert m < 4096 or r["launches"] >= 3 - refresh
 
 
 def test_power_method_when_the_perturbation_moves_nothing(emu):
