@@ -1158,7 +1158,7 @@ class GlobalPkj : public GlobalRkc {
     // the granule input enters at ion updates only (pkj_update_ion_and_matrix)
     const bool net = do_ion && net_.on();
     PkjState S{v_, ca_, rev_, iext_, shell_, cond_, gate_, b_, syn_g_, syn_.e_syn, nc_,
-               net ? net_s_ : nullptr, net ? std::exp(-dt / 0.6) : 0.0};
+               net ? net_s_ : nullptr, net ? exp_cr(-dt / 0.6) : 0.0};
     k_pkj_ion_b<<<nblk(nc_), 256, 0, st_>>>(S, vv, dt, do_ion ? 1 : 0);
   }
  public:

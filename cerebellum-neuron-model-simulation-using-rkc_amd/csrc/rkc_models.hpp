@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include "engine.hpp"
+#include "exp_acc.hpp"
 #include "ion_state.hpp"
 #include "pkj_model.hpp"
 #include "rkc_resident.hpp"
@@ -21,7 +22,7 @@ struct PkjState {
   double syn_e;
   int nc;
   const double *net_s;  // synaptic current of the macro step (granule input), may be null
-  double net_decay;     // exp(-dt / 0.6), dt the ion interval
+  double net_decay;     // exp(-dt / 0.6), dt the ion interval; correctly rounded on either path
 };
 
 // pkj_update_ion_RKC (pkj_ion.cu:304-358) followed by pkj_update_matrix
@@ -121,7 +122,7 @@ struct PkjModel {
   static constexpr bool GAP = false, HELP = true;
   __device__ __attribute__((noinline)) static double ion(const State *Sp, int i, double vn, double dt, GapView *) {
     State S = *Sp;
-    if (S.net_s) S.net_decay = exp(-dt / 0.6);
+    if (S.net_s) S.net_decay = exp_cr(-dt / 0.6);
     return pkj_ion_current(S, i, vn, dt, true);
   }
 };

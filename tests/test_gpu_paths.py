@@ -101,7 +101,7 @@ def test_network(ref_data, tmp_path):
         print("interval", k, flush=True)
         for net in nets:
             net.run(1)
-        for x, y, name in zip(*pops, ("gr", "go")):
+        for x, y, name in zip(*pops, ("gr", "go", "pkj")):
             assert x.stats() == y.stats(), name
             same(x, y, FIELDS + (cbrkc.F_Y, cbrkc.F_YN, cbrkc.F_FN))
     for pop in (cbrkc.NET_GR, cbrkc.NET_GO, cbrkc.NET_PKJ):
