@@ -77,7 +77,7 @@ int guarded(F &&f) {
     g_err = e.msg;
     if (e.msg.rfind("HIP error", 0) == 0) return CB_E_HIP;
     if (e.code > 0) return CB_E_SOLVER;
-    if (e.code == CB_E_UNSUP) return CB_E_UNSUP;
+    if (e.code == CB_E_UNSUP || e.code == CB_E_HIP) return e.code;
     return CB_E_ARG;
   } catch (const std::exception &e) {
     g_err = e.what();
@@ -704,6 +704,15 @@ int cb_pop_launch_path(cb_pop *p, int on) {
   return guarded([&]() -> int {
     if (!p) return fail(CB_E_ARG, "null population");
     if (!p->eng->use_launches(on != 0)) return fail(CB_E_UNSUP, "the population has one path only");
+    return CB_OK;
+  });
+}
+
+int cb_pop_wait_limit(cb_pop *p, double seconds) {
+  return guarded([&]() -> int {
+    if (!p) return fail(CB_E_ARG, "null population");
+    if (!(seconds >= 0.0) || seconds > 1e9) return fail(CB_E_ARG, "the limit must be 0 to 1e9 s");
+    p->eng->wait_limit(seconds);
     return CB_OK;
   });
 }

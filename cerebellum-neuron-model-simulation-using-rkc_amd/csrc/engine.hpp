@@ -85,6 +85,9 @@ class Engine {
   }
   // selects the mapping with this many threads per cell; false if none
   virtual bool select_mapping(int threads) { return threads == 0; }
+  // how long a workgroup of a kernel waits for another one's values before the
+  // call fails (engines whose workgroups wait for one another)
+  virtual void wait_limit(double seconds) { (void)seconds; }
   // on: a launch per stage or iteration instead of the kernel that runs whole
   // steps or solves (off: that kernel again); the results are the same bits.
   // False where the engine or the population's size leaves no choice.

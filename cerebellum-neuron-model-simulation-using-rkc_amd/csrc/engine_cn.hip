@@ -1220,6 +1220,7 @@ class CnEngine : public Engine {
     S_.direct = resident_ ? 1 : 0;
     return true;
   }
+  void wait_limit(double seconds) override { A_.wait = wait_ticks(seconds); }
   std::string mapping() const override {
     if (resident_)
       return "Krylov solve in one kernel, " + std::to_string(res_grid_) + " workgroups of " + std::to_string(A_.rb) + " rows";
@@ -1339,7 +1340,7 @@ class CnEngine : public Engine {
     cap = n;
   }
   void check_late() const {
-    if (late_host_ && *(volatile int *)late_host_) throw Error("CN / BE: a workgroup of the solve waited for another one in vain");
+    if (late_host_ && *(volatile int *)late_host_) throw Error("CN / BE: a workgroup of the solve waited for another one in vain", -3);
   }
 
   template <typename T>
@@ -1470,7 +1471,8 @@ class CnEngine : public Engine {
     std::memcpy(&empty, &e, sizeof(empty));
     a.ghost = res_put(std::vector<double>((size_t)6 * std::max(1, a.nslot), empty));
     a.parts = res_put(std::vector<double>((size_t)3 * a.nch, empty));
-    a.q = res_put(std::vector<unsigned>(1, 0u));
+    a.q = res_put(std::vector<unsigned>(2, 0u));
+    a.wait = WAIT_TICKS;
     a.lrow = res_put(lrow);
     a.lcol = res_put(lcol);
     a.ldpos = res_put(ldpos);

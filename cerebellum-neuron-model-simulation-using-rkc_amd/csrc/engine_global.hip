@@ -377,6 +377,7 @@ class GlobalRkc : public Engine {
     std::memcpy(o, o_, sizeof(o_));
     std::memcpy(hw, hw_, sizeof(hw_));
   }
+  void wait_limit(double seconds) override { A_.wait = wait_ticks(seconds); }
   std::string mapping() const override {
     if (!resident_) return "one thread per compartment, one launch per stage";
     return std::to_string(A_.nblk) + " workgroups of " + std::to_string(A_.cpb) +
@@ -596,7 +597,7 @@ class GlobalRkc : public Engine {
     if (c.status == 0 || A_.resume) return;
     if (c.status == NONFINITE)
       throw Error("RKC: non-finite state (error estimate " + std::to_string(c.err) + ")", NONFINITE);
-    if (c.status == TIMED_OUT) throw Error("RKC: a workgroup of the step kernel waited for another one in vain");
+    if (c.status == TIMED_OUT) throw Error("RKC: a workgroup of the step kernel waited for another one in vain", -3);
     throw Error("RKC failed: idid = " + std::to_string(c.status), c.status);
   }
 
@@ -772,6 +773,7 @@ class GlobalRkc : public Engine {
     CB_HIP(hipHostMalloc((void **)&ctl_host_, sizeof(RkcCtl), hipHostMallocMapped | hipHostMallocCoherent));
     *ctl_host_ = c;
     CB_HIP(hipHostGetDevicePointer((void **)&a.ctl_host, ctl_host_, 0));
+    a.wait = WAIT_TICKS;
     a.integ = integ_;
     a.rho_floor = rho_floor_;
     a.strict = res_strict();

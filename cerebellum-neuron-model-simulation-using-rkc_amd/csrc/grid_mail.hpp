@@ -14,9 +14,14 @@
 // exchange q + 1 knows that all of q + 2's slots are empty.  The number of the
 // next exchange (modulo 3) is kept with the controller between launches.
 //
-// Every wait ends: a poll gives up after SPIN_TICKS of the 100 MHz clock and
-// the kernel then reports TIMED_OUT.  All workgroups have to be resident, so
-// kernels with more than one are launched cooperatively.
+// Every wait ends: a poll gives up after the population's limit (60 s unless it
+// is set), and from then on no wait of that workgroup lasts: whoever gives up
+// marks the workgroup's LDS word, every other poll looks at it, and the kernel
+// leaves its loops at the next sum and reports TIMED_OUT.  What the limit bounds
+// is so a launch, not a poll: the workgroups wait for a lost one side by side, in
+// a chain of coupled values and then in the sum, about two limits in all.  All
+// workgroups have to be resident, so kernels with more than one are launched
+// cooperatively.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -28,7 +33,15 @@ namespace cbrkc {
 
 constexpr int TIMED_OUT = 8;   // status: a workgroup waited for another one in vain
 constexpr unsigned long long MAIL_EMPTY = 0x7FF4CE11AB1E0001ull;   // a NaN no arithmetic makes
-constexpr unsigned long long SPIN_TICKS = 60ull * 100000000ull;    // 60 s
+constexpr unsigned long long WAIT_TICKS = 60ull * 100000000ull;    // the limit of a wait: 60 s of the 100 MHz clock
+
+inline unsigned long long wait_ticks(double seconds) { return (unsigned long long)(seconds * 1e8); }
+
+// The limit of a wait and the workgroup's LDS word that is set once one gave up
+struct Wait {
+  unsigned long long ticks;
+  volatile int *late;
+};
 
 __device__ inline void mail_put(double *slot, double v) {
   unsigned long long b = (unsigned long long)__double_as_longlong(v);
@@ -38,33 +51,36 @@ __device__ inline void mail_put(double *slot, double v) {
 __device__ inline void mail_clear(double *slot) {
   __hip_atomic_store((unsigned long long *)slot, MAIL_EMPTY, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// the slot's value once it is there; *late is set when the wait gives up
-__device__ inline double mail_get(const double *slot, int *late) {
+// the slot's value once it is there, or 0 when the wait gives up (with a limit
+// of 0 at the first look that finds nothing)
+__device__ inline double mail_get(const double *slot, const Wait &W) {
   unsigned long long b = __hip_atomic_load((const unsigned long long *)slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if (b == MAIL_EMPTY) {
     const unsigned long long t0 = wall_clock64();
-    int n = 0;
-    do {
+    bool give_up = *W.late || W.ticks == 0;
+    for (int n = 1; !give_up; n++) {
       b = __hip_atomic_load((const unsigned long long *)slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if ((++n & 1023) == 0 && wall_clock64() - t0 > SPIN_TICKS) {
-        *late = 1;
-        return 0.0;
-      }
-    } while (b == MAIL_EMPTY);
+      if (b != MAIL_EMPTY) break;
+      if ((n & 1023) == 0) give_up = *W.late || wall_clock64() - t0 > W.ticks;
+    }
+    if (give_up) {
+      *W.late = 1;
+      return 0.0;
+    }
   }
   return __longlong_as_double((long long)b);
 }
 // mail_get for a wait that may be long: it leaves 256 cycles between looks
-__device__ inline double mail_wait(const double *slot, int *late) {
+__device__ inline double mail_wait(const double *slot, const Wait &W) {
   const unsigned long long t0 = wall_clock64();
   while (__hip_atomic_load((const unsigned long long *)slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == MAIL_EMPTY) {
     __builtin_amdgcn_s_sleep(4);
-    if (wall_clock64() - t0 > SPIN_TICKS) {
-      *late = 1;
+    if (*W.late || wall_clock64() - t0 > W.ticks) {
+      *W.late = 1;
       return 0.0;
     }
   }
-  return mail_get(slot, late);
+  return mail_get(slot, W);
 }
 // the thread's own stores have reached memory
 __device__ inline void mail_settle() {
@@ -111,12 +127,12 @@ struct SumPlan {
 // The total of the rows' terms.  term (LDS): the workgroup's own rows, filled
 // by the same thread for i = tid, tid + NT, ..., with room for 255 more; part
 // (LDS): nch + 8 doubles; terms [3][nc] and parts [3][nch]: mailboxes; q: the
-// exchange's number modulo 3, advanced.  late becomes set for the whole
+// exchange's number modulo 3, advanced.  late becomes true for the whole
 // workgroup when any of its waits gave up.  The order is that of k_reduce256 over the
 // whole vector, so the total equals the multi-launch reduction bit for bit.
 template <int NT>
 __device__ inline double grid_sum(const SumPlan &P, double *term, double *part, double *terms, double *parts,
-                                  unsigned &q, int *late) {
+                                  unsigned &q, const Wait &W, bool &late) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, R = P.r1 - P.r0;
   double *tq = terms + (size_t)q * P.nc, *pq = parts + (size_t)q * P.nch;
   if (!P.alone) {
@@ -125,7 +141,7 @@ __device__ inline double grid_sum(const SumPlan &P, double *term, double *part, 
     // its waves' emptied slots have to be settled before the first of them
     if (P.nown == 0) __syncthreads();
     for (int i = tid; i < P.head; i += NT) mail_put(tq + P.r0 + i, term[i]);
-    for (int i = tid; i < P.tail; i += NT) term[R + i] = mail_get(tq + P.r1 + i, late);
+    for (int i = tid; i < P.tail; i += NT) term[R + i] = mail_get(tq + P.r1 + i, W);
   }
   __syncthreads();
   for (int c = wave; c < P.nown; c += NT / 64) {
@@ -139,9 +155,9 @@ __device__ inline double grid_sum(const SumPlan &P, double *term, double *part, 
     }
   }
   if (!P.alone)
-    for (int k = tid; k < P.nch; k += NT) part[k] = mail_get(pq + k, late);
+    for (int k = tid; k < P.nch; k += NT) part[k] = mail_get(pq + k, W);
   if (P.alone) __syncthreads();
-  else *late = __syncthreads_or(*late);
+  else late = __syncthreads_or(*W.late);
   // the partials by the same tree, level by level (at most 2048 of them)
   int m = P.nch;
   const double *in = part;

@@ -42,8 +42,9 @@ struct KryArgs {
   double *ghost;                         // [3][2][nslot]: r, and BiCG's shadow residual
   int nslot;
   double *parts;                         // [3][nch]
-  unsigned *q;                           // number (modulo 3) of the next sum
-  int *late;                             // mapped host memory: a wait gave up
+  unsigned *q;                           // number (modulo 3) of the next sum; nonzero once a wait gave up
+  int *late;                             // the same in mapped host memory
+  unsigned long long wait;               // the limit of a wait (grid_mail.hpp)
   const double *diag, *b;
   double *v;
   int *flag, f_done, f_iters, f_total;
@@ -52,6 +53,7 @@ struct KryArgs {
 template <int NT, int K, bool BICG>
 __global__ void __launch_bounds__(NT) k_kry_resident(KryArgs A) {
   extern __shared__ double sm[];
+  __shared__ int s_late;
   const int tid = threadIdx.x, w = blockIdx.x, r0 = w * A.rb, R = min(A.rb, A.nc - r0), ps = A.rb + A.ghost_max;
   double *P = sm, *PS = P + ps, *T = BICG ? PS + ps : PS, *part = T + A.rb, *LV = part + A.nch + 8;
   double *TV = LV + A.nnz_max;
@@ -59,8 +61,13 @@ __global__ void __launch_bounds__(NT) k_kry_resident(KryArgs A) {
   unsigned short *TR = LC + A.nnz_max, *TC = TR + A.rb + 1;
   SumPlan S;
   S.set(A.nc, r0, r0 + R);
-  int late = 0;
-  unsigned q = *A.q;
+  const Wait W{A.wait, &s_late};
+  bool late = false;
+  unsigned q = A.q[0];
+  // a solve before this one ended with its mailboxes half read: those already
+  // queued after it fall through
+  if (A.q[1]) return;
+  if (tid == 0) s_late = 0;
   const int z0 = A.lnz0[w], nz = A.lnz0[w + 1] - z0;
   for (int k = tid; k < nz; k += NT) {
     LV[k] = A.lval[z0 + k];
@@ -109,7 +116,7 @@ __global__ void __launch_bounds__(NT) k_kry_resident(KryArgs A) {
     P[A.rb + g] = bi;
     if (BICG) PS[A.rb + g] = bi;
   }
-  auto sum = [&]() { return grid_sum<NT>(S, T, part, (double *)nullptr, A.parts, q, &late); };
+  auto sum = [&]() { return grid_sum<NT>(S, T, part, (double *)nullptr, A.parts, q, W, late); };
   const double bnorm = sum();
   double rr = bnorm, beta = 0.0;
   int iters = 0, done = 0;
@@ -125,8 +132,8 @@ __global__ void __launch_bounds__(NT) k_kry_resident(KryArgs A) {
         }
       }
       for (int g = tid; g < ng; g += NT) {
-        P[A.rb + g] = beta * P[A.rb + g] + mail_get(gq + g0 + g, &late);
-        if (BICG) PS[A.rb + g] = beta * PS[A.rb + g] + mail_get(gq + A.nslot + g0 + g, &late);
+        P[A.rb + g] = beta * P[A.rb + g] + mail_get(gq + g0 + g, W);
+        if (BICG) PS[A.rb + g] = beta * PS[A.rb + g] + mail_get(gq + A.nslot + g0 + g, W);
       }
       __syncthreads();
     }
@@ -201,7 +208,10 @@ __global__ void __launch_bounds__(NT) k_kry_resident(KryArgs A) {
     const int i = tid + j * NT;
     if (i < R) A.v[r0 + i] = x[j];
   }
-  if (tid == 0 && late) *A.late = 1;
+  if (tid == 0 && late) {
+    A.q[1] = 1u;
+    *A.late = 1;
+  }
   if (w == 0 && tid == 0) {
     A.flag[A.f_iters] = iters;
     A.flag[A.f_done] = 1;

@@ -120,7 +120,7 @@ struct PkjModel {
   using State = PkjState;
   static constexpr int NT = 512, K0 = 0, K1 = 0, K2 = 4, NONFINITE_STATUS = NONFINITE;
   static constexpr bool GAP = false, HELP = true;
-  __device__ __attribute__((noinline)) static double ion(const State *Sp, int i, double vn, double dt, GapView *) {
+  __device__ __attribute__((noinline)) static double ion(const State *Sp, int i, double vn, double dt, const GapView *) {
     State S = *Sp;
     if (S.net_s) S.net_decay = exp_cr(-dt / 0.6);
     return pkj_ion_current(S, i, vn, dt, true);
@@ -130,7 +130,7 @@ struct IoModel {
   using State = IoState;
   static constexpr int NT = 256, K0 = 0, K1 = 1, K2 = 7, NONFINITE_STATUS = NONFINITE;
   static constexpr bool GAP = true, HELP = false;
-  __device__ __forceinline__ static double ion(const State *S, int i, double vn, double dt, GapView *gap) {
+  __device__ __forceinline__ static double ion(const State *S, int i, double vn, double dt, const GapView *gap) {
     return io_ion_gap_current(*S, i, vn, dt, true, [&](int cell) { return (*gap)(cell); });
   }
 };
@@ -138,7 +138,7 @@ struct GoModel {
   using State = GoState;
   static constexpr int NT = 256, K0 = 0, K1 = 1, K2 = 7, NONFINITE_STATUS = NONFINITE;
   static constexpr bool GAP = false, HELP = false;
-  __device__ __forceinline__ static double ion(const State *S, int i, double vn, double dt, GapView *) {
+  __device__ __forceinline__ static double ion(const State *S, int i, double vn, double dt, const GapView *) {
     return go_ion_net_current(*S, i, vn, dt, true);
   }
 };
@@ -146,7 +146,7 @@ struct GrModel {
   using State = GrState;
   static constexpr int NT = 256, K0 = 1, K1 = 3, K2 = 7, NONFINITE_STATUS = NONFINITE;
   static constexpr bool GAP = false, HELP = true;
-  __device__ __attribute__((noinline)) static double ion(const State *S, int i, double vn, double dt, GapView *) {
+  __device__ __attribute__((noinline)) static double ion(const State *S, int i, double vn, double dt, const GapView *) {
     return gr_ion_net_current(*S, i, vn, dt, true);
   }
 };

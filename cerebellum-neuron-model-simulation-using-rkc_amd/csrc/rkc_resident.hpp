@@ -69,6 +69,7 @@ struct RkcArgs {
   const double *xval;
   const int *x0;                         // first further entry of each workgroup (nblk + 1)
   const int *imp0, *exp0, *exp_row, *exp_slot;   // ghosts fetched, rows posted (null: uncoupled cells)
+  unsigned long long wait;               // the limit of a wait (grid_mail.hpp)
   double *ghost;                         // [3][GHOST_STAGES][nslot]
   int nslot;
   double *terms, *parts;                 // grid_sum's mailboxes
@@ -155,10 +156,11 @@ __device__ inline CubeRoots cube_roots(double x) {
 // the workgroup's vector or in the mailbox
 struct GapView {
   const double *y, *gap;
-  int cell0, cells, comp, late;
-  __device__ double operator()(int cell) {
+  int cell0, cells, comp;
+  const Wait *wait;
+  __device__ double operator()(int cell) const {
     if (cell >= cell0 && cell < cell0 + cells) return y[(cell - cell0) * comp];
-    return mail_get(gap + cell, &late);
+    return mail_get(gap + cell, *wait);
   }
 };
 
@@ -180,14 +182,17 @@ __device__ inline void rkc_helper(const RkcArgs &A, const typename Model::State 
   constexpr int NT = Model::NT;
   const int tid = threadIdx.x, RM = A.cpb * A.comp, R = min(RM, A.nc - w * RM);
   const int l0 = min(R, (j + 1) * A.own), l1 = min(R, l0 + A.own), r0 = w * RM;
-  int late = 0;
+  __shared__ int s_late;
+  if (tid == 0) s_late = 0;
+  const Wait W{A.wait, &s_late};
   for (unsigned g = A.gq0;; g = g == 2 ? 0 : g + 1) {
     if (tid == 0) {
       const double *rq = A.req + ((size_t)g * A.nblk + w) * 2;
-      sm[0] = mail_wait(rq, &late);
-      sm[1] = mail_get(rq + 1, &late);
+      sm[0] = mail_wait(rq, W);
+      sm[1] = mail_get(rq + 1, W);
     }
-    late = __syncthreads_or(late);
+    __syncthreads();
+    const bool late = s_late;
     const double dt = sm[0], t = sm[1];
     __syncthreads();
     const size_t copy = (size_t)g * A.nc, old = (size_t)(g == 0 ? 2 : g - 1) * A.nc;
@@ -197,7 +202,11 @@ __device__ inline void rkc_helper(const RkcArgs &A, const typename Model::State 
       const int row = r0 + i;
       if (A.do_stim && row % A.comp == A.stim_comp)
         A.iext[row] = (A.stim_t0 <= t && t < A.stim_t1) ? A.amp[row / A.comp] : 0.0;
-      if (!late && dt >= 0.0) mail_put(A.bout + copy + row, Model::ion(S, row, mail_get(A.vin + copy + row, &late), dt, nullptr));
+      if (!late && dt >= 0.0) {
+        const double vn = mail_get(A.vin + copy + row, W);
+        // without its voltages the helper posts nothing, and its workgroup gives up in turn
+        if (!*W.late) mail_put(A.bout + copy + row, Model::ion(S, row, vn, dt, nullptr));
+      }
       mail_clear(A.bout + old + row);
     }
     if (late || !(dt >= 0.0)) return;
@@ -226,7 +235,10 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, const typena
   double *Yv = sm, *YN = Yv + RS, *FN = YN + RS, *V1 = FN + RS, *V2 = V1 + RS;
   double *T = V2 + RS, *part = T + RM + RED_BLOCK, *C4 = part + A.nch + 8, *XV = C4 + 4 * RES_COEF;
   unsigned short *XC = (unsigned short *)(XV + A.ext_max);
-  int late = 0;
+  __shared__ int s_late;
+  if (tid == 0) s_late = 0;
+  const Wait W{A.wait, &s_late};
+  bool late = false;   // the same in the whole workgroup: s_late as of the last sum or ion update
   SumPlan P;
   P.set(A.nc, r0, r0 + R);
 
@@ -319,7 +331,7 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, const typena
       if (i < R) f(k, i);
     }
   };
-  auto total = [&]() { return grid_sum<NT>(P, T, part, A.terms, A.parts, q, &late); };
+  auto total = [&]() { return grid_sum<NT>(P, T, part, A.terms, A.parts, q, W, late); };
   // coupled cells: the neighbours' compartments of vector v into its tail.
   // Every exchange between two sums has slots of its own; they are emptied
   // like the sum's, after the next one.
@@ -341,7 +353,7 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, const typena
     double *g = A.ghost + ((size_t)q * GHOST_STAGES + gs) * A.nslot;
     for (int k = A.exp0[w] + tid; k < A.exp0[w + 1]; k += NT) mail_put(g + A.exp_slot[k], v[A.exp_row[k]]);
     const int m0 = A.imp0[w], ni = A.imp0[w + 1] - m0;
-    for (int k = tid; k < ni; k += NT) v[R + k] = mail_get(g + m0 + k, &late);
+    for (int k = tid; k < ni; k += NT) v[R + k] = mail_get(g + m0 + k, W);
     gs++;
     __syncthreads();
   };
@@ -370,14 +382,13 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, const typena
         }
       }
     }
-    GapView gv{Yv, A.gap + (size_t)gq * A.n, cell0, cells, A.comp, 0};
+    const GapView gv{Yv, A.gap + (size_t)gq * A.n, cell0, cells, A.comp, &W};
     const int own = helped ? min(R, A.own) : R;
     if (helped) request(dt, own);
 #pragma unroll 1
     for (int i = tid; i < own; i += NT) T[i] = Model::ion(S, r0 + i, Yv[i], dt, &gv);
-    late |= gv.late;
     if (helped) {
-      for (int i = own + tid; i < R; i += NT) T[i] = mail_get(A.bout + (size_t)gq * A.nc + r0 + i, &late);
+      for (int i = own + tid; i < R; i += NT) T[i] = mail_get(A.bout + (size_t)gq * A.nc + r0 + i, W);
       forget(own);
       __syncthreads();   // T's rows change threads here
     }
@@ -388,7 +399,7 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, const typena
       fetch(YN);
       rows([&](int k, int i) { FN[i] = rhs(k, YN[i], YN); });
     }
-    late = __syncthreads_or(late);
+    late = __syncthreads_or(s_late);
   };
 
   // rkcrho (solve_rkc.cu:562-754)

@@ -211,6 +211,13 @@ int cb_pop_mapping(const cb_pop *p, char *buf, int len);
  * only.  No counterpart in the reference. */
 int cb_pop_launch_path(cb_pop *p, int on);
 
+/* Population-global RKC, CN and BE engines: how long a workgroup waits for
+ * values of another one, which is not running, before the call fails with
+ * CB_E_HIP (60 s unless set; 0 to 1e9).  Other work that fills the GPU counts: raise
+ * it where single kernels of other programs or streams may run longer.  Not to be
+ * called beside another call on the population.  No counterpart in the reference. */
+int cb_pop_wait_limit(cb_pop *p, double seconds);
+
 /* Global-controller scalars: h_others[14] and h_work[8] (param.h:22,
  * solve_rkc.cu:453-476).  CB_E_UNSUP for per-cell engines. */
 int cb_pop_controller(const cb_pop *p, double *others14, double *hwork8);

@@ -89,7 +89,7 @@ struct Still {   // constant frozen currents
   };
   static constexpr int NT = 64, NONFINITE_STATUS = 7;
   static constexpr bool GAP = false, HELP = true;
-  static double ion(const State *S, int i, double, double, GapView *) { return S->b[i]; }
+  static double ion(const State *S, int i, double, double, const GapView *) { return S->b[i]; }
 };
 }  // namespace cbrkc
 using namespace cbrkc;
@@ -103,7 +103,7 @@ extern "C" {
 // come back.  Returns the last status.
 int emu_rkc(int n, int comp, int cpb, int nhelp, int present, const int *row, const int *col, const double *val,
             const double *cm, const double *b, double *vec, double *o16, double *hw8, long long *cnt5, int nsteps,
-            double rho_floor, int refresh, int *launches) {
+            double rho_floor, int refresh, double wait, int *launches) {
   const int nc = n * comp, RM = cpb * comp, nblk = (n + cpb - 1) / cpb;
   RkcArgs a{};
   a.n = n;
@@ -198,6 +198,7 @@ int emu_rkc(int n, int comp, int cpb, int nhelp, int present, const int *row, co
   a.coef = table.data();
   a.start = start.data();
   a.integ = 1e30;
+  a.wait = wait_ticks(wait);
   a.rho_floor = rho_floor;
   a.refresh_fn = refresh;
   a.iext = iext.data();

@@ -11,7 +11,12 @@
   each macro step is exactly one accepted step per controller, whatever its
   error; rejections that fall below hmin are counted and then accepted, and
   the run ends without an error.
+* A workgroup that waits for another one in vain: with a limit of no time at
+  all (cb_pop_wait_limit) the first empty mailbox ends the launch, and the call
+  fails at once; solves already queued fall through.
 """
+import time
+
 import numpy as np
 import pytest
 
@@ -57,3 +62,21 @@ def test_steps_below_hmin_fall_through_as_accepted(morph2, engine):
     assert s1["steps"] - s0["steps"] == 6 * ncontrollers, (s0, s1)
     # some 0.125 ms steps miss the 1e-6 tolerance: rejected, then accepted at hmin
     assert s1["rejects"] - s0["rejects"] > 0, (s0, s1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("solver", [cbrkc.CN, cbrkc.BE], ids=["cn", "be"])
+def test_a_solve_that_waits_in_vain_fails_the_run(tmp_path, solver):
+    print(f"4 Purkinje cells, solver {solver}, no time to wait", flush=True)
+    morph = str(tmp_path / "pkj4.txt")
+    cbrkc.synth_pkj_morph(morph, seed=7, ncell=4)
+    p = cbrkc.Population(cbrkc.PKJ, 4, 1, solver=solver, morph=morph, v0=[-68.0, -67.0, -66.0, -67.5])
+    assert "13 workgroups" in p.mapping()
+    p.wait_limit(0.0)
+    t0 = time.monotonic()
+    with pytest.raises(cbrkc.CbError, match="in vain"):
+        p.run(4, 0.0, 0)   # 20 solves, queued before the first is looked at
+    p.wait_limit(60.0)   # what is left in the mailboxes is never read
+    with pytest.raises(cbrkc.CbError, match="in vain"):
+        p.run(1, 0.5, 0)
+    assert time.monotonic() - t0 < 10.0

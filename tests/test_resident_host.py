@@ -7,6 +7,7 @@ import ctypes
 import os
 import shutil
 import subprocess
+import time
 
 import numpy as np
 import pytest
@@ -25,7 +26,7 @@ def emu(tmp_path_factory):
     return ctypes.CDLL(str(out / "libresident.so"))
 
 
-def run(emu, o, n, cpb=1, nsteps=1, nhelp=0, present=1 << 20, floor=0.0, refresh=False):
+def run(emu, o, n, cpb=1, nsteps=1, nhelp=0, present=1 << 20, floor=0.0, refresh=False, wait=60.0):
     """nsteps macro steps of the oracle population o, as n cells, on the host
     build, from o's present state, with this floor of the spectral radius and
     refresh of fn after ion updates; o itself stays"""
@@ -41,7 +42,8 @@ def run(emu, o, n, cpb=1, nsteps=1, nhelp=0, present=1 << 20, floor=0.0, refresh
     launches = ctypes.c_int()
     p = lambda a: a.ctypes.data_as(ctypes.c_void_p)  # noqa: E731
     status = emu.emu_rkc(n, comp, cpb, nhelp, present, p(row), p(col), p(keep[0]), p(keep[1]), p(keep[2]), p(vec), p(c),
-                         p(hw), p(cnt), nsteps, ctypes.c_double(floor), 1 if refresh else 0, ctypes.byref(launches))
+                         p(hw), p(cnt), nsteps, ctypes.c_double(floor), 1 if refresh else 0, ctypes.c_double(wait),
+                         ctypes.byref(launches))
     return dict(status=status, vec=vec, ctl=c[:14], hw=hw, cnt=cnt, launches=launches.value)
 
 
@@ -79,6 +81,21 @@ def test_macro_steps(emu, n, comp, cpb, nhelp):
 def test_coupled_workgroups(emu):
     o = cables(2, 30, 5.0, pairs=[(3, 41), (29, 30), (3, 55)])
     check(o, run(emu, o, 2, nsteps=2), 2)
+
+
+@pytest.mark.parametrize("n,comp,nhelp,pairs", [(2, 30, 0, ()), (2, 30, 0, [(3, 41), (29, 30)]), (3, 30, 0, [(29, 30), (59, 60)]),
+                                                (1, 150, 2, ())])
+def test_a_lost_workgroup_ends_the_launch(emu, n, comp, nhelp, pairs):
+    # Only the first workgroup runs (or, of three, the first two): it gives up
+    # once, not at every one of a step's 140 exchanges, and says so
+    o = cables(n, comp, 0.5, pairs=pairs, spread=1e-3)
+    t0 = time.monotonic()
+    r = run(emu, o, n, nhelp=nhelp, present=max(1, n - 1), floor=2e5, wait=0.5, nsteps=2)
+    assert r["status"] == 8
+    assert time.monotonic() - t0 < 4.0
+    # no waiting at all: the first look that finds nothing
+    assert run(emu, o, n, nhelp=nhelp, present=max(1, n - 1), floor=2e5, wait=0.0,
+               nsteps=2)["status"] == 8
 
 
 @pytest.mark.parametrize("pairs,refresh", [((), False), ([(3, 41), (29, 30)], True)])
