@@ -344,6 +344,7 @@ class GlobalRkc : public Engine {
     if (rec_) (void)hipFree(rec_);
     if (bits_) (void)hipFree(bits_);
     if (ctl_host_) (void)hipHostFree(ctl_host_);
+    if (late_host_) (void)hipHostFree(late_host_);
     for (void *p : {(void *)v_, (void *)iext_, (void *)cm_, (void *)b_, (void *)dammy_, (void *)row_, (void *)col_,
                     (void *)val_, (void *)red_a_, (void *)red_b_, (void *)bad_, (void *)amp_, (void *)syn_g_,
                     (void *)zero_, (void *)net_s_})
@@ -400,6 +401,7 @@ class GlobalRkc : public Engine {
 
   void advance() override {
     started_ = true;
+    check_failed();
     if (resident_) {
       if (net_.on() && net_s_) syn_macro_current(net_, vec_[Y], net_s_, nc_, st_);
       for (const long m0 = macro_; macro_ == m0; check_steps()) res_launch(A_, 1, 0.0, (int)macro_);
@@ -462,6 +464,7 @@ class GlobalRkc : public Engine {
       CB_HIP(hipMemsetAsync(bits_, 0, sizeof(uint32_t) * (size_t)nsteps * words, st_));
     }
     started_ = true;
+    check_failed();
     const long m0 = macro_;
     while (macro_ < m0 + nsteps) {
       const int k = (int)(macro_ - m0);
@@ -497,6 +500,7 @@ class GlobalRkc : public Engine {
   hipStream_t stream() const override { return st_; }
 
   void read(int field, double *dst) override {
+    check_failed();
     const double *src = nullptr;
     switch (field) {
       case F_VNEW: src = vec_[VNEW]; break;
@@ -580,6 +584,13 @@ class GlobalRkc : public Engine {
       CB_HIP(hipLaunchCooperativeKernel(res_fn_, dim3(res_grid_), dim3(res_threads()), args, (unsigned)res_lds_, st_));
   }
 
+  // A launch whose workgroups lost one another leaves them at different steps and
+  // values in the mailboxes that the next launch would take for its own: the
+  // population is of no use from then on, its voltages included
+  void check_failed() const {
+    if (failed_) throw Error("RKC: a workgroup of the step kernel waited for another one in vain", -3);
+  }
+
   // waits for the launch, takes the kernel's question if it stopped for one
   // (the next launch brings the answer); a failed step ends the run as on the
   // other path
@@ -587,6 +598,9 @@ class GlobalRkc : public Engine {
     CB_HIP(hipGetLastError());
     CB_HIP(hipStreamSynchronize(st_));
     const RkcCtl &c = *ctl_host_;
+    // (any of the workgroups may have given up, the others having ended well)
+    failed_ = *(volatile int *)late_host_ != 0;
+    check_failed();
     macro_ = c.macro;
     A_.resume = c.status == ASK_POW || c.status == ASK_STAGE ? c.status : 0;
     if (c.status == ASK_POW) {
@@ -597,7 +611,6 @@ class GlobalRkc : public Engine {
     if (c.status == 0 || A_.resume) return;
     if (c.status == NONFINITE)
       throw Error("RKC: non-finite state (error estimate " + std::to_string(c.err) + ")", NONFINITE);
-    if (c.status == TIMED_OUT) throw Error("RKC: a workgroup of the step kernel waited for another one in vain", -3);
     throw Error("RKC failed: idid = " + std::to_string(c.status), c.status);
   }
 
@@ -774,6 +787,9 @@ class GlobalRkc : public Engine {
     *ctl_host_ = c;
     CB_HIP(hipHostGetDevicePointer((void **)&a.ctl_host, ctl_host_, 0));
     a.wait = WAIT_TICKS;
+    CB_HIP(hipHostMalloc((void **)&late_host_, sizeof(int), hipHostMallocMapped | hipHostMallocCoherent));
+    *late_host_ = 0;
+    CB_HIP(hipHostGetDevicePointer((void **)&a.late, late_host_, 0));
     a.integ = integ_;
     a.rho_floor = rho_floor_;
     a.strict = res_strict();
@@ -1111,6 +1127,8 @@ class GlobalRkc : public Engine {
   bool started_ = false;                       // a macro step has been asked for
   RkcArgs A_{};
   RkcCtl *ctl_host_ = nullptr;   // written by the kernel as it ends
+  int *late_host_ = nullptr;     // set by the kernel: a wait gave up
+  bool failed_ = false;
   const void *res_fn_ = nullptr;
   void *state_dev_ = nullptr;    // the model's state struct, and what is in it
   std::vector<char> state_host_;

@@ -70,6 +70,7 @@ struct RkcArgs {
   const int *x0;                         // first further entry of each workgroup (nblk + 1)
   const int *imp0, *exp0, *exp_row, *exp_slot;   // ghosts fetched, rows posted (null: uncoupled cells)
   unsigned long long wait;               // the limit of a wait (grid_mail.hpp)
+  int *late;                             // mapped host memory: set by whichever workgroup or helper gave up
   double *ghost;                         // [3][GHOST_STAGES][nslot]
   int nslot;
   double *terms, *parts;                 // grid_sum's mailboxes
@@ -209,7 +210,10 @@ __device__ inline void rkc_helper(const RkcArgs &A, const typename Model::State 
       }
       mail_clear(A.bout + old + row);
     }
-    if (late || !(dt >= 0.0)) return;
+    if (late || !(dt >= 0.0)) {
+      if (late && tid == 0) *A.late = 1;
+      return;
+    }
   }
 }
 
@@ -729,7 +733,8 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, const typena
       A.v2[r0 + i] = V2[i];
     }
   });
-  if ((w == 0 || status == TIMED_OUT) && tid == 0) {
+  if (tid == 0 && s_late) *A.late = 1;
+  if (w == 0 && tid == 0) {
     RkcCtl c = *ctl;
     c.o[1] = absh; c.o[2] = sprad; c.o[3] = naccpt; c.o[6] = idid; c.o[7] = gt;
     c.o[8] = gt_old; c.o[9] = lt; c.o[10] = tend; c.o[11] = errold; c.o[12] = hold;

@@ -199,6 +199,8 @@ int emu_rkc(int n, int comp, int cpb, int nhelp, int present, const int *row, co
   a.start = start.data();
   a.integ = 1e30;
   a.wait = wait_ticks(wait);
+  int late = 0;
+  a.late = &late;
   a.rho_floor = rho_floor;
   a.refresh_fn = refresh;
   a.iext = iext.data();
@@ -245,6 +247,7 @@ int emu_rkc(int n, int comp, int cpb, int nhelp, int present, const int *row, co
     a.p1 = std::pow(host.err, 1.0 / 3.0);
     a.p2 = std::pow(host.err, 2.0 / 3.0);
     if (host.status == ASK_STAGE) rkc_stage_start(host.m, &a.asked.x, &a.asked.y);
+    if (late) return TIMED_OUT;
     if (host.status != 0 && !a.resume) break;
   }
   std::memcpy(o16, host.o, sizeof(host.o));

@@ -15,6 +15,7 @@
   all (cb_pop_wait_limit) the first empty mailbox ends the launch, and the call
   fails at once; solves already queued fall through.
 """
+import os
 import time
 
 import numpy as np
@@ -79,4 +80,22 @@ def test_a_solve_that_waits_in_vain_fails_the_run(tmp_path, solver):
     p.wait_limit(60.0)   # what is left in the mailboxes is never read
     with pytest.raises(cbrkc.CbError, match="in vain"):
         p.run(1, 0.5, 0)
+    assert time.monotonic() - t0 < 10.0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cell,nx,ny,f,v", [("IO", 13, 40, "IO.txt", -60.0), ("GO", 3, 2, "Go_131.txt", -60.0),
+                                            ("PKJ", 3, 1, "Pkj.txt", -68.0), ("GR", 1, 1, "Gr.txt", -70.0)])
+def test_a_step_that_waits_in_vain_fails_the_population(ref_data, cell, nx, ny, f, v):
+    # several workgroups, gap currents, gap junctions, and a single cell's helpers
+    print(f"{nx * ny} {cell} cells, no time to wait", flush=True)
+    p = cbrkc.Population(getattr(cbrkc, cell), nx, ny, morph=os.path.join(ref_data, f), v0=np.full(nx * ny, v))
+    p.wait_limit(0.0)
+    t0 = time.monotonic()
+    with pytest.raises(cbrkc.CbError, match="in vain"):
+        p.run(4, 0.0, 0)
+    p.wait_limit(60.0)
+    for call in (lambda: p.run(1, 0.5, 0), p.advance, p.read):
+        with pytest.raises(cbrkc.CbError, match="in vain"):
+            call()
     assert time.monotonic() - t0 < 10.0

@@ -92,7 +92,7 @@ def test_a_lost_workgroup_ends_the_launch(emu, n, comp, nhelp, pairs):
     t0 = time.monotonic()
     r = run(emu, o, n, nhelp=nhelp, present=max(1, n - 1), floor=2e5, wait=0.5, nsteps=2)
     assert r["status"] == 8
-    assert time.monotonic() - t0 < 4.0
+    assert time.monotonic() - t0 < 30.0   # 140 limits would be 70 s
     # no waiting at all: the first look that finds nothing
     assert run(emu, o, n, nhelp=nhelp, present=max(1, n - 1), floor=2e5, wait=0.0,
                nsteps=2)["status"] == 8
