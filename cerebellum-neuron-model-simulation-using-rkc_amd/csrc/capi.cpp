@@ -349,6 +349,7 @@ void syn_step(cb_syn *s, double t) {
   const double *pv = nullptr;
   if (s->pre) {
     s->pre->eng->sync();
+    s->pre->eng->check();
     pv = s->pre->eng->device_v();
     if (!pv) throw Error("the presynaptic population's engine exposes no voltage");
   }

@@ -76,6 +76,9 @@ class Engine {
   virtual int ncell() const = 0;
   virtual void controller(double *others14, double *hwork8) const { (void)others14; (void)hwork8; }
   virtual void sync() {}
+  // throws where an earlier step (finished: sync first) left the population
+  // without valid voltages
+  virtual void check() const {}
   // picks the launch mapping by timing short trials from the current state
   // (the state is left unchanged); returns the chosen threads per cell
   virtual int autotune(int trial_steps, double t0) {

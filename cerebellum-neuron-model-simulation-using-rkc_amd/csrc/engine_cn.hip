@@ -1150,6 +1150,9 @@ class CnEngine : public Engine {
   int nc() const override { return nc_; }
   int ncell() const override { return n_; }
   void sync() override { CB_HIP(hipStreamSynchronize(st_)); }
+  void check() const override {
+    if (late_host_ && *(volatile int *)late_host_) throw Error("CN / BE: a workgroup of the solve waited for another one in vain", -3);
+  }
   Stats stats() const override {
     Stats s = st;
     int f[F_NFLAG];
@@ -1235,6 +1238,15 @@ class CnEngine : public Engine {
 
   // one CN (BE) step of CN_DT (BE_DT): xx_solve_update_v with that solver
   void advance() override {
+    check();
+    step();
+    if (resident_ && res_grid_ > 1) {   // (the cooperative launch has waited for the solve already)
+      sync();
+      check();
+    }
+  }
+  // the step queued, whose solve may yet fail (check)
+  void step() {
     prep();
     if (direct_) {
       tree_solve(chain_, S_.diag, S_.b, S_.v);
@@ -1259,6 +1271,7 @@ class CnEngine : public Engine {
   // l_dt < H_MAX); records compartment rec_comp of every cell after it
   void run(int nsteps, double t0, int rec_comp, double *rec_out) override {
     if (nsteps <= 0) return;
+    check();
     const int per = rec_comp >= 0 ? 1 : comp_;
     const int words = (n_ + 31) / 32;
     const bool raster = raster_comp_ >= 0;
@@ -1275,13 +1288,13 @@ class CnEngine : public Engine {
         // a set step: exactly H_MAX / dt steps, at whole multiples of dt
         for (int j = 0; j < nsub_; j++) {
           set_current(t + j * dt_);
-          advance();
+          step();
         }
       } else {
         double l_dt = 0.0;
         while (l_dt < H_MAX) {
           set_current(t + l_dt);
-          advance();
+          step();
           l_dt += dt_;
         }
       }
@@ -1295,7 +1308,7 @@ class CnEngine : public Engine {
       CB_HIP(hipMemcpyAsync(rec_out, drec, sizeof(double) * (size_t)nsteps * n_ * per, hipMemcpyDeviceToHost, st_));
     if (dbits) CB_HIP(hipMemcpyAsync(bits.data(), dbits, sizeof(uint32_t) * bits.size(), hipMemcpyDeviceToHost, st_));
     CB_HIP(hipStreamSynchronize(st_));
-    check_late();
+    check();
     if (rec_cap_ > REC_KEPT) {   // a large recording's buffer is given back
       (void)hipFree(rec_);
       rec_ = nullptr;
@@ -1325,7 +1338,7 @@ class CnEngine : public Engine {
     }
     if (!src) throw Error("field not available for this population");
     CB_HIP(hipStreamSynchronize(st_));
-    check_late();
+    check();
     CB_HIP(hipMemcpy(dst, src, sizeof(double) * nc_, hipMemcpyDeviceToHost));
   }
 
@@ -1339,10 +1352,6 @@ class CnEngine : public Engine {
     p = dal<T>(n);
     cap = n;
   }
-  void check_late() const {
-    if (late_host_ && *(volatile int *)late_host_) throw Error("CN / BE: a workgroup of the solve waited for another one in vain", -3);
-  }
-
   template <typename T>
   T *res_put(const std::vector<T> &h) {
     T *d = dup(h);

@@ -386,6 +386,12 @@ class GlobalRkc : public Engine {
            (A_.nhelp ? ", " + std::to_string(A_.nhelp) + " helpers each for the ion updates" : "") + (A_.imp0 ? ", gap-junction values exchanged per stage" : "");
   }
   void sync() override { CB_HIP(hipStreamSynchronize(st_)); }
+  // A launch whose workgroups lost one another leaves them at different steps and
+  // values in the mailboxes that the next launch would take for its own: the
+  // population is of no use from then on, its voltages included
+  void check() const override {
+    if (failed_) throw Error("RKC: a workgroup of the step kernel waited for another one in vain", -3);
+  }
   // the two paths keep the controller in different places, so the choice is
   // made before the first macro step
   bool use_launches(bool on) override {
@@ -401,7 +407,7 @@ class GlobalRkc : public Engine {
 
   void advance() override {
     started_ = true;
-    check_failed();
+    check();
     if (resident_) {
       if (net_.on() && net_s_) syn_macro_current(net_, vec_[Y], net_s_, nc_, st_);
       for (const long m0 = macro_; macro_ == m0; check_steps()) res_launch(A_, 1, 0.0, (int)macro_);
@@ -464,7 +470,7 @@ class GlobalRkc : public Engine {
       CB_HIP(hipMemsetAsync(bits_, 0, sizeof(uint32_t) * (size_t)nsteps * words, st_));
     }
     started_ = true;
-    check_failed();
+    check();
     const long m0 = macro_;
     while (macro_ < m0 + nsteps) {
       const int k = (int)(macro_ - m0);
@@ -500,7 +506,7 @@ class GlobalRkc : public Engine {
   hipStream_t stream() const override { return st_; }
 
   void read(int field, double *dst) override {
-    check_failed();
+    check();
     const double *src = nullptr;
     switch (field) {
       case F_VNEW: src = vec_[VNEW]; break;
@@ -584,13 +590,6 @@ class GlobalRkc : public Engine {
       CB_HIP(hipLaunchCooperativeKernel(res_fn_, dim3(res_grid_), dim3(res_threads()), args, (unsigned)res_lds_, st_));
   }
 
-  // A launch whose workgroups lost one another leaves them at different steps and
-  // values in the mailboxes that the next launch would take for its own: the
-  // population is of no use from then on, its voltages included
-  void check_failed() const {
-    if (failed_) throw Error("RKC: a workgroup of the step kernel waited for another one in vain", -3);
-  }
-
   // waits for the launch, takes the kernel's question if it stopped for one
   // (the next launch brings the answer); a failed step ends the run as on the
   // other path
@@ -600,7 +599,7 @@ class GlobalRkc : public Engine {
     const RkcCtl &c = *ctl_host_;
     // (any of the workgroups may have given up, the others having ended well)
     failed_ = *(volatile int *)late_host_ != 0;
-    check_failed();
+    check();
     macro_ = c.macro;
     A_.resume = c.status == ASK_POW || c.status == ASK_STAGE ? c.status : 0;
     if (c.status == ASK_POW) {

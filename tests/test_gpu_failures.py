@@ -80,6 +80,14 @@ def test_a_solve_that_waits_in_vain_fails_the_run(tmp_path, solver):
     p.wait_limit(60.0)   # what is left in the mailboxes is never read
     with pytest.raises(cbrkc.CbError, match="in vain"):
         p.run(1, 0.5, 0)
+    with pytest.raises(cbrkc.CbError, match="in vain"):
+        p.read()
+    q = cbrkc.Population(cbrkc.PKJ, 4, 1, solver=solver, morph=morph, v0=[-68.0, -67.0, -66.0, -67.5])
+    q.wait_limit(0.0)
+    q.set_current(0.0)
+    for _ in range(2):   # the step itself, and every one after it
+        with pytest.raises(cbrkc.CbError, match="in vain"):
+            q.advance()
     assert time.monotonic() - t0 < 10.0
 
 
