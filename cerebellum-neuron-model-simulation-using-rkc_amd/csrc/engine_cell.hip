@@ -1439,8 +1439,6 @@ class CellPkj : public Engine {
   }
 
   bool select_mapping(int threads) override {
-    // (the FP64 engine takes its 512 threads by itself; asked for, they stay refused)
-    if (sizeof(T) == 8 && threads == 512) return false;
     for (size_t v = 0; v < variants_.size(); v++)
       if (variants_[v].nt == threads && (long)variants_[v].nt * variants_[v].k >= C_) {
         cur_ = (int)v;

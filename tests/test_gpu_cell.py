@@ -96,3 +96,19 @@ def test_single_macro_steps_equal_one_long_launch(synth_dir):
         rows.append(p2.read(cbrkc.F_VNEW)[1599::1600])
     assert np.array_equal(np.array(rows), tr)
     assert np.array_equal(p1.read(cbrkc.F_VNEW), p2.read(cbrkc.F_VNEW))
+
+
+@pytest.mark.parametrize("engine", [cbrkc.ENGINE_CELL_FP64, cbrkc.ENGINE_CELL_MIXED], ids=["fp64", "mixed"])
+def test_every_mapping_can_be_asked_for(synth_dir, engine):
+    # the default's 512 threads too, after another choice
+    print(f"mappings of engine {engine}, 2 cells, 4 macro steps", flush=True)
+    morph = str(synth_dir / "pkjm2.txt")
+    cbrkc.synth_pkj_morph(morph, seed=23, ncell=2)
+    p = [cbrkc.Population(cbrkc.PKJ, 2, 1, morph=morph, v0=[-68.0, -67.0], stim=(1599, 0.0, 1e9, 1e-3), engine=engine,
+                          **STABLE) for _ in range(2)]
+    for threads in (256, 320, 512):
+        p[1].autotune(0, threads=threads)
+    assert p[0].mapping() == p[1].mapping()
+    assert np.array_equal(p[0].run(4, 0.0, 1599), p[1].run(4, 0.0, 1599))
+    with pytest.raises(cbrkc.CbError):
+        p[1].autotune(0, threads=128)
