@@ -45,6 +45,7 @@
 #include "engine.hpp"
 #include "kry_resident.hpp"
 #include "record.hpp"
+#include "table_pack.hpp"
 #include "go_model.hpp"
 #include "gr_model.hpp"
 #include "io_model.hpp"
@@ -1131,7 +1132,7 @@ class CnEngine : public Engine {
   }
   ~CnEngine() override {
     (void)hipStreamSynchronize(st_);
-    for (void *p : res_bufs_) (void)hipFree(p);
+    if (res_buf_) (void)hipFree(res_buf_);
     if (late_host_) (void)hipHostFree(late_host_);
     for (const void *p : {(const void *)S_.row, (const void *)S_.col, (const void *)S_.dpos, (const void *)S_.val,
                           (const void *)S_.trow, (const void *)S_.tcol, (const void *)S_.tsrc, (const void *)S_.cm,
@@ -1352,13 +1353,6 @@ class CnEngine : public Engine {
     p = dal<T>(n);
     cap = n;
   }
-  template <typename T>
-  T *res_put(const std::vector<T> &h) {
-    T *d = dup(h);
-    res_bufs_.push_back((void *)d);
-    return d;
-  }
-
   // The resident kernel's shape and tables.  One workgroup of 1024 threads when
   // the rows fit it and its LDS (no exchange between workgroups), else
   // workgroups of 512 threads with as few rows per thread as leave at most one
@@ -1394,16 +1388,27 @@ class CnEngine : public Engine {
   bool plan_resident(const std::vector<int> &row, const std::vector<int> &col, const std::vector<double> &val,
                      const std::vector<int> &dpos, const std::vector<int> &trow, const std::vector<int> &tcol,
                      const std::vector<int> &tsrc, bool bicg, int nt, int k, int rb, int grid, size_t lds_max) {
+    // the LDS that the matrix alone needs, before anything is laid out
+    const size_t m = bicg ? 2 : 1;
     KryArgs a{};
     a.nc = nc_;
     a.nch = (nc_ + NB - 1) / NB;
     a.rb = rb;
-    std::vector<unsigned short> lrow, lcol, ldpos(nc_), tr, tc, tdpos(nc_);
-    std::vector<double> lval, tv;
+    for (int w = 0; w < grid; w++)
+      a.nnz_max = std::max(a.nnz_max, row[std::min(nc_, (w + 1) * rb)] - row[w * rb]);
+    auto lds_bytes = [&]() {
+      const size_t b = sizeof(double) * (m * (rb + a.ghost_max) + rb + a.nch + 8 + m * a.nnz_max) +
+                       sizeof(unsigned short) * m * (rb + 1 + a.nnz_max);
+      return (b + 15) & ~(size_t)15;
+    };
+    if (a.nnz_max > 65535 || lds_bytes() > lds_max) return false;
+    const size_t nnz = col.size(), nrow = (size_t)grid * (rb + 1);
+    std::vector<unsigned short> lrow(nrow), lcol(nnz), ldpos(nc_), tc(bicg ? nnz : 0), tdpos(bicg ? nc_ : 0);
+    std::vector<double> tv(bicg ? nnz : 0);
     std::vector<int> lnz0(1, 0), imp0(1, 0), imp;
     std::vector<int> at(nc_, -1);   // ghost index of a row in the present workgroup
     for (int w = 0; w < grid; w++) {
-      const int r0 = w * rb, r1 = std::min(nc_, r0 + rb), z0 = lnz0[w];
+      const int r0 = w * rb, r1 = std::min(nc_, r0 + rb), z0 = row[r0];
       const size_t m0 = imp.size();
       auto local = [&](int c) {
         if (c >= r0 && c < r1) return c - r0;
@@ -1413,44 +1418,35 @@ class CnEngine : public Engine {
         }
         return rb + at[c];
       };
-      for (int i = r0; i < r0 + rb; i++) {   // (rows past the last one are empty)
-        lrow.push_back((unsigned short)((int)lval.size() - z0));
-        tr.push_back(lrow.back());
+      unsigned short *lr = &lrow[(size_t)w * (rb + 1)];
+      for (int i = r0; i <= r0 + rb; i++) {   // (rows past the last one are empty)
+        lr[i - r0] = (unsigned short)(row[std::min(i, r1)] - z0);
         if (i >= r1) continue;
-        // the sparsity is symmetric, so a row of the transpose has the row's columns
-        if (trow[i + 1] - trow[i] != row[i + 1] - row[i]) return false;
-        for (int e = 0; e < row[i + 1] - row[i]; e++) {
-          const int j = row[i] + e, t = trow[i] + e;
-          if (j == dpos[i]) ldpos[i] = (unsigned short)((int)lval.size() - z0);
-          if (tcol[t] == i) tdpos[i] = (unsigned short)((int)lval.size() - z0);
-          const int lc = local(col[j]), lt = local(tcol[t]);
-          if (lc > 65535 || lt > 65535) return false;
-          lcol.push_back((unsigned short)lc);
-          lval.push_back(val[j]);
-          tc.push_back((unsigned short)lt);
-          tv.push_back(val[tsrc[t]]);
+        for (int j = row[i]; j < row[i + 1]; j++) lcol[j] = (unsigned short)local(col[j]);
+        ldpos[i] = (unsigned short)(dpos[i] - z0);
+        if (!bicg) continue;
+        // the sparsity is symmetric, so a row of the transpose has the row's columns and place
+        if (trow[i] != row[i] || trow[i + 1] != row[i + 1]) return false;
+        for (int t = trow[i]; t < trow[i + 1]; t++) {
+          if (tcol[t] == i) tdpos[i] = (unsigned short)(t - z0);
+          tc[t] = (unsigned short)local(tcol[t]);
+          tv[t] = val[tsrc[t]];
         }
       }
-      const int nz = (int)lval.size() - z0;
-      if (nz > 65535) return false;
-      lrow.push_back((unsigned short)nz);
-      tr.push_back((unsigned short)nz);
-      lnz0.push_back((int)lval.size());
+      if (rb + (int)(imp.size() - m0) > 65536) return false;
+      lnz0.push_back(row[r1]);
       for (size_t g = m0; g < imp.size(); g++) at[imp[g]] = -1;
       imp0.push_back((int)imp.size());
-      a.nnz_max = std::max(a.nnz_max, nz);
       a.ghost_max = std::max(a.ghost_max, (int)(imp.size() - m0));
     }
-    const size_t m = bicg ? 2 : 1;
-    size_t lds = sizeof(double) * (m * (rb + a.ghost_max) + rb + a.nch + 8 + m * a.nnz_max) +
-                 sizeof(unsigned short) * m * (rb + 1 + a.nnz_max);
-    lds = (lds + 15) & ~(size_t)15;
+    const size_t lds = lds_bytes();
     if (lds > lds_max) return false;
     const void *fn = kry_kernel(nt, k, bicg);
     CB_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     int fit = 0;
     CB_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, fn, nt, lds));
     if (fit < 1 || (grid > 1 && !coop_available(st_))) return false;
+    TablePack T;
     a.nslot = (int)imp.size();
     if (a.nslot > 0) {
       std::vector<std::vector<std::pair<int, int>>> out(grid);   // (thread, row and slot) of each workgroup
@@ -1468,31 +1464,32 @@ class CnEngine : public Engine {
         }
         exp0.push_back((int)er.size());
       }
-      a.imp0 = res_put(imp0);
-      a.imp = res_put(imp);
-      a.exp0 = res_put(exp0);
-      a.exp_t0 = res_put(et);
-      a.exp_row = res_put(er);
-      a.exp_slot = res_put(es);
+      T.put(a.imp0, std::move(imp0));
+      T.put(a.imp, std::move(imp));
+      T.put(a.exp0, std::move(exp0));
+      T.put(a.exp_t0, std::move(et));
+      T.put(a.exp_row, std::move(er));
+      T.put(a.exp_slot, std::move(es));
     }
     unsigned long long e = MAIL_EMPTY;
     double empty;
     std::memcpy(&empty, &e, sizeof(empty));
-    a.ghost = res_put(std::vector<double>((size_t)6 * std::max(1, a.nslot), empty));
-    a.parts = res_put(std::vector<double>((size_t)3 * a.nch, empty));
-    a.q = res_put(std::vector<unsigned>(2, 0u));
+    T.put(a.ghost, std::vector<double>((size_t)6 * std::max(1, a.nslot), empty));
+    T.put(a.parts, std::vector<double>((size_t)3 * a.nch, empty));
+    T.put(a.q, std::vector<unsigned>(2, 0u));
     a.wait = WAIT_TICKS;
-    a.lrow = res_put(lrow);
-    a.lcol = res_put(lcol);
-    a.ldpos = res_put(ldpos);
-    a.lval = res_put(lval);
-    a.lnz0 = res_put(lnz0);
+    T.put(a.lrow, std::move(lrow));
+    T.put(a.lcol, std::move(lcol));
+    T.put(a.ldpos, std::move(ldpos));
+    a.lval = S_.val;   // the entries keep their order
+    T.put(a.lnz0, std::move(lnz0));
     if (bicg) {
-      a.trow = res_put(tr);
-      a.tcol = res_put(tc);
-      a.tdpos = res_put(tdpos);
-      a.tval = res_put(tv);
+      T.put(a.tcol, std::move(tc));
+      T.put(a.tdpos, std::move(tdpos));
+      T.put(a.tval, std::move(tv));
     }
+    res_buf_ = T.upload();
+    a.trow = a.lrow;
     CB_HIP(hipHostMalloc((void **)&late_host_, sizeof(int), hipHostMallocMapped | hipHostMallocCoherent));
     *late_host_ = 0;
     CB_HIP(hipHostGetDevicePointer((void **)&a.late, late_host_, 0));
@@ -1546,7 +1543,7 @@ class CnEngine : public Engine {
   KryArgs A_{};
   size_t res_lds_ = 0;
   int res_grid_ = 0, res_nt_ = 0;
-  std::vector<void *> res_bufs_;
+  void *res_buf_ = nullptr;
   int *late_host_ = nullptr;
   static constexpr size_t REC_KEPT = (size_t)8 << 20;   // doubles of recording kept for the next run
   int stim_on_ = -1;             // the window's state in iext (-1: not set yet)

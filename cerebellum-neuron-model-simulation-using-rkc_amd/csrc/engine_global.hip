@@ -40,6 +40,7 @@
 #include "pkj_model.hpp"
 #include "record.hpp"
 #include "rkc_models.hpp"
+#include "table_pack.hpp"
 
 namespace cbrkc {
 
@@ -340,11 +341,11 @@ class GlobalRkc : public Engine {
 
   ~GlobalRkc() override {
     (void)hipStreamSynchronize(st_);
-    for (void *p : res_bufs_) (void)hipFree(p);
+    if (res_buf_) (void)hipFree(res_buf_);
+    if (state_dev_) (void)hipFree(state_dev_);
     if (rec_) (void)hipFree(rec_);
     if (bits_) (void)hipFree(bits_);
     if (ctl_host_) (void)hipHostFree(ctl_host_);
-    if (late_host_) (void)hipHostFree(late_host_);
     for (void *p : {(void *)v_, (void *)iext_, (void *)cm_, (void *)b_, (void *)dammy_, (void *)row_, (void *)col_,
                     (void *)val_, (void *)red_a_, (void *)red_b_, (void *)bad_, (void *)amp_, (void *)syn_g_,
                     (void *)zero_, (void *)net_s_})
@@ -574,7 +575,6 @@ class GlobalRkc : public Engine {
     // when synapses are attached
     if (!state_dev_) {
       CB_HIP(hipMalloc(&state_dev_, sizeof(State)));
-      res_bufs_.push_back(state_dev_);
     }
     if (state_host_.size() != sizeof(State) || std::memcmp(state_host_.data(), &S, sizeof(State)) != 0) {
       state_host_.assign((const char *)&S, (const char *)&S + sizeof(State));
@@ -621,14 +621,6 @@ class GlobalRkc : public Engine {
     cap = 0;
     p = dalloc<T>(n);
     cap = n;
-  }
-
-  template <typename T>
-  T *res_put(const std::vector<T> &h) {
-    T *d = dalloc<T>(h.size());
-    res_bufs_.push_back((void *)d);
-    h2d(d, h);
-    return d;
   }
 
   // Decides whether the population runs on the resident kernel and lays out
@@ -716,6 +708,7 @@ class GlobalRkc : public Engine {
       a.own = ((RM + a.nhelp) / (a.nhelp + 1) + 63) / 64 * 64;
     }
     res_grid_ = a.nblk * (1 + a.nhelp);
+    TablePack T;
     const int nslot = (int)imp.size();
     if (nslot > 0) {
       if ((size_t)nslot * 3 * GHOST_STAGES * sizeof(double) > (size_t)1 << 30) return;
@@ -729,27 +722,27 @@ class GlobalRkc : public Engine {
         }
         exp0.push_back((int)er.size());
       }
-      a.imp0 = res_put(imp0);
-      a.exp0 = res_put(exp0);
-      a.exp_row = res_put(er);
-      a.exp_slot = res_put(es);
-      a.ghost = empty_mail((size_t)3 * GHOST_STAGES * nslot);
+      T.put(a.imp0, std::move(imp0));
+      T.put(a.exp0, std::move(exp0));
+      T.put(a.exp_row, std::move(er));
+      T.put(a.exp_slot, std::move(es));
+      T.space(a.ghost, (size_t)3 * GHOST_STAGES * nslot);
       a.nslot = nslot;
     }
-    a.lcol = res_put(lcol);
-    a.lval = res_put(lval);
-    a.xcol = res_put(xcol);
-    a.xval = res_put(xval);
-    a.x0 = res_put(x0);
+    T.put(a.lcol, std::move(lcol));
+    T.put(a.lval, std::move(lval));
+    T.put(a.xcol, std::move(xcol));
+    T.put(a.xval, std::move(xval));
+    T.put(a.x0, std::move(x0));
     if (a.nblk > 1) {
-      a.terms = empty_mail((size_t)3 * nc_);
-      a.parts = empty_mail((size_t)3 * a.nch);
-      a.gap = empty_mail((size_t)3 * n_);
+      T.space(a.terms, (size_t)3 * nc_);
+      T.space(a.parts, (size_t)3 * a.nch);
+      T.space(a.gap, (size_t)3 * n_);
     }
     if (a.nhelp > 0) {
-      a.req = empty_mail((size_t)6 * a.nblk);
-      a.vin = empty_mail((size_t)3 * nc_);
-      a.bout = empty_mail((size_t)3 * nc_);
+      T.space(a.req, (size_t)6 * a.nblk);
+      T.space(a.vin, (size_t)3 * nc_);
+      T.space(a.bout, (size_t)3 * nc_);
     }
     a.y = vec_[Y];
     a.yn = vec_[YN];
@@ -761,13 +754,13 @@ class GlobalRkc : public Engine {
     a.v2 = vec_[VT2];
     a.cm = cm_;
     static const std::vector<double> stage_table = rkc_stage_table(RES_COEF);   // the same for every population
-    a.coef = res_put(stage_table);
+    T.put_static(a.coef, stage_table);
     static const std::vector<double2> start_table = [] {
       std::vector<double2> t(RES_START + 1);
       for (int m = 0; m <= RES_START; m++) rkc_stage_start(m, &t[m].x, &t[m].y);
       return t;
     }();
-    a.start = res_put(start_table);
+    T.put_static(a.start, start_table);
     RkcCtl c{};
     std::memcpy(c.o, o_, sizeof(o_));
     std::memcpy(c.hw, hw_, sizeof(hw_));
@@ -781,14 +774,20 @@ class GlobalRkc : public Engine {
     c.last = last_;
     c.newspc = newspc_;
     c.jacatt = jacatt_;
-    a.ctl = res_put(std::vector<RkcCtl>(1, c));
-    CB_HIP(hipHostMalloc((void **)&ctl_host_, sizeof(RkcCtl), hipHostMallocMapped | hipHostMallocCoherent));
+    T.put(a.ctl, std::vector<RkcCtl>(1, c));
+    double *mail = nullptr;
+    res_buf_ = T.upload(&mail);
+    if (T.spaces() > 0) {
+      k_empty_mail<<<(unsigned)((T.spaces() + 255) / 256), 256, 0, st_>>>((unsigned long long *)mail, T.spaces());
+      CB_HIP(hipGetLastError());
+    }
+    CB_HIP(hipHostMalloc((void **)&ctl_host_, sizeof(RkcCtl) + sizeof(int), hipHostMallocMapped | hipHostMallocCoherent));
     *ctl_host_ = c;
     CB_HIP(hipHostGetDevicePointer((void **)&a.ctl_host, ctl_host_, 0));
     a.wait = WAIT_TICKS;
-    CB_HIP(hipHostMalloc((void **)&late_host_, sizeof(int), hipHostMallocMapped | hipHostMallocCoherent));
+    late_host_ = (int *)(ctl_host_ + 1);
     *late_host_ = 0;
-    CB_HIP(hipHostGetDevicePointer((void **)&a.late, late_host_, 0));
+    a.late = (int *)(a.ctl_host + 1);
     a.integ = integ_;
     a.rho_floor = rho_floor_;
     a.strict = res_strict();
@@ -809,14 +808,6 @@ class GlobalRkc : public Engine {
     A_ = a;
     CB_HIP(hipStreamSynchronize(st_));
     laid_out_ = resident_ = true;
-  }
-
-  double *empty_mail(size_t n) {
-    double *d = dalloc<double>(n);
-    res_bufs_.push_back((void *)d);
-    k_empty_mail<<<(unsigned)((n + 255) / 256), 256, 0, st_>>>((unsigned long long *)d, n);
-    CB_HIP(hipGetLastError());
-    return d;
   }
 
   Csr csr() const { return Csr{row_, col_, val_}; }
@@ -1126,7 +1117,7 @@ class GlobalRkc : public Engine {
   bool started_ = false;                       // a macro step has been asked for
   RkcArgs A_{};
   RkcCtl *ctl_host_ = nullptr;   // written by the kernel as it ends
-  int *late_host_ = nullptr;     // set by the kernel: a wait gave up
+  int *late_host_ = nullptr;     // behind it, set by the kernel: a wait gave up
   bool failed_ = false;
   const void *res_fn_ = nullptr;
   void *state_dev_ = nullptr;    // the model's state struct, and what is in it
@@ -1134,7 +1125,7 @@ class GlobalRkc : public Engine {
   size_t res_lds_ = 0;
   int res_grid_ = 1;             // workgroups with their helpers
   long macro_ = 0;
-  std::vector<void *> res_bufs_;
+  void *res_buf_ = nullptr;      // the tables and mailboxes
   std::vector<int> row_h_, col_h_;
   std::vector<double> val_h_;
   double *rec_ = nullptr;
