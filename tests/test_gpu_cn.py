@@ -15,11 +15,11 @@ device's and the host's exp / log in the ion updates:
   granule cells with a step current, 12 ms: first interval to 1e-9 mV, spike
   counts equal, times within one output interval.
 
-Populations of at most 16 x 256 compartments (all of the above) run each
-step's whole solve in one workgroup (k_kry_small); larger ones launch the
-two halves of every iteration over the whole grid (k_kry_a / k_kry_b).  Both
-reduce in the same order, so both match the oracle alike; the 2 x 4 granule
-population (4 624 compartments, 19 blocks) checks the multi-block path.
+All of these run a step's whole solve in the resident kernel
+(csrc/kry_resident.hpp), the first three in one workgroup and the 2 x 4 granule
+population (4 624 compartments) in several.  The launches that larger systems
+take (k_kry_small, k_kry_a / k_kry_b) reduce in the same order;
+test_gpu_paths.py compares them with the resident kernel bit for bit.
 """
 import ctypes
 import os
@@ -136,7 +136,7 @@ def test_cn_multiblock_gr_population(ref_data):
     p = cbrkc.Population(cbrkc.GR, 2, 4, solver=cbrkc.CN, morph=os.path.join(ref_data, "Gr.txt"), v0=v0)
     assert p.nc > 16 * 256
     o = oracle_cn(gr_pop(ref_data, 2, 4, v0=v0))
-    print("CN GR 2x4 (multi-block Krylov launches), 4 output intervals", flush=True)
+    print("CN GR 2x4 (several workgroups), 4 output intervals", flush=True)
     run_pair(p, o, 4, 16, 578, 1e-9)
     st = p.stats()
     assert st["steps"] == 20 and 0 < st["stages"] <= 2000, st

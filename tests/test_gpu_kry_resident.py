@@ -8,7 +8,8 @@ and sums are the oracle's in its order, so the difference is that of exp in
 the ion updates (1e-9 mV, the bar of the other CN tests; the truncated BE
 iterates move by up to 2e-4 mV under one ulp of the input,
 test_oracle_be.py::test_truncated_cg_noise_floor), and the iteration counts
-are equal."""
+are equal.  (That the iterates are those of the launches per iteration bit for
+bit is tested in test_gpu_paths.py.)"""
 import os
 
 import numpy as np
@@ -51,6 +52,7 @@ def test_one_interval(ref_data, solver, cell, nx, ny, grid):
     d = np.abs(p.read(cbrkc.F_V) - o.get(orc.V)).max()
     print("max |GPU - oracle|", d, p.stats(), flush=True)
     assert d <= (1e-9 if solver == cbrkc.CN or cell in ("io", "go") else 1e-3)
+    assert p.stats()["stages"] == o.stats()["stages"]
     if cell != "io":
         # trees at these steps never reach 1e-15: 100 iterations each
         assert cell == "go" or p.stats()["stages"] == 500
