@@ -606,7 +606,7 @@ class GlobalRkc : public Engine {
       A_.p1 = std::pow(c.err, 1.0 / 3.0);
       A_.p2 = std::pow(c.err, 2.0 / 3.0);
     }
-    if (c.status == ASK_STAGE) rkc_stage_start(c.m, &A_.asked.x, &A_.asked.y);
+    if (c.status == ASK_STAGE) rkc_stage_start(c.m, &A_.p1, &A_.p2);
     if (c.status == 0 || A_.resume) return;
     if (c.status == NONFINITE)
       throw Error("RKC: non-finite state (error estimate " + std::to_string(c.err) + ")", NONFINITE);
@@ -753,14 +753,13 @@ class GlobalRkc : public Engine {
     a.v1 = vec_[VT1];
     a.v2 = vec_[VT2];
     a.cm = cm_;
-    static const std::vector<double> stage_table = rkc_stage_table(RES_COEF);   // the same for every population
-    T.put_static(a.coef, stage_table);
-    static const std::vector<double2> start_table = [] {
-      std::vector<double2> t(RES_START + 1);
-      for (int m = 0; m <= RES_START; m++) rkc_stage_start(m, &t[m].x, &t[m].y);
+    static const std::vector<double> stage_table = [] {   // the same for every population
+      std::vector<double> t = rkc_stage_table(RES_COEF);
+      t.resize(RES_COEFS + 2 * (RES_START + 1));
+      for (int m = 0; m <= RES_START; m++) rkc_stage_start(m, &t[RES_COEFS + 2 * m], &t[RES_COEFS + 2 * m + 1]);
       return t;
     }();
-    T.put_static(a.start, start_table);
+    T.put_static(a.coef, stage_table);
     RkcCtl c{};
     std::memcpy(c.o, o_, sizeof(o_));
     std::memcpy(c.hw, hw_, sizeof(hw_));
@@ -787,7 +786,6 @@ class GlobalRkc : public Engine {
     a.wait = WAIT_TICKS;
     late_host_ = (int *)(ctl_host_ + 1);
     *late_host_ = 0;
-    a.late = (int *)(a.ctl_host + 1);
     a.integ = integ_;
     a.rho_floor = rho_floor_;
     a.strict = res_strict();

@@ -37,10 +37,12 @@ constexpr unsigned long long WAIT_TICKS = 60ull * 100000000ull;    // the limit 
 
 inline unsigned long long wait_ticks(double seconds) { return (unsigned long long)(seconds * 1e8); }
 
-// The limit of a wait and the workgroup's LDS word that is set once one gave up
+// The limit of a wait, the workgroup's LDS word that is set once one gave up, and
+// whether this thread's did (looked at in every sum: a register)
 struct Wait {
   unsigned long long ticks;
   volatile int *late;
+  int mine;
 };
 
 __device__ inline void mail_put(double *slot, double v) {
@@ -53,30 +55,31 @@ __device__ inline void mail_clear(double *slot) {
 }
 // the slot's value once it is there, or 0 when the wait gives up (with a limit
 // of 0 at the first look that finds nothing)
-__device__ inline double mail_get(const double *slot, const Wait &W) {
-  unsigned long long b = __hip_atomic_load((const unsigned long long *)slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  if (b == MAIL_EMPTY) {
-    const unsigned long long t0 = wall_clock64();
-    bool give_up = *W.late || W.ticks == 0;
-    for (int n = 1; !give_up; n++) {
-      b = __hip_atomic_load((const unsigned long long *)slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (b != MAIL_EMPTY) break;
-      if ((n & 1023) == 0) give_up = *W.late || wall_clock64() - t0 > W.ticks;
-    }
-    if (give_up) {
-      *W.late = 1;
-      return 0.0;
+__device__ inline double mail_get(const double *slot, Wait &W) {
+  // (neither the clock nor the LDS word is looked at before the 128th look, some
+  // 100 us: a value is there after a few)
+  unsigned long long b, t0 = 0;
+  for (unsigned n = 1;; n++) {
+    b = __hip_atomic_load((const unsigned long long *)slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (b != MAIL_EMPTY) break;
+    if ((n & 127) == 0 || W.ticks == 0) {
+      const unsigned long long t = wall_clock64();
+      if (t0 == 0) t0 = t;
+      if (*W.late || t - t0 >= W.ticks) {
+        W.mine = *W.late = 1;
+        return 0.0;
+      }
     }
   }
   return __longlong_as_double((long long)b);
 }
 // mail_get for a wait that may be long: it leaves 256 cycles between looks
-__device__ inline double mail_wait(const double *slot, const Wait &W) {
+__device__ inline double mail_wait(const double *slot, Wait &W) {
   const unsigned long long t0 = wall_clock64();
   while (__hip_atomic_load((const unsigned long long *)slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == MAIL_EMPTY) {
     __builtin_amdgcn_s_sleep(4);
     if (*W.late || wall_clock64() - t0 > W.ticks) {
-      *W.late = 1;
+      W.mine = *W.late = 1;
       return 0.0;
     }
   }
@@ -132,7 +135,7 @@ struct SumPlan {
 // whole vector, so the total equals the multi-launch reduction bit for bit.
 template <int NT>
 __device__ inline double grid_sum(const SumPlan &P, double *term, double *part, double *terms, double *parts,
-                                  unsigned &q, const Wait &W, bool &late) {
+                                  unsigned &q, Wait &W, bool &late) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, R = P.r1 - P.r0;
   double *tq = terms + (size_t)q * P.nc, *pq = parts + (size_t)q * P.nch;
   if (!P.alone) {
@@ -157,7 +160,7 @@ __device__ inline double grid_sum(const SumPlan &P, double *term, double *part, 
   if (!P.alone)
     for (int k = tid; k < P.nch; k += NT) part[k] = mail_get(pq + k, W);
   if (P.alone) __syncthreads();
-  else late = __syncthreads_or(*W.late);
+  else late = __syncthreads_or(W.mine);
   // the partials by the same tree, level by level (at most 2048 of them)
   int m = P.nch;
   const double *in = part;

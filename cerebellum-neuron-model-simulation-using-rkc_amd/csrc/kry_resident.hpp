@@ -61,7 +61,7 @@ __global__ void __launch_bounds__(NT) k_kry_resident(KryArgs A) {
   unsigned short *TR = LC + A.nnz_max, *TC = TR + A.rb + 1;
   SumPlan S;
   S.set(A.nc, r0, r0 + R);
-  const Wait W{A.wait, &s_late};
+  Wait W{A.wait, &s_late, 0};
   bool late = false;
   unsigned q = A.q[0];
   // a solve before this one ended with its mailboxes half read: those already

@@ -51,15 +51,14 @@ constexpr int ASK_POW = 9;     // status: the host has to give the powers of err
 constexpr int ASK_STAGE = 10;  // status: the host has to give w1 and mu~_1 for m
 constexpr int RES_COEF = 128;
 constexpr int RES_START = 4096;
+constexpr int RES_COEFS = (RES_COEF + 1) * RES_COEF * 4;   // doubles of the coefficient table
 constexpr int ROW_W = 3;            // neighbours of a compartment held in registers (parent and two children)
 constexpr int GHOST_STAGES = 136;   // exchanges of coupled values between two sums
 
 struct RkcArgs {
   int n, nc, comp, nblk, cpb;            // cells, rows, rows per cell, workgroups, cells per workgroup
   int ext_max, ghost_max, nch;           // LDS sizes: further entries and ghosts of a workgroup, chunks
-  const int *row, *col;                  // CSR of the cable matrix
-  const double *val;
-  // the same rows without the diagonal, columns local (ghosts from the
+  // the rows of the cable matrix without the diagonal, columns local (ghosts from the
   // workgroup's row count on): the first ROW_W entries of row i in lval[k nc + i]
   // and the 16-bit quarters of lcol[i], whose last holds the row's further
   // entries, start << 4 | count, in the workgroup's xcol / xval
@@ -70,7 +69,6 @@ struct RkcArgs {
   const int *x0;                         // first further entry of each workgroup (nblk + 1)
   const int *imp0, *exp0, *exp_row, *exp_slot;   // ghosts fetched, rows posted (null: uncoupled cells)
   unsigned long long wait;               // the limit of a wait (grid_mail.hpp)
-  int *late;                             // mapped host memory: set by whichever workgroup or helper gave up
   double *ghost;                         // [3][GHOST_STAGES][nslot]
   int nslot;
   double *terms, *parts;                 // grid_sum's mailboxes
@@ -84,14 +82,14 @@ struct RkcArgs {
   double *req, *vin, *bout;
   unsigned gq0;                          // number of the launch's first ion update
   double *y, *yn, *fn, *ede, *vnew, *b, *v1, *v2;
-  const double *cm, *coef;
-  const double2 *start;                  // {w1, mu~_1} of m = 0 .. RES_START stages
-  RkcCtl *ctl, *ctl_host;                // the record, and its copy in mapped host memory
+  const double *cm, *coef;               // coef: the coefficients, then {w1, mu~_1} of m = 0 .. RES_START stages
+  // the record, and its copy in mapped host memory with a word behind it that
+  // whichever workgroup or helper gives up sets
+  RkcCtl *ctl, *ctl_host;
   // the attempt that stopped goes on: ASK_POW with err's powers p1, p2,
-  // ASK_STAGE with w1 and mu~_1 in asked (0: no attempt stopped)
+  // ASK_STAGE with w1 and mu~_1 in them (0: no attempt stopped)
   int resume;
   double p1, p2;
-  double2 asked;
   double integ, rho_floor;
   int strict, refresh_fn;
   // per macro step: the stimulus, the Poisson drive, the recorder
@@ -158,7 +156,7 @@ __device__ inline CubeRoots cube_roots(double x) {
 struct GapView {
   const double *y, *gap;
   int cell0, cells, comp;
-  const Wait *wait;
+  Wait *wait;
   __device__ double operator()(int cell) const {
     if (cell >= cell0 && cell < cell0 + cells) return y[(cell - cell0) * comp];
     return mail_get(gap + cell, *wait);
@@ -185,7 +183,7 @@ __device__ inline void rkc_helper(const RkcArgs &A, const typename Model::State 
   const int l0 = min(R, (j + 1) * A.own), l1 = min(R, l0 + A.own), r0 = w * RM;
   __shared__ int s_late;
   if (tid == 0) s_late = 0;
-  const Wait W{A.wait, &s_late};
+  Wait W{A.wait, &s_late, 0};
   for (unsigned g = A.gq0;; g = g == 2 ? 0 : g + 1) {
     if (tid == 0) {
       const double *rq = A.req + ((size_t)g * A.nblk + w) * 2;
@@ -211,7 +209,7 @@ __device__ inline void rkc_helper(const RkcArgs &A, const typename Model::State 
       mail_clear(A.bout + old + row);
     }
     if (late || !(dt >= 0.0)) {
-      if (late && tid == 0) *A.late = 1;
+      if (late && tid == 0) *(int *)(A.ctl_host + 1) = 1;
       return;
     }
   }
@@ -241,14 +239,15 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, const typena
   unsigned short *XC = (unsigned short *)(XV + A.ext_max);
   __shared__ int s_late;
   if (tid == 0) s_late = 0;
-  const Wait W{A.wait, &s_late};
-  bool late = false;   // the same in the whole workgroup: s_late as of the last sum or ion update
+  Wait W{A.wait, &s_late, 0};
+  bool late = false;   // the same in the whole workgroup: a wait gave up before the last sum or ion update
   SumPlan P;
   P.set(A.nc, r0, r0 + R);
 
   RkcCtl *ctl = A.ctl;
   const double at = ctl->o[4], rt = ctl->o[5], hmin = ctl->hw[6], mmax = ctl->o[0];
   __shared__ double s_ctl[NT / 64][16];
+  __shared__ int s_m;              // stages of the attempt that the host is asked about: thread 0's
   __shared__ long long s_cnt[5];   // steps, rejects, stages, power iterations, ion updates: kept by thread 0
   double *cs = s_ctl[tid >> 6];
   double &absh = cs[0], &sprad = cs[1], &naccpt = cs[2], &idid = cs[3], &gt = cs[4], &gt_old = cs[5], &lt = cs[6],
@@ -268,7 +267,7 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, const typena
   unsigned q = ctl->q, gq = A.gq0;
   int status = 0, done_steps = 0;
   int resume = A.resume;
-  int loops = ctl->loops, m_now = ctl->m;
+  int loops = ctl->loops;
   CubeRoots ce;
   ce.p1 = A.p1;
   ce.p2 = A.p2;
@@ -403,7 +402,7 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, const typena
       fetch(YN);
       rows([&](int k, int i) { FN[i] = rhs(k, YN[i], YN); });
     }
-    late = __syncthreads_or(s_late);
+    late = __syncthreads_or(W.mine);
   };
 
   // rkcrho (solve_rkc.cu:562-754)
@@ -478,8 +477,8 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, const typena
   };
 
   // step (solve_rkc.cu:815-906)
-  auto step = [&](double h, int m, double w1, double mus) {
-    double w0 = 0.0;
+  auto step = [&](double h, int m) {
+    double w0 = 0.0, w1 = 0.0, mus;
     const bool tab = m >= 2 && m <= RES_COEF;
     if (tab) {
       const double *ct = A.coef + (size_t)m * RES_COEF * 4;
@@ -487,6 +486,8 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, const typena
       mus = ct[0];
     } else {
       w0 = 1.0 + 2.0 / (13.0 * m * m);
+      w1 = m > RES_START ? A.p1 : A.coef[RES_COEFS + 2 * m];
+      mus = m > RES_START ? A.p2 : A.coef[RES_COEFS + 2 * m + 1];
     }
     const double hm = h * mus;
     for (int i = tid; i < R; i += NT) {
@@ -547,39 +548,35 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, const typena
 
   // an attempt of rkclow (solve_rkc.cu:908-1096) up to its error norm
   auto attempt = [&]() {
-    double2 w = A.asked;
-    if (!resume) {
-      if (newspc) {
-        rkcrho();
-        if (sprad < A.rho_floor) sprad = A.rho_floor;
-        jacatt = true;
-      }
-      last = false;
-      if (1.1 * absh >= fabs(tend - lt)) {
-        absh = fabs(tend - lt);
-        last = true;
-      }
-      const double mr = sqrt(1.54 * absh * sprad + 1.0);
-      int m = (mr < mmax) ? 1 + (int)mr : (int)mmax + 1;
-      if (m > mmax) {
-        m = (int)mmax;
-        absh = (m * m - 1) / (1.54 * sprad);
-        last = false;
-      }
-      double h = absh;
-      if (h <= hmin) h = hmin;
-      h_now = h;
-      m_now = m;
-      if (m > RES_START) {
-        status = ASK_STAGE;
-        return;
-      }
-      if (m < 2 || m > RES_COEF) w = A.start[m];
+    if (newspc) {
+      rkcrho();
+      if (sprad < A.rho_floor) sprad = A.rho_floor;
+      jacatt = true;
     }
-    resume = 0;
-    const double h = h_now;
-    const int m = m_now;
-    step(h, m, w.x, w.y);
+    const double absh_in = absh;
+    last = false;
+    if (1.1 * absh >= fabs(tend - lt)) {
+      absh = fabs(tend - lt);
+      last = true;
+    }
+    const double mr = sqrt(1.54 * absh * sprad + 1.0);
+    int m = (mr < mmax) ? 1 + (int)mr : (int)mmax + 1;
+    if (m > mmax) {
+      m = (int)mmax;
+      absh = (m * m - 1) / (1.54 * sprad);
+      last = false;
+    }
+    if (__builtin_expect(m > RES_START && !resume, 0)) {   // the attempt begins again, but for the spectral radius
+      absh = absh_in;
+      newspc = false;
+      status = ASK_STAGE;
+      if (tid == 0) s_m = m;
+      return;
+    }
+    double h = absh;
+    if (h <= hmin) h = hmin;
+    h_now = h;
+    step(h, m);
     // f(Y_m) and the error estimate (every weight is positive: atol > 0)
     fetch(Yv);
     double fo[K], to[K];
@@ -608,6 +605,7 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, const typena
       } else {
         if (!resume && ++loops > 1000) return;
         attempt();
+        resume = 0;
         if (late || status != 0) return;
         if (!isfinite(err)) {
           status = Model::NONFINITE_STATUS;
@@ -733,7 +731,7 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, const typena
       A.v2[r0 + i] = V2[i];
     }
   });
-  if (tid == 0 && s_late) *A.late = 1;
+  if (tid == 0 && s_late) *(int *)(A.ctl_host + 1) = 1;
   if (w == 0 && tid == 0) {
     RkcCtl c = *ctl;
     c.o[1] = absh; c.o[2] = sprad; c.o[3] = naccpt; c.o[6] = idid; c.o[7] = gt;
@@ -743,7 +741,7 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, const typena
     c.steps = s_cnt[0]; c.rejects = s_cnt[1]; c.stages = s_cnt[2]; c.rho_iters = s_cnt[3]; c.ions = s_cnt[4];
     c.macro += done_steps;
     c.last = last; c.newspc = newspc; c.jacatt = jacatt; c.status = status;
-    c.q = q; c.ions_q = gq; c.ghost_used = gs_old; c.loops = loops; c.m = m_now; c.ghost_now = gs;
+    c.q = q; c.ions_q = gq; c.ghost_used = gs_old; c.loops = loops; c.m = s_m; c.ghost_now = gs;
     *ctl = c;
     *A.ctl_host = c;
   }

@@ -10,7 +10,7 @@ mkdir -p "$OUT"
 for f in detsum grid_mail rkc_resident; do
   sed -e 's/extern __shared__ double sm\[\];/double *const sm = emu_lds();/' \
       -e 's/__shared__ int s_late;/int \&s_late = *emu_late();/' \
-      -e 's/__shared__ \(double\|long long\) s_/static thread_local \1 s_/' \
+      -e 's/__shared__ \(double\|long long\|int\) s_/static thread_local \1 s_/' \
       -e 's/asm volatile("s_waitcnt vmcnt(0)" ::: "memory");/__atomic_thread_fence(__ATOMIC_SEQ_CST);/' \
       "$C/$f.hpp" > "$OUT/$f.hpp"
 done

@@ -162,9 +162,9 @@ int emu_rkc(int n, int comp, int cpb, int nhelp, int present, const int *row, co
   std::vector<double> ghost((size_t)3 * GHOST_STAGES * max(1, nslot), empty), terms((size_t)3 * nc, empty),
       parts((size_t)3 * a.nch, empty), gap((size_t)3 * n, empty), req((size_t)6 * nblk, empty),
       vin((size_t)3 * nc, empty), bout((size_t)3 * nc, empty), v1(nc), v2(nc), bb(b, b + nc), iext(nc), amp(n);
-  const std::vector<double> table = rkc_stage_table(RES_COEF);
-  std::vector<double2> start(RES_START + 1);
-  for (int m = 0; m <= RES_START; m++) rkc_stage_start(m, &start[m].x, &start[m].y);
+  std::vector<double> table = rkc_stage_table(RES_COEF);
+  table.resize(RES_COEFS + 2 * (RES_START + 1));
+  for (int m = 0; m <= RES_START; m++) rkc_stage_start(m, &table[RES_COEFS + 2 * m], &table[RES_COEFS + 2 * m + 1]);
   if (nslot > 0) {
     a.imp0 = imp0.data();
     a.exp0 = exp0.data();
@@ -196,16 +196,15 @@ int emu_rkc(int n, int comp, int cpb, int nhelp, int present, const int *row, co
   a.v2 = v2.data();
   a.cm = cm;
   a.coef = table.data();
-  a.start = start.data();
   a.integ = 1e30;
   a.wait = wait_ticks(wait);
-  int late = 0;
-  a.late = &late;
   a.rho_floor = rho_floor;
   a.refresh_fn = refresh;
   a.iext = iext.data();
   a.amp = amp.data();
-  RkcCtl ctl{}, host{};
+  RkcCtl ctl{}, hosts[2] = {};   // the copy, and the word behind it
+  RkcCtl &host = hosts[0];
+  const int &late = *(const int *)&hosts[1];
   std::memcpy(ctl.o, o16, sizeof(ctl.o));
   std::memcpy(ctl.hw, hw8, sizeof(ctl.hw));
   ctl.errold3 = std::pow(ctl.o[11], 1.0 / 3.0);
@@ -246,7 +245,7 @@ int emu_rkc(int n, int comp, int cpb, int nhelp, int present, const int *row, co
     a.resume = host.status == ASK_POW || host.status == ASK_STAGE ? host.status : 0;
     a.p1 = std::pow(host.err, 1.0 / 3.0);
     a.p2 = std::pow(host.err, 2.0 / 3.0);
-    if (host.status == ASK_STAGE) rkc_stage_start(host.m, &a.asked.x, &a.asked.y);
+    if (host.status == ASK_STAGE) rkc_stage_start(host.m, &a.p1, &a.p2);
     if (late) return TIMED_OUT;
     if (host.status != 0 && !a.resume) break;
   }
