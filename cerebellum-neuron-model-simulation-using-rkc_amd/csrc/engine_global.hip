@@ -627,7 +627,14 @@ class GlobalRkc : public Engine {
   // its tables.  Whole cells go to a workgroup, as few as leave at most one
   // workgroup per CU (more CUs shorten the ion update, whose rows run one to a
   // thread) but at least a row per thread; the population has to fit the LDS of
-  // the chip's CUs.  Larger ones are bound by the vectors' traffic and stay on
+  // the chip's CUs.  Measured, ms a call at this and more cells to a workgroup:
+  // 256 Golgi cells at 1 / 2 / 4 / 8: 24.8 / 31.6 / 36.8 / 48.3; 100 granule cells at 1 /
+  // 2 / 3: 8.5 / 10.6 / 11.8; 512 granule chains of 4 rows at 64 / 128 / 256 / 448, the
+  // further rows' ion updates on helpers: 38.7 / 41.6 / 52.1 / 63.1 (128 chains, 64 /
+  // 128: 37.1 / 34.2); 1024 olive cells at 32 / 64 / 85 / 128: 5.3 / 5.2 / 5.2 / 7.5.  A
+  // norm costs about the same among 2 and among 256 workgroups, rows beyond one to a
+  // thread cost an ion update each, so only populations that one workgroup
+  // holds would gain from more rows.  Larger ones are bound by the vectors' traffic and stay on
   // the launch-per-stage path, and so do populations of several workgroups in a
   // process that may not launch cooperatively.
   void make_resident() {
