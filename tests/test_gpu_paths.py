@@ -7,6 +7,8 @@ counter, recording and spike is the same bits, with ion updates, stimulus,
 gap junctions, Poisson drive and synapses; so the small populations here, and
 with them the oracle's tests of either path, cover both."""
 import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -22,11 +24,15 @@ T0 = 600.0   # inside the reference's stimulus windows
 FIELDS = (cbrkc.F_VNEW, cbrkc.F_V, cbrkc.F_CA, cbrkc.F_B, cbrkc.F_IEXT)
 
 
-def make(ref_data, cell, nx, ny, **kw):
+def population(ref_data, cell, nx, ny, **kw):
     kind, f, v, _ = KIND[cell.split()[0]]
     gj = os.path.join(ref_data, "Pkj_GJ.csv") if cell == "pkj gj" else ""
     v0 = v + 0.05 * (np.arange(nx * ny) % 31)
-    pops = [cbrkc.Population(kind, nx, ny, morph=os.path.join(ref_data, f), gj=gj, v0=v0, **kw) for _ in range(2)]
+    return cbrkc.Population(kind, nx, ny, morph=os.path.join(ref_data, f), gj=gj, v0=v0, **kw)
+
+
+def make(ref_data, cell, nx, ny, **kw):
+    pops = [population(ref_data, cell, nx, ny, **kw) for _ in range(2)]
     pops[1].launch_path()
     assert "workgroups" in pops[0].mapping() and "workgroups" not in pops[1].mapping(), [p.mapping() for p in pops]
     return pops
@@ -107,3 +113,35 @@ def test_network(ref_data, tmp_path):
     for pop in (cbrkc.NET_GR, cbrkc.NET_GO, cbrkc.NET_PKJ):
         g = [net.conductance(pop, cbrkc.NET_AMPA) for net in nets]
         assert np.array_equal(*g) and g[0].any()
+
+
+CHILD = """
+import sys
+sys.path[:0] = sys.argv[1:3]
+import numpy as np
+import cbrkc
+import test_gpu_paths as T
+out = {}
+for name, cell, nx, ny, kw in T.ELSEWHERE:
+    p = T.population(sys.argv[3], cell, nx, ny, **kw)
+    print(name, p.mapping(), flush=True)
+    out[name] = np.concatenate([p.run(2, T.T0, -1).ravel(), p.read(cbrkc.F_B)])
+np.savez(sys.argv[4], **out)
+"""
+ELSEWHERE = [("io", "io", 13, 40, {}), ("gr", "gr", 1, 1, {}), ("pkj cn", "pkj", 4, 1, dict(solver=cbrkc.CN))]
+
+
+def test_a_second_process(ref_data, tmp_path):
+    # This process has launched cooperatively and keeps the barrier resource to its
+    # end; another one that is refused it takes the other path, with the same results
+    here, out = {}, str(tmp_path / "out.npz")
+    for name, cell, nx, ny, kw in ELSEWHERE:
+        p = population(ref_data, cell, nx, ny, **kw)
+        here[name] = np.concatenate([p.run(2, T0, -1).ravel(), p.read(cbrkc.F_B)])
+    r = subprocess.run([sys.executable, "-c", CHILD, os.path.dirname(cbrkc.__file__), os.path.dirname(__file__), ref_data,
+                        out], capture_output=True, text=True, timeout=100)
+    print(r.stdout, r.stderr[-2000:], flush=True)
+    assert r.returncode == 0
+    there = np.load(out)
+    for name in here:
+        assert np.array_equal(here[name], there[name]), name
