@@ -4,7 +4,8 @@
 // Populations that fit the LDS of the chip's CUs run on the resident kernel
 // (rkc_resident.hpp: many macro steps a launch, the controller on the device).
 // The rest of this file is the launch-per-stage path of larger ones, which also
-// initialises every population; the two give the same bits.
+// initialises every population; the two give the same bits, and a small population
+// can be made to take this one (use_launches).
 //
 // One thread per compartment, structure-of-arrays FP64 state in HBM.  The
 // differences from the reference are in how the work is laid out, not in

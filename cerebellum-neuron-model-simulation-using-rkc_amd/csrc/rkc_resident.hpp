@@ -11,12 +11,13 @@
 // the error norm's partial sums.  Cells whose cable matrix couples them
 // (gap junctions) also exchange the coupled compartments' values at every
 // stage.  The additions of every right-hand side, stage and norm are those of
-// the launch-per-stage path in the same order, so the two agree bit for bit.
+// the launch-per-stage path in the same order, and what either takes from libm
+// the other does too, so the two agree bit for bit.
 // Measured, Population.run from the initial state and then on average over the
-// next passes (ms): 64 olive cells, 40 macro steps, 81.4 / 13.7 -> 11.9 / 3.1;
-// 256 Golgi cells, 40 steps, 22.7 / 65.1 -> 8.6 / 24.5; 16 granule cells, one
-// step, 39.0 / 25.9 -> 12.0 / 8.3; 64 coupled Purkinje cells, 8 steps, 10.0 /
-// 3.1 -> 4.9 / 1.7; 9 uncoupled ones 6.8 / 9.0 -> 3.9 / 5.4.
+// eleven calls after it, launch per stage -> this kernel (ms): 64 olive cells, 40
+// macro steps, 101 / 15.3 -> 12.0 / 3.1; 256 Golgi cells, 40 steps, 22.7 / 65.9 -> 8.7 /
+// 24.8; 16 granule cells, one step, 39.6 / 26.5 -> 10.1 / 6.9; 64 coupled Purkinje
+// cells, 8 steps, 9.3 / 2.9 -> 4.6 / 1.5; 9 uncoupled ones 6.5 / 8.1 -> 2.9 / 3.9.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -117,8 +118,9 @@ struct RkcArgs {
 // voltage by 1e-4 mV within 0.5 ms.  libm's pow misses the nearest double only
 // where the value lies within 0.0083 ulp of the middle between two (measured,
 // 12 million arguments, 8e-4 of them missed), so a result that is POW_SLACK or more away from
-// a middle is libm's result too; for the others (sure = false, one in 50) the
-// kernel stops and the host answers with pow.
+// a middle is libm's result too; for the others (sure = false, one power in 50) the
+// kernel stops and the host answers with pow: one attempt in 26 (olive) to 32 (granule,
+// Golgi), since an accepted one needs both powers.
 constexpr double POW_SLACK = 0.01;
 struct CubeRoots {
   double p1, p2;
@@ -169,6 +171,7 @@ struct GapView {
 // update takes up to 430 registers, so nothing lives across it: the controller
 // stays in LDS (a copy for every wave), the thread's matrix rows are read again
 // after it, and it is inlined at one place only.
+
 // The ion updates of some of workgroup w's rows.  A cell of 1600 compartments
 // is four rows to a thread of its workgroup, one after the other, while most
 // CUs have nothing to do: 9 cells, 8 macro steps, 5.4 -> 3.9 ms with three
