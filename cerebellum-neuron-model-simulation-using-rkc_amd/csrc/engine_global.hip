@@ -602,12 +602,13 @@ class GlobalRkc : public Engine {
     failed_ = *(volatile int *)late_host_ != 0;
     check();
     macro_ = c.macro;
-    A_.resume = c.status == ASK_POW || c.status == ASK_STAGE ? c.status : 0;
+    A_.resume = c.status == ASK_POW || c.status == ASK_STAGE || c.status == ASK_DECAY ? c.status : 0;
     if (c.status == ASK_POW) {
       A_.p1 = std::pow(c.err, 1.0 / 3.0);
       A_.p2 = std::pow(c.err, 2.0 / 3.0);
     }
     if (c.status == ASK_STAGE) rkc_stage_start(c.m, &A_.p1, &A_.p2);
+    if (c.status == ASK_DECAY) A_.p1 = std::exp(-c.sum_dt / 0.6);
     if (c.status == 0 || A_.resume) return;
     if (c.status == NONFINITE)
       throw Error("RKC: non-finite state (error estimate " + std::to_string(c.err) + ")", NONFINITE);
@@ -748,7 +749,7 @@ class GlobalRkc : public Engine {
       T.space(a.gap, (size_t)3 * n_);
     }
     if (a.nhelp > 0) {
-      T.space(a.req, (size_t)6 * a.nblk);
+      T.space(a.req, (size_t)9 * a.nblk);
       T.space(a.vin, (size_t)3 * nc_);
       T.space(a.bout, (size_t)3 * nc_);
     }
@@ -1174,7 +1175,7 @@ class GlobalPkj : public GlobalRkc {
     // the granule input enters at ion updates only (pkj_update_ion_and_matrix)
     const bool net = do_ion && net_.on();
     PkjState S{v_, ca_, rev_, iext_, shell_, cond_, gate_, b_, syn_g_, syn_.e_syn, nc_,
-               net ? net_s_ : nullptr, net ? exp_cr(-dt / 0.6) : 0.0};
+               net ? net_s_ : nullptr, net ? std::exp(-dt / 0.6) : 0.0};
     k_pkj_ion_b<<<nblk(nc_), 256, 0, st_>>>(S, vv, dt, do_ion ? 1 : 0);
   }
  public:

@@ -6,7 +6,6 @@
 #include <hip/hip_runtime.h>
 
 #include "engine.hpp"
-#include "exp_acc.hpp"
 #include "ion_state.hpp"
 #include "pkj_model.hpp"
 #include "rkc_resident.hpp"
@@ -22,7 +21,7 @@ struct PkjState {
   double syn_e;
   int nc;
   const double *net_s;  // synaptic current of the macro step (granule input), may be null
-  double net_decay;     // exp(-dt / 0.6), dt the ion interval; correctly rounded on either path
+  double net_decay;     // exp(-dt / 0.6), dt the ion interval, as the host's libm gives it
 };
 
 // pkj_update_ion_RKC (pkj_ion.cu:304-358) followed by pkj_update_matrix
@@ -119,17 +118,24 @@ __device__ inline double gr_ion_net_current(const GrState &S, int i, double vn, 
 struct PkjModel {
   using State = PkjState;
   static constexpr int NT = 512, K0 = 0, K1 = 0, K2 = 4, NONFINITE_STATUS = NONFINITE;
-  static constexpr bool GAP = false, HELP = true;
-  __device__ __attribute__((noinline)) static double ion(const State *Sp, int i, double vn, double dt, const GapView *) {
+  static constexpr bool GAP = false, HELP = true, DECAY = true;
+  // (a call, so that populations without synapses do not pay for it in registers)
+  __device__ __attribute__((noinline)) static double decay(double dt) {
+    bool sure;
+    const double d = exp_libm(-dt / 0.6, sure);
+    return sure ? d : __longlong_as_double(0x7FF8000000000000ll);
+  }
+  __device__ __attribute__((noinline)) static double ion(const State *Sp, int i, double vn, double dt, const GapView *,
+                                                         double decay) {
     State S = *Sp;
-    if (S.net_s) S.net_decay = exp_cr(-dt / 0.6);
+    S.net_decay = decay;
     return pkj_ion_current(S, i, vn, dt, true);
   }
 };
 struct IoModel {
   using State = IoState;
   static constexpr int NT = 256, K0 = 0, K1 = 1, K2 = 7, NONFINITE_STATUS = NONFINITE;
-  static constexpr bool GAP = true, HELP = false;
+  static constexpr bool GAP = true, HELP = false, DECAY = false;
   __device__ __forceinline__ static double ion(const State *S, int i, double vn, double dt, const GapView *gap) {
     return io_ion_gap_current(*S, i, vn, dt, true, [&](int cell) { return (*gap)(cell); });
   }
@@ -137,7 +143,7 @@ struct IoModel {
 struct GoModel {
   using State = GoState;
   static constexpr int NT = 256, K0 = 0, K1 = 1, K2 = 7, NONFINITE_STATUS = NONFINITE;
-  static constexpr bool GAP = false, HELP = false;
+  static constexpr bool GAP = false, HELP = false, DECAY = false;
   __device__ __forceinline__ static double ion(const State *S, int i, double vn, double dt, const GapView *) {
     return go_ion_net_current(*S, i, vn, dt, true);
   }
@@ -145,7 +151,7 @@ struct GoModel {
 struct GrModel {
   using State = GrState;
   static constexpr int NT = 256, K0 = 1, K1 = 3, K2 = 7, NONFINITE_STATUS = NONFINITE;
-  static constexpr bool GAP = false, HELP = true;
+  static constexpr bool GAP = false, HELP = true, DECAY = false;
   __device__ __attribute__((noinline)) static double ion(const State *S, int i, double vn, double dt, const GapView *) {
     return gr_ion_net_current(*S, i, vn, dt, true);
   }

@@ -21,6 +21,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "exp_acc.hpp"
 #include "grid_mail.hpp"
 #include "philox.hpp"
 
@@ -50,6 +51,7 @@ struct RkcCtl {
 // input sets in, carries to 1e-10 mV.)
 constexpr int ASK_POW = 9;     // status: the host has to give the powers of err
 constexpr int ASK_STAGE = 10;  // status: the host has to give w1 and mu~_1 for m
+constexpr int ASK_DECAY = 11;  // status: the host has to give the synaptic decay of the ion update over sum_dt
 constexpr int RES_COEF = 128;
 constexpr int RES_START = 4096;
 constexpr int RES_COEFS = (RES_COEF + 1) * RES_COEF * 4;   // doubles of the coefficient table
@@ -76,8 +78,8 @@ struct RkcArgs {
   double *gap;                           // [3][n]: dendrite voltages for the olive's gap currents
   // Helpers: workgroups beyond nblk that only run ion updates, nhelp for each
   // of the others, which keeps the rows before own and gives every helper the
-  // next own ones.  req [3][nblk][2]: the update's interval (< 0: the launch
-  // ends) and the macro step's time; vin, bout [3][nc]: the rows' new voltages
+  // next own ones.  req [3][nblk][3]: the update's interval (< 0: the launch
+  // ends), the macro step's time and the synaptic decay; vin, bout [3][nc]: the rows' new voltages
   // and their frozen currents.
   int nhelp, own;
   double *req, *vin, *bout;
@@ -87,8 +89,8 @@ struct RkcArgs {
   // the record, and its copy in mapped host memory with a word behind it that
   // whichever workgroup or helper gives up sets
   RkcCtl *ctl, *ctl_host;
-  // the attempt that stopped goes on: ASK_POW with err's powers p1, p2,
-  // ASK_STAGE with w1 and mu~_1 in them (0: no attempt stopped)
+  // what stopped goes on: ASK_POW with err's powers p1, p2, ASK_STAGE with w1 and
+  // mu~_1 in them, ASK_DECAY with the decay in p1 (0: nothing stopped)
   int resume;
   double p1, p2;
   double integ, rho_floor;
@@ -126,13 +128,6 @@ struct CubeRoots {
   double p1, p2;
   bool sure1, sure2;
 };
-__device__ inline double round_sure(double hi, double lo, bool &sure) {
-  const double s = hi + lo, rem = (hi - s) + lo;
-  const long long e = (__double_as_longlong(s) & 0x7FF0000000000000ll) - (52ll << 52);
-  const double ulp = __longlong_as_double(e);   // s within (1e-20, 1e20): a normal number
-  sure = fabs(fabs(rem) - 0.5 * ulp) > POW_SLACK * ulp;
-  return s;
-}
 __device__ inline CubeRoots cube_roots(double x) {
   CubeRoots r;
   if (!(x > 1e-30 && x < 1e30)) {
@@ -148,8 +143,8 @@ __device__ inline CubeRoots cube_roots(double x) {
   const double q = p * y, qe = fma(p, y, -q);
   const double c = ((x - q) - qe - pe * y) / (3.0 * p);
   const double d = 1.850371707708594e-17 * ((double)l2 * 0.6931471805599453);
-  r.p1 = round_sure(y, c - y * d, r.sure1);
-  r.p2 = round_sure(p, pe + 2.0 * y * c - p * (2.0 * d), r.sure2);
+  r.p1 = round_sure(y, c - y * d, POW_SLACK, r.sure1);
+  r.p2 = round_sure(p, pe + 2.0 * y * c - p * (2.0 * d), POW_SLACK, r.sure2);
   return r;
 }
 
@@ -166,11 +161,20 @@ struct GapView {
 };
 
 // Model: NT threads, the state struct, ion(S, i, vn, dt, gap) = ion update and
-// frozen current of row i, GAP = the olive's explicit gap currents, HELP = helpers
+// frozen current of row i (DECAY: with the synaptic current's decay over dt, which
+// follows the host's libm like the powers of err: decay(dt) is its value, or NaN where
+// it has to be asked), GAP = the olive's explicit gap currents, HELP = helpers
 // may run it.  The
 // update takes up to 430 registers, so nothing lives across it: the controller
 // stays in LDS (a copy for every wave), the thread's matrix rows are read again
 // after it, and it is inlined at one place only.
+
+template <class Model>
+__device__ __forceinline__ double model_ion(const typename Model::State *S, int i, double vn, double dt,
+                                            const GapView *gap, double decay) {
+  if constexpr (Model::DECAY) return Model::ion(S, i, vn, dt, gap, decay);
+  else return Model::ion(S, i, vn, dt, gap);
+}
 
 // The ion updates of some of workgroup w's rows.  A cell of 1600 compartments
 // is four rows to a thread of its workgroup, one after the other, while most
@@ -189,13 +193,14 @@ __device__ inline void rkc_helper(const RkcArgs &A, const typename Model::State 
   Wait W{A.wait, &s_late, 0};
   for (unsigned g = A.gq0;; g = g == 2 ? 0 : g + 1) {
     if (tid == 0) {
-      const double *rq = A.req + ((size_t)g * A.nblk + w) * 2;
+      const double *rq = A.req + ((size_t)g * A.nblk + w) * 3;
       sm[0] = mail_wait(rq, W);
       sm[1] = mail_get(rq + 1, W);
+      sm[2] = mail_get(rq + 2, W);
     }
     __syncthreads();
     const bool late = s_late;
-    const double dt = sm[0], t = sm[1];
+    const double dt = sm[0], t = sm[1], decay = sm[2];
     __syncthreads();
     const size_t copy = (size_t)g * A.nc, old = (size_t)(g == 0 ? 2 : g - 1) * A.nc;
     mail_settle();
@@ -207,7 +212,7 @@ __device__ inline void rkc_helper(const RkcArgs &A, const typename Model::State 
       if (!late && dt >= 0.0) {
         const double vn = mail_get(A.vin + copy + row, W);
         // without its voltages the helper posts nothing, and its workgroup gives up in turn
-        if (!*W.late) mail_put(A.bout + copy + row, Model::ion(S, row, vn, dt, nullptr));
+        if (!*W.late) mail_put(A.bout + copy + row, model_ion<Model>(S, row, vn, dt, nullptr, decay));
       }
       mail_clear(A.bout + old + row);
     }
@@ -366,18 +371,18 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, const typena
 
   // an ion update for the helpers, and the emptying of the one before it
   double t_now = t0;
-  auto request = [&](double dt, int own) {
+  auto request = [&](double dt, int own, double decay) {
     mail_settle();
     __syncthreads();
     for (int i = own + tid; i < R && dt >= 0.0; i += NT) mail_put(A.vin + (size_t)gq * A.nc + r0 + i, Yv[i]);
-    if (tid < 2) mail_put(A.req + ((size_t)gq * A.nblk + w) * 2 + tid, tid == 0 ? dt : t_now);
+    if (tid < 3) mail_put(A.req + ((size_t)gq * A.nblk + w) * 3 + tid, tid == 0 ? dt : tid == 1 ? t_now : decay);
   };
   auto forget = [&](int own) {
     const size_t old = gq == 0 ? 2 : gq - 1;
     for (int i = own + tid; i < R; i += NT) mail_clear(A.vin + old * A.nc + r0 + i);
-    if (tid < 2) mail_clear(A.req + (old * A.nblk + w) * 2 + tid);
+    if (tid < 3) mail_clear(A.req + (old * A.nblk + w) * 3 + tid);
   };
-  auto ion_and_b = [&](double dt) {
+  auto ion_and_b = [&](double dt, double decay) {
     count(4, 1);
     if constexpr (Model::GAP) {
       // the dendrites' new voltages, for the gap currents of other workgroups' cells
@@ -390,9 +395,9 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, const typena
     }
     const GapView gv{Yv, A.gap + (size_t)gq * A.n, cell0, cells, A.comp, &W};
     const int own = helped ? min(R, A.own) : R;
-    if (helped) request(dt, own);
+    if (helped) request(dt, own, decay);
 #pragma unroll 1
-    for (int i = tid; i < own; i += NT) T[i] = Model::ion(S, r0 + i, Yv[i], dt, &gv);
+    for (int i = tid; i < own; i += NT) T[i] = model_ion<Model>(S, r0 + i, Yv[i], dt, &gv, decay);
     if (helped) {
       for (int i = own + tid; i < R; i += NT) T[i] = mail_get(A.bout + (size_t)gq * A.nc + r0 + i, W);
       forget(own);
@@ -679,10 +684,20 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, const typena
         A.syn_g[r0 + i] = A.syn_g[r0 + i] * A.syn_decay + ((u < A.syn_p) ? A.syn_event : 0.0);
       }
     }
-    bool ion_due = sum_dt != 0.0 && !resume;
+    bool ion_due = sum_dt != 0.0 && (!resume || resume == ASK_DECAY);
     while (true) {
       if (ion_due) {
-        ion_and_b(sum_dt);
+        double decay = 0.0;
+        if constexpr (Model::DECAY)
+          if (S->net_s) {
+            decay = resume ? A.p1 : Model::decay(sum_dt);
+            resume = 0;
+            if (!(decay == decay)) {
+              status = ASK_DECAY;
+              break;
+            }
+          }
+        ion_and_b(sum_dt, decay);
         sum_dt = 0.0;
         ion_due = false;
       }
@@ -720,7 +735,7 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, const typena
   }
 
   if (helped) {
-    request(-1.0, R);
+    request(-1.0, R, 0.0);
     forget(min(R, A.own));
     gq = gq == 2 ? 0 : gq + 1;
   }

@@ -14,5 +14,5 @@ for f in detsum grid_mail rkc_resident; do
       -e 's/asm volatile("s_waitcnt vmcnt(0)" ::: "memory");/__atomic_thread_fence(__ATOMIC_SEQ_CST);/' \
       "$C/$f.hpp" > "$OUT/$f.hpp"
 done
-g++ -std=c++17 -O1 -g -Wno-unknown-pragmas -ffp-contract=off -fPIC -shared -pthread -I "$HERE" -I "$OUT" -I "$C" \
+g++ -std=c++17 -O1 -g -Wno-unknown-pragmas -DCB_HOST_EMU_HOST -ffp-contract=off -fPIC -shared -pthread -I "$HERE" -I "$OUT" -I "$C" \
   "$HERE/resident_emu.cpp" "$C/rkc_coef.cpp" -o "$OUT/libresident.so"

@@ -88,7 +88,7 @@ struct Still {   // constant frozen currents
     const double *b;
   };
   static constexpr int NT = 64, NONFINITE_STATUS = 7;
-  static constexpr bool GAP = false, HELP = true;
+  static constexpr bool GAP = false, HELP = true, DECAY = false;
   static double ion(const State *S, int i, double, double, const GapView *) { return S->b[i]; }
 };
 }  // namespace cbrkc
@@ -160,7 +160,7 @@ int emu_rkc(int n, int comp, int cpb, int nhelp, int present, const int *row, co
   double empty;
   std::memcpy(&empty, &MAIL_EMPTY, 8);
   std::vector<double> ghost((size_t)3 * GHOST_STAGES * max(1, nslot), empty), terms((size_t)3 * nc, empty),
-      parts((size_t)3 * a.nch, empty), gap((size_t)3 * n, empty), req((size_t)6 * nblk, empty),
+      parts((size_t)3 * a.nch, empty), gap((size_t)3 * n, empty), req((size_t)9 * nblk, empty),
       vin((size_t)3 * nc, empty), bout((size_t)3 * nc, empty), v1(nc), v2(nc), bb(b, b + nc), iext(nc), amp(n);
   std::vector<double> table = rkc_stage_table(RES_COEF);
   table.resize(RES_COEFS + 2 * (RES_START + 1));

@@ -1,7 +1,8 @@
 """exp_cr (csrc/exp_acc.hpp), the device exponential of the granule, Golgi and
 olive models, returns exp_acc's value bit for bit: built for the host with
 hipcc, over random arguments of the models' and the whole range, tiny ones,
-the ends of the range, infinities and NaN.  (exp_acc itself is pinned to
+the ends of the range, infinities and NaN; exp_libm, the synaptic decay of
+the resident RKC kernel, is the C library's wherever it claims to be.  (exp_acc itself is pinned to
 60-digit values in test_exp_acc_cpu.py.)"""
 import os
 import subprocess
@@ -14,6 +15,7 @@ HIPCC = "/opt/rocm/bin/hipcc"
 
 PROGRAM = r"""
 #include "exp_acc.hpp"
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -36,6 +38,16 @@ int main() {
   for (double x : {0.0, -0.0, 5e-324, 708.999, -707.999, 709.0, 709.79, 710.0, -708.0, -745.2, -746.0, 1e300, -1e300,
                    1.0 / 0.0, -1.0 / 0.0, 0.0 / 0.0, 0.34657359027997264, -0.34657359027997264})
     one(x);
+  // exp_libm: the host libm's value wherever it says so, and that nearly always
+  long unsure = 0, n = 2000000;
+  for (long i = 0; i < n; i++) {
+    const double u = drand48(), x = i % 2 ? -0.21 * u : -5.0 * u;
+    bool sure;
+    const double a = cbrkc::exp_libm(x, sure), b = std::exp(x);
+    if (!sure) unsure++;
+    else if (a != b && bad++ < 5) std::printf("exp_libm %a: %a, not %a\n", x, a, b);
+  }
+  if (unsure > n / 35) std::printf("unsure %ld of %ld\n", unsure, n);
   std::printf("bad %ld\n", bad);
 }
 """
