@@ -558,6 +558,7 @@ __global__ void __launch_bounds__(Model::NT) k_rkc_steps(RkcArgs A, const typena
   auto attempt = [&]() {
     if (newspc) {
       rkcrho();
+      if (late) return;   // (the estimate is of no use, and could ask for thousands of stages)
       if (sprad < A.rho_floor) sprad = A.rho_floor;
       jacatt = true;
     }

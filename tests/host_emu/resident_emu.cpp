@@ -7,7 +7,6 @@
 #include <hip/hip_runtime.h>
 
 #include <atomic>
-#include <chrono>
 #include <cstring>
 #include <memory>
 #include <thread>
@@ -38,6 +37,8 @@ struct Group {
   std::vector<double> lds;
 };
 thread_local Group *t_group = nullptr;
+thread_local unsigned long long t_polls = 0;
+std::atomic<unsigned long long> max_polls{0};
 
 }  // namespace
 
@@ -46,7 +47,10 @@ thread_local emu_dim3 blockIdx;
 double emu_shfl_xor(double x, int) { return x; }
 void emu_wave_barrier() { t_group->bar.wait(); }
 void emu_syncthreads() { t_group->bar.wait(); }
-void emu_pause() { std::this_thread::yield(); }   // a poll lets the other lanes run
+void emu_pause() {   // a poll lets the other lanes run
+  t_polls++;
+  std::this_thread::yield();
+}
 int emu_syncthreads_or(int x) {
   t_group->is[threadIdx.x] = x;
   t_group->bar.wait();
@@ -69,11 +73,7 @@ int emu_first_lane(int x) {
   t_group->bar.wait();
   return y;
 }
-unsigned long long emu_clock() {   // 100 MHz, as the device's
-  return (unsigned long long)std::chrono::duration_cast<std::chrono::nanoseconds>(
-             std::chrono::steady_clock::now().time_since_epoch())
-             .count() / 10;
-}
+unsigned long long emu_clock() { return t_polls; }   // a lane's time: its looks at mailboxes
 static double *emu_lds() { return t_group->lds.data(); }
 static int *emu_late() { return &t_group->late; }
 
@@ -97,13 +97,14 @@ using namespace cbrkc;
 extern "C" {
 // nsteps macro steps of n cells of comp rows (at most 64 K rows of a cell), cpb
 // cells to a workgroup, nhelp helpers to each; present: workgroups that are
-// started at all (fewer: the others wait in vain); launches: how often the
-// kernel was started.  vec: y, yn, fn, ede, vnew.
+// started at all (fewer: the others wait in vain); wait: the limit of a wait, in looks;
+// launches: how often the kernel was started; polls: the most looks of a lane.  vec: y, yn, fn, ede, vnew.
 // o16, hw8 and cnt5 (steps, rejects, stages, power iterations, ion updates)
 // come back.  Returns the last status.
 int emu_rkc(int n, int comp, int cpb, int nhelp, int present, const int *row, const int *col, const double *val,
             const double *cm, const double *b, double *vec, double *o16, double *hw8, long long *cnt5, int nsteps,
-            double rho_floor, int refresh, double wait, int *launches) {
+            double rho_floor, int refresh, long long wait, int *launches,
+            long long *polls) {
   const int nc = n * comp, RM = cpb * comp, nblk = (n + cpb - 1) / cpb;
   RkcArgs a{};
   a.n = n;
@@ -197,7 +198,8 @@ int emu_rkc(int n, int comp, int cpb, int nhelp, int present, const int *row, co
   a.cm = cm;
   a.coef = table.data();
   a.integ = 1e30;
-  a.wait = wait_ticks(wait);
+  a.wait = (unsigned long long)wait;
+  max_polls = 0;
   a.rho_floor = rho_floor;
   a.refresh_fn = refresh;
   a.iext = iext.data();
@@ -239,8 +241,12 @@ int emu_rkc(int n, int comp, int cpb, int nhelp, int present, const int *row, co
           const int left = nsteps - (int)host.macro;
           if (RM <= 64) k_rkc_steps<Still, 1>(a, &S, left, 0.0, 0);
           else k_rkc_steps<Still, 4>(a, &S, left, 0.0, 0);
+          unsigned long long most = max_polls;
+          while (most < t_polls && !max_polls.compare_exchange_weak(most, t_polls)) {
+          }
         });
     for (auto &t : th) t.join();
+    *polls = (long long)max_polls.load();
     ++*launches;
     a.resume = host.status == ASK_POW || host.status == ASK_STAGE ? host.status : 0;
     a.p1 = std::pow(host.err, 1.0 / 3.0);

@@ -7,7 +7,6 @@ import ctypes
 import os
 import shutil
 import subprocess
-import time
 
 import numpy as np
 import pytest
@@ -26,7 +25,7 @@ def emu(tmp_path_factory):
     return ctypes.CDLL(str(out / "libresident.so"))
 
 
-def run(emu, o, n, cpb=1, nsteps=1, nhelp=0, present=1 << 20, floor=0.0, refresh=False, wait=60.0):
+def run(emu, o, n, cpb=1, nsteps=1, nhelp=0, present=1 << 20, floor=0.0, refresh=False, wait=1 << 60):
     """nsteps macro steps of the oracle population o, as n cells, on the host
     build, from o's present state, with this floor of the spectral radius and
     refresh of fn after ion updates; o itself stays"""
@@ -39,12 +38,12 @@ def run(emu, o, n, cpb=1, nsteps=1, nhelp=0, present=1 << 20, floor=0.0, refresh
     c, hw = np.zeros(16), np.zeros(8)
     c[:14], hw[:] = o.controller()[0], o.controller()[1]
     cnt = np.array([o.stats()[k] for k in ("steps", "rejects", "stages", "rho_iters", "ion_updates")], dtype=np.int64)
-    launches = ctypes.c_int()
+    launches, polls = ctypes.c_int(), ctypes.c_longlong()
     p = lambda a: a.ctypes.data_as(ctypes.c_void_p)  # noqa: E731
     status = emu.emu_rkc(n, comp, cpb, nhelp, present, p(row), p(col), p(keep[0]), p(keep[1]), p(keep[2]), p(vec), p(c),
-                         p(hw), p(cnt), nsteps, ctypes.c_double(floor), 1 if refresh else 0, ctypes.c_double(wait),
-                         ctypes.byref(launches))
-    return dict(status=status, vec=vec, ctl=c[:14], hw=hw, cnt=cnt, launches=launches.value)
+                         p(hw), p(cnt), nsteps, ctypes.c_double(floor), 1 if refresh else 0, ctypes.c_longlong(wait),
+                         ctypes.byref(launches), ctypes.byref(polls))
+    return dict(status=status, vec=vec, ctl=c[:14], hw=hw, cnt=cnt, launches=launches.value, polls=polls.value)
 
 
 def check(o, r, nsteps=1):
@@ -89,12 +88,13 @@ def test_a_lost_workgroup_ends_the_launch(emu, n, comp, nhelp, pairs):
     # Only the first workgroup runs (or, of three, the first two): it gives up
     # once, not at every one of a step's 140 exchanges, and says so
     o = cables(n, comp, 0.5, pairs=pairs, spread=1e-3)
-    t0 = time.monotonic()
-    r = run(emu, o, n, nhelp=nhelp, present=max(1, n - 1), floor=2e5, wait=0.5, nsteps=2)
+    wait = 20000   # looks at mailboxes, a lane's clock on the host
+    r = run(emu, o, n, nhelp=nhelp, present=max(1, n - 1), floor=2e5, wait=wait, nsteps=2)
     assert r["status"] == 8
-    assert time.monotonic() - t0 < 30.0   # 140 limits would be 70 s
+    # two limits, and 128 looks at each of the step's other exchanges; not a limit at each
+    assert r["polls"] < 2 * wait + 1000 + 200 * 128 < 10 * wait
     # no waiting at all: the first look that finds nothing
-    assert run(emu, o, n, nhelp=nhelp, present=max(1, n - 1), floor=2e5, wait=0.0,
+    assert run(emu, o, n, nhelp=nhelp, present=max(1, n - 1), floor=2e5, wait=0,
                nsteps=2)["status"] == 8
 
 
